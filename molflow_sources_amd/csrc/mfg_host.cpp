@@ -880,11 +880,11 @@ struct mfg_context {
     uint32_t features = 0;
     bool loaded = false, accel = false;
     uint32_t stack_size = 0;             // traversal stack entries a walk may need
-    DevBuf<int32_t> stack_spill;         // per-lane entries beyond the LDS part
+    DevBuf<int32_t> stack_spill;         // per-lane entries beyond the LDS part (transparent models)
+    uint32_t task_bits = 26;             // bits of a node or leaf record index in a walk task
     int bvh_width = MFG_BVH_WIDTH, leaf_size = 2;   // children per BVH node, facets per leaf
-    // BVH nodes each block keeps in LDS (top of the breadth-first array):
-    // 16 KB, which leaves 256-thread blocks their occupancy up to 5 waves
-    // per SIMD
+    // BVH nodes a block of up to 256 lanes keeps in LDS at most (top of the
+    // breadth-first array)
     uint32_t node_cache = 128;
     size_t lds_per_block = 65536;        // the device's LDS limit for one block
     // device data
@@ -1274,6 +1274,9 @@ void build_accel(mfg_context* c, int width, int leaf) {
     uint32_t need = (uint32_t)((width - 1) * depth + width);
     if (need > MFG_MAX_STACK) throw Err(MFG_ERR_LIMIT, "BVH too deep for the LDS traversal stack (depth " + std::to_string(depth) + ")");
     c->stack_size = need;
+    // a walk task packs its ray above the index of its node or record
+    c->task_bits = 26;
+    while (c->task_bits < 31 && std::max(nodes.size(), leafs.size()) > ((size_t)1 << c->task_bits)) ++c->task_bits;
     if (leafs.size() >= ((size_t)1 << 27)) throw Err(MFG_ERR_LIMIT, "more than 2^27 BVH leaf records");
     hipStream_t s = c->stream;
     c->nodes.upload(nodes, s);
@@ -1300,18 +1303,16 @@ void build_accel(mfg_context* c, int width, int leaf) {
     reset_graph(c);
 }
 
-// Nodes read from LDS: the top of the tree of a single-variant model.
-uint32_t lds_node_count(const mfg_context* c, int block) {
+// Nodes read from LDS: the top of the tree of a single-variant model, as
+// many as fit beside the waves' walk areas and the hot facets in a block's
+// share of the CU's LDS (all of it for a block of 768 or 1024 lanes, else a
+// 1 / waves part for every 256 lanes).
+uint32_t lds_node_count(const mfg_context* c, int block, int waves) {
     if (c->dvars.size() != 1) return 0;
-    size_t n = c->node_cache;
-    if (block > 256) {
-        // a block of 768 or 1024 lanes serves a whole CU: the LDS its stacks and hot
-        // facets leave (at least four times a 256-lane block's copy)
-        const size_t used = (size_t)block * std::min<uint32_t>(c->stack_size, MFG_LDS_STACK) * sizeof(int32_t) +
-                            c->hot.size() * 8 * sizeof(double);
-        const size_t room = c->lds_per_block > used + 2048 ? (c->lds_per_block - used - 2048) / sizeof(BvhNode) : 0;
-        n = std::max<size_t>(4 * (size_t)c->node_cache, room);
-    }
+    const size_t share = block > 256 ? c->lds_per_block : c->lds_per_block * (size_t)block / 256 / (size_t)std::max(1, waves);
+    const size_t used = (size_t)(block / 64) * MFG_WAVE_LDS + c->hot.size() * 8 * sizeof(double) + 256;
+    size_t n = share > used ? (share - used) / sizeof(BvhNode) : 0;
+    if (block <= 256) n = std::min<size_t>(n, c->node_cache);
     return (uint32_t)std::min<size_t>(n, c->nodes.n);
 }
 
@@ -1320,9 +1321,9 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     p.facets = c->facets.p; p.phys = c->phys.p; p.poly = c->poly.p; p.nodes = c->nodes.p;
     p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p; p.roots = c->roots.p; p.variants = c->variants.p;
     p.var_prefix = c->prefix.p; p.n_variants = (uint32_t)c->dvars.size();
-    p.stack_size = std::min<uint32_t>(c->stack_size, MFG_LDS_STACK);
+    p.task_bits = c->task_bits;
     p.stack_total = c->stack_size;
-    p.stack_spill = p.stack_total > p.stack_size ? c->stack_spill.p : nullptr;
+    p.stack_spill = p.stack_total > MFG_LANE_STACK ? c->stack_spill.p : nullptr;
     p.src_cum = c->src_cum.p; p.src_facet = c->src_facet.p; p.og_cdf = c->og_cdf.p; p.am_src = c->am_src.p;
     p.hot_fc = c->hot_fc.p; p.n_hot = (uint32_t)c->hot.size();
     p.guides = c->guides.p; p.tab_x = c->tab_x.p; p.tab_y = c->tab_y.p; p.params = c->params.p; p.ids = c->ids.p;
@@ -1363,8 +1364,8 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
         else block = 256;
     }
     auto lds_bytes = [&](int b) {
-        return (size_t)b * std::min<uint32_t>(c->stack_size, MFG_LDS_STACK) * sizeof(int32_t) +
-               c->hot.size() * 8 * sizeof(double) + (size_t)lds_node_count(c, b) * sizeof(BvhNode);
+        return (size_t)(b / 64) * MFG_WAVE_LDS + c->hot.size() * 8 * sizeof(double) +
+               (size_t)lds_node_count(c, b, waves) * sizeof(BvhNode);
     };
     if (block > 256 && mfg_trace_occupancy(feats, waves, block, lds_bytes(block)) < 1) {
         block = 256;   // the block's LDS does not fit
@@ -1428,8 +1429,8 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
         if (c->adj_seg_t.n < seg) { c->adj_seg_t.alloc(seg); c->adj_seg_x.alloc(seg); reset_graph(c); }
     }
     if (c->carry_on) ensure_carry(c, (uint64_t)grid * (uint64_t)block);
-    if (c->stack_size > MFG_LDS_STACK) {
-        size_t need = (size_t)grid * block * (c->stack_size - MFG_LDS_STACK);
+    if ((feats & FEAT_TRANSPARENT) && c->stack_size > MFG_LANE_STACK) {
+        size_t need = (size_t)grid * block * (c->stack_size - MFG_LANE_STACK);
         if (c->stack_spill.n < need) { c->stack_spill.alloc(need); reset_graph(c); }
     }
     // read the global counters before the run to report this run's hits
@@ -1438,13 +1439,21 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     HIPCHK(hipMemcpyAsync(before.data(), c->glob.p, nv * sizeof(DGlobal), hipMemcpyDeviceToHost, s));
     *c->stop_host = 0;
     TraceParams p = make_params(c, total, max_events);
-    p.lds_nodes = lds_node_count(c, block);
+    p.lds_nodes = lds_node_count(c, block, waves);
+    // lanes of a wave that take particles: all once there is one for every
+    // lane, else the items are spread over all waves, whose other lanes then
+    // help with the walks (a wave's step gets shorter the fewer rays it has:
+    // 1000 tube particles 3.1 -> 1.6 ms, 2e4 adjoint ones 394 -> 114 ms with
+    // the shared walk, one wave in ten having had all of the latter before)
+    const uint64_t n_waves = (uint64_t)grid * (uint64_t)(block / 64);
+    const uint64_t cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
+    p.lane_quota = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cap, (total + c->in_flight + n_waves - 1) / n_waves));
     std::vector<uint64_t> key(n_des, n_des + nv);
     key.push_back(max_events); key.push_back(feats); key.push_back((uint64_t)grid); key.push_back(block);
     key.push_back((uint64_t)waves);
     key.push_back((uint64_t)(uintptr_t)p.carry); key.push_back(p.carry_keep);
     key.push_back((uint64_t)(uintptr_t)p.hot_fc); key.push_back(p.n_hot); key.push_back(p.time_limit);
-    key.push_back(p.lds_nodes);
+    key.push_back(p.lds_nodes); key.push_back(p.lane_quota);
     // the events bracket the trace kernel alone (eager path) or the whole
     // graph (replay path)
     auto enqueue = [&](bool events) {
@@ -1659,7 +1668,11 @@ void launch_batch(mfg_context* c, uint64_t n, const double* dO, const double* dD
     IsectParams p{};
     p.facets = c->facets.p; p.poly = c->poly.p; p.nodes = c->nodes.p; p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p;
     p.root = c->h_roots.at(c->dvars[0].root_base + (uint32_t)structure);
-    p.stack_size = c->stack_size; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
+    // few rays are spread over the CUs, 8 a wave at least (the wave's lanes
+    // share their walks)
+    const uint64_t spread = n / ((uint64_t)c->n_cu * 8), cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
+    p.rays_per_wave = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(8, spread));
+    p.task_bits = c->task_bits; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
     p.out_facet = dF; p.out_t = dT; p.out_u = dU; p.out_v = dV; p.facet_base = c->dvars[0].facet_base;
     if (mfg_launch_intersect(p, c->stream)) throw Err(MFG_ERR_DEVICE, "intersect launch failed");
 }

@@ -20,9 +20,10 @@
 #define MFG_ADJ_SEG 32            // target scores kept per lane for the adjoint's cutoff term
 #define MFG_BVH_WIDTH 8          // children per node (a 4-wide build uses 4 of the 8 slots)
 #define MFG_MAX_STACK 64
-#ifndef MFG_LDS_STACK
-#define MFG_LDS_STACK 16         // traversal stack entries per lane kept in LDS by the tracer
-#endif
+#define MFG_WALK_NODES 512       // (ray, node) tasks of one wave's walk
+#define MFG_WALK_RESERVE 72      // of these for the depth-first tail: width - 1 entries a level, + width
+#define MFG_WALK_LEAVES 256      // (ray, facet record) tasks waiting: below 64 plus one node's 8 leaves of 16
+#define MFG_LANE_STACK ((MFG_WALK_NODES + MFG_WALK_LEAVES) / 64)   // entries of a lane's own stack in the same LDS
 #define MFG_MAX_GROUPS 64
 #define MFG_MAXWELL_GUIDE 128
 #define MFG_MAX_HOT 32           // facets whose counters are privatised per block
@@ -162,6 +163,24 @@ struct alignas(64) LeafUV {
 };
 static_assert(sizeof(LeafUV) == 64, "LeafUV layout");
 
+#ifdef __HIPCC__
+// LDS of one wave's walk: slot r holds ray r (the ray of lane r). The FP32
+// copy serves the box tests, the FP64 one the facet tests.
+struct alignas(16) WaveLds {
+    float4 ra[64];                     // origin, nearest t so far (widened)
+    float4 rb[64];                     // 1 / direction, facet to skip (bits)
+    double2 p01[64], p2d0[64], d12[64];   // position x y | z, direction x | y z
+    unsigned long long t[64];          // nearest t so far (bits of a positive double)
+    int32_t facet[64];                 // its facet, -1 none
+    uint32_t nodes[MFG_WALK_NODES];    // ray << task_bits | node
+    uint32_t leaves[MFG_WALK_LEAVES];  // ray << task_bits | facet record
+};
+#endif
+#define MFG_WAVE_LDS 8960
+#ifdef __HIPCC__
+static_assert(sizeof(WaveLds) == MFG_WAVE_LDS, "MFG_WAVE_LDS is the size of WaveLds");
+#endif
+
 // global counters of one variant (mfg_global_counters)
 struct DGlobal {
     unsigned long long nb_mc_hit;
@@ -243,8 +262,9 @@ struct TraceParams {
     const DVariant* variants;
     const uint64_t* var_prefix;       // n_variants+1 prefix of this run's desorptions
     uint32_t n_variants;
-    uint32_t stack_size;              // LDS stack entries per lane
-    uint32_t stack_total;             // entries a walk may need; the ones past stack_size
+    uint32_t task_bits;               // bits of a walk task's node or record index (the rest: its ray)
+    uint32_t lane_quota;              // lanes of a wave that take particles
+    uint32_t stack_total;             // entries a lane's own walk may need; the ones past MFG_LANE_STACK
     int32_t* stack_spill;             // live in this per-lane global area (lane-major)
     const double* src_cum;            // cumulative source weights
     const int32_t* src_facet;
@@ -325,7 +345,8 @@ struct IsectParams {
     const LeafFacet* leaves;
     const LeafUV* leaf_uv;
     int32_t root;
-    uint32_t stack_size;
+    uint32_t task_bits;
+    uint32_t rays_per_wave;
     uint64_t n;
     const double* origins;
     const double* dirs;

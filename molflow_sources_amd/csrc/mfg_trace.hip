@@ -3,11 +3,10 @@
 // k_trace: one persistent launch traces a whole batch of desorptions. Each
 // lane owns one particle in registers; dead lanes refill from a global work
 // queue with one atomic per wave (ballot + mbcnt), first from the particles
-// the previous launch parked. Per event a lane walks an 8-wide BVH of 128 B
-// nodes with 8-bit quantised FP32 boxes (the top of the tree copied to LDS
-// per block, traversal stack in LDS laid out [entry][lane]); leaf children
-// go on the stack and the wave tests them together once enough lanes hold
-// one; facets are tested in FP64. It then applies the event of reference
+// the previous launch parked. Per event the lanes of a wave walk an 8-wide
+// BVH of 128 B nodes with 8-bit quantised FP32 boxes together, from one task
+// stack in LDS (the top of the tree is copied to LDS per block); facets are
+// tested in FP64. A lane then applies the event of reference
 // src/Simulation/Particle.cpp:207-396 (desorption, bounce, absorption,
 // transparent pass, teleport, link, leak, volume events). Tallies are u64 /
 // FP64 atomics: lanes of a wave that update the same facet counter (or
@@ -564,17 +563,16 @@ __device__ __forceinline__ double td_opacity(const TraceParams& P, const DVarian
     return interp_y(time, XYRef{P.tab_x + tb.off, P.tab_y + tb.off, tb.n}, tb.log_x, tb.log_y, false);
 }
 
-// Traversal stack of one lane: the first `lds_cap` entries in LDS (laid out
-// [entry][lane]), deeper entries (rare) in a per-lane global area.
+// Traversal stack of one lane (the second walk of a transparent model): the
+// first `lds_cap` entries in LDS (laid out [entry][lane]), deeper entries
+// (rare) in a per-lane global area.
 struct LaneStack {
-    int32_t* lds;
-    uint32_t stride, lds_cap, cap;
+    uint32_t* lds;
+    uint32_t lds_cap, cap;
     int32_t* spill;
-    // entry sp of a lane sits sp * stride words after its first one (both
-    // below 2^24: a full-rate 24-bit multiply)
     __device__ __forceinline__ void push(uint32_t& sp, int32_t v) const {
         if (sp < lds_cap) {
-            lds[__umul24(sp, stride)] = v;
+            lds[sp * 64u] = (uint32_t)v;
             ++sp;
         } else if (sp < cap) {
             spill[sp - lds_cap] = v;
@@ -583,121 +581,208 @@ struct LaneStack {
     }
     __device__ __forceinline__ int32_t pop(uint32_t& sp) const {
         --sp;
-        return sp < lds_cap ? lds[__umul24(sp, stride)] : spill[sp - lds_cap];
+        return sp < lds_cap ? (int32_t)lds[sp * 64u] : spill[sp - lds_cap];
     }
 };
 
-// Nearest hard hit below tmax. With TRANSP, non-opaque facets are hard with
-// probability `opacity` (coin per event and facet); opaque_only ignores
-// opacity (fixed ray batches).
-//
-// Each lane holds one stack entry: a node (>= 0) or a leaf (< 0: ~(first
-// record << 4 | facets - 1)). A node step tests the children's boxes and
-// pushes the inner children (slot order), then the leaf children on top,
-// so that leaves come off first and shrink tmax early. Each iteration the
-// wave votes: lanes holding a leaf test its facets together once at least
-// kLeafBatch of them hold one, or twice as many as hold a node, or when no
-// lane holds a node; otherwise the node lanes step. Testing a node's leaves
-// inside the node step instead ran the facet loop about 49 times per
-// traversal of a beam-pipe wave with 7 of 64 lanes active; the vote cuts
-// the wave's node plus facet iterations by about 29 % there (CPU emulation
-// of both on the same tree) and leaves every hit unchanged: the nearest
-// hit does not depend on the order facets are tested in (ties go to the
-// lower facet id), and the opacity coin is a function of event and facet.
-// A near-to-far sort of the children left the node visits per ray within
-// 2 % on these trees but cost about a hundred instructions per node.
-constexpr uint32_t kLeafBatch = 24;
-
-__device__ __forceinline__ int32_t leaf_entry(uint32_t first, uint32_t cnt) {
-    return ~(int32_t)((first << 4) | (cnt - 1u));
+// Orders this wave's LDS accesses before and after it (the hardware runs
+// them in order; this keeps the compiler from moving them or from splitting
+// the control flow around it).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive sum over the lanes below and including this one (all 64 active).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
+// What the opacity coin of a ray needs from the lane that owns it.
+struct CoinState {
+    uint32_t k0, k1, p0, p1, event;
+    double time;
+    const DVariant* var;
+};
+
+// Nearest hard hit of the wave's up to 64 rays, walked together: ray r sits
+// in slot r of W (walk_load), and the wave shares one stack of (ray, node)
+// tasks and one list of (ray, facet record) tasks. A node step gives each
+// lane one of the topmost tasks, whichever ray it belongs to; the inner
+// children hit go back on the stack and the facets of the leaf children hit
+// into the list, at offsets from one scan over the lanes. A facet step
+// gives each lane one record. A facet step runs once 64 records wait or no
+// node does, so both kinds of step run with nearly all lanes at work as
+// long as the wave has work, and a ray whose walk is long is helped by the
+// lanes whose rays are done: with one ray per lane instead (each lane its
+// own stack, leaves tested by wave vote) 14 % of the lanes were active on
+// the beam pipe, for 28 node and 21 facet iterations per wave where the 64
+// rays' 11 nodes and 5 facets each fill about 18. Beam pipe (1e5 facets, 6e5
+// desorptions a launch): 121.5 -> 91.3 ms per launch, its drain 166 -> 82 ms;
+// 2e4 low-flux particles (all tail) 456 -> 158 ms; the 1e6-particle tube 7.7
+// -> 5.7 ms.
+//
+// The nearest hit is the minimum over the same facet tests, with ties going
+// to the lower facet id, so it does not depend on the order or the lanes
+// the tests run on.
+//
+// Bounds. A node step commits the tasks of its first lanes only, as many as
+// leave the stack below its capacity less a reserve and the list within
+// its capacity; the other tasks stay where they are. Lane 0 (the topmost
+// task) may use the reserve, so once the stack is up to it the walk is depth
+// first, which adds at most width - 1 entries a level: the reserve holds
+// that for the deepest tree the host accepts. The list has room for lane
+// 0's facets (8 leaves of 16) whenever a node step runs (below 64 waiting).
 template <bool TRANSP>
-__device__ HitRec traverse(const TraceParams& P, int32_t root, d3 Pp, d3 D, int32_t skip, double tmax,
-                           const LaneStack& S, const Rng* rng,
-                           uint32_t event, const DVariant* var, double time, bool opaque_only,
-                           const uint4* lnodes) {
-    HitRec h{-1, tmax, 0.0, 0.0};
-    if (root < 0) return h;
-    Ray32 r = make_ray32(Pp, D);
-    float tbf = widen(tmax);
-    uint32_t sp = 0;
-    int32_t cur = root;
-    bool live = true;
-    for (;;) {
-        const bool on_leaf = live && cur < 0, on_node = live && cur >= 0;
-        const uint32_t nl = (uint32_t)__popcll(__ballot(on_node));
-        const uint32_t ll = (uint32_t)__popcll(__ballot(on_leaf));
-        if (nl + ll == 0) break;
-        if (ll >= kLeafBatch || ll >= 2 * nl) {
-            if (on_leaf) {
-                const uint32_t e = ~(uint32_t)cur, first = e >> 4, cnt = (e & 15u) + 1u;
-                for (uint32_t k = 0; k < cnt; ++k) {
-                    double t, u, v;
-                    int32_t f;
-                    uint32_t fl;
-                    bool hit = leaf_test(P.leaves + first + k, P.leaf_uv + first + k, P.poly, Pp, D, skip, t, u, v, f, fl);
-                    if (!hit) continue;
-                    if (!(t < h.t || (t == h.t && f < h.facet))) continue;
-                    bool hard = true;
-                    if constexpr (TRANSP) {
-                        if (!opaque_only && !(fl & FF_OPAQUE)) {
-                            double op = (fl & FF_TD_OPACITY) ? td_opacity(P, var, f, time) : (double)P.phys[f].opacity;
-                            if (op < 1.0) hard = (op > 0.0) && rng->coin(event, (uint32_t)(f - (int32_t)var->facet_base)) < op;
-                        }
-                    }
-                    if (hard) {
-                        h.facet = f; h.t = t; h.u = u; h.v = v;
-                        tbf = widen(t);
+__device__ void walk(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint32_t lane, bool live, int32_t root,
+                     const CoinState& cs) {
+    const uint32_t bits = P.task_bits, low = (1u << bits) - 1u;
+    uint32_t top, waiting = 0;   // wave-uniform
+    {
+        const bool on = live && root >= 0;
+        const uint64_t m = __ballot(on);
+        top = (uint32_t)__popcll(m);
+        if (on) W.nodes[mbcnt(m)] = (lane << bits) | (uint32_t)root;
+    }
+    wave_sync();
+    while (top + waiting != 0) {
+        if (waiting < 64u && top != 0) {
+            const bool on = lane < top;
+            uint32_t tag = 0, inner = 0, im = 0, lm = 0, cw = 0, own = 0;
+            int32_t node_base = 0;
+            NodeRegs nd{};
+            if (on) {
+                const uint32_t w = W.nodes[top - 1u - lane], ray = w >> bits;
+                tag = w & ~low;
+                nd = load_node_at(P.nodes, lnodes, P.lds_nodes, (int32_t)(w & low));
+                const float4 a = W.ra[ray], b = W.rb[ray];
+                const Ray32 r{a.x, a.y, a.z, b.x, b.y, b.z};
+                const uint32_t m = node_hits(nd, r, a.w);   // children entering before the nearest hit
+                inner = node_inner(nd);
+                im = m & inner;
+                lm = m & node_leaves(nd);
+                cw = nd.c1.z;
+                node_base = (int32_t)nd.c1.x;
+                // facets of the hit leaves: one more than each one's 4-bit count
+                uint32_t e = (lm | (lm << 12)) & 0x000f000fu;
+                e = (e | (e << 6)) & 0x03030303u;
+                e = (e | (e << 3)) & 0x11111111u;
+                own = (uint32_t)__popc(im) | (((uint32_t)__popc(lm) + nibble_sum(cw & (e * 15u))) << 16);
+            }
+            const uint32_t upto = wave_scan(own);
+            // lanes that commit: a prefix
+            const uint32_t after = top - 1u - lane + (upto & 0xffffu);
+            const bool fits = on && after <= (lane == 0 ? MFG_WALK_NODES : MFG_WALK_NODES - MFG_WALK_RESERVE) &&
+                              waiting + (upto >> 16) <= MFG_WALK_LEAVES;
+            const uint64_t miss = __ballot(!fits);
+            const uint32_t n = miss ? (uint32_t)__builtin_ctzll(miss) : 64u;
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)n - 1);
+            wave_sync();
+            if (lane < n) {
+                uint32_t at = top - n + (total & 0xffffu) - (upto & 0xffffu);   // lane 0's children on top
+                while (im) {
+                    const uint32_t c = (uint32_t)__builtin_ctz(im);
+                    im &= im - 1u;
+                    W.nodes[at++] = tag | (uint32_t)(node_base + (int32_t)__popc(inner & ((1u << c) - 1u)));
+                }
+                at = waiting + ((upto - own) >> 16);
+                while (lm) {
+                    const uint32_t c = (uint32_t)__builtin_ctz(lm);
+                    lm &= lm - 1u;
+                    uint32_t first, cnt;
+                    node_leaf_child(nd, c, first, cnt);
+                    for (uint32_t k = 0; k < cnt; ++k) W.leaves[at++] = tag | (first + k);
+                }
+            }
+            top = (uint32_t)__builtin_amdgcn_readfirstlane((int)(top - n + (total & 0xffffu)));
+            waiting = (uint32_t)__builtin_amdgcn_readfirstlane((int)(waiting + (total >> 16)));
+            wave_sync();
+        } else {
+            const uint32_t n = waiting < 64u ? waiting : 64u;
+            waiting -= n;
+            uint32_t ray = 0;
+            double t = 0.0, u, v;
+            int32_t f = -1;
+            uint32_t fl = FF_OPAQUE;
+            bool hit = false;
+            if (lane < n) {
+                const uint32_t w = W.leaves[waiting + lane];
+                ray = w >> bits;
+                const uint32_t rec = w & low;
+                const double2 a = W.p01[ray], b = W.p2d0[ray], c = W.d12[ray];
+                hit = leaf_test(P.leaves + rec, P.leaf_uv + rec, P.poly, mk(a.x, a.y, b.x), mk(b.y, c.x, c.y),
+                                __float_as_int(W.rb[ray].w), t, u, v, f, fl);
+            }
+            if constexpr (TRANSP) {
+                const bool coin = hit && !(fl & FF_OPAQUE);
+                if (__ballot(coin)) {
+                    // the ray's stream, event and clock, from the lane that owns it
+                    Rng g;
+                    g.k0 = __shfl(cs.k0, ray, 64); g.k1 = __shfl(cs.k1, ray, 64);
+                    g.p0 = __shfl(cs.p0, ray, 64); g.p1 = __shfl(cs.p1, ray, 64);
+                    const uint32_t ev = __shfl(cs.event, ray, 64);
+                    const double tm = __shfl(cs.time, ray, 64);
+                    const DVariant* var = (const DVariant*)__shfl((unsigned long long)cs.var, ray, 64);
+                    if (coin) {
+                        double op = (fl & FF_TD_OPACITY) ? td_opacity(P, var, f, tm) : (double)P.phys[f].opacity;
+                        if (op < 1.0) hit = (op > 0.0) && g.coin(ev, (uint32_t)(f - (int32_t)var->facet_base)) < op;
                     }
                 }
-                if (sp == 0) live = false;
-                else cur = S.pop(sp);
             }
-        } else if (on_node) {
-            const NodeRegs nd = load_node_at(P.nodes, lnodes, P.lds_nodes, cur);
-            const uint32_t m = node_hits(nd, r, tbf);   // children entering before tmax
-            uint32_t im = m & node_inner(nd);
-            uint32_t lm = m & node_leaves(nd);
-            // the entry the stack would hand back first (the lowest leaf
-            // slot, else the lowest inner slot) becomes the next one
-            // directly, without its push and pop
-            int32_t next = 0;
-            const bool direct = (im | lm) != 0;
-            if (lm) {
-                const uint32_t c = (uint32_t)__builtin_ctz(lm);
-                lm &= lm - 1u;
-                uint32_t first, cnt;
-                node_leaf_child(nd, c, first, cnt);
-                next = leaf_entry(first, cnt);
-            } else if (im) {
-                const uint32_t c = (uint32_t)__builtin_ctz(im);
-                im &= im - 1u;
-                next = node_inner_child(nd, c);
+            if (__ballot(hit)) {
+                // lanes of one ray settle their nearest t by an LDS minimum
+                // (t > 0: its bits order like the number), then the facet
+                const unsigned long long tb = hit ? (unsigned long long)__double_as_longlong(t) : ~0ull;
+                unsigned long long old = 0, cur = 0;
+                if (hit) old = atomicMin(&W.t[ray], tb);
+                wave_sync();
+                if (hit) cur = W.t[ray];
+                const bool best = hit && cur == tb;
+                if (best && old > tb) W.facet[ray] = 0x7fffffff;   // first at this distance
+                wave_sync();
+                if (best) {
+                    atomicMin(&W.facet[ray], f);
+                    W.ra[ray].w = widen(t);
+                }
             }
-#pragma unroll
-            for (int c = 7; c >= 0; --c)
-                if (im & (1u << c)) S.push(sp, node_inner_child(nd, (uint32_t)c));
-            while (lm) {
-                const uint32_t c = 31u - (uint32_t)__builtin_clz(lm);
-                lm &= ~(1u << c);
-                uint32_t first, cnt;
-                node_leaf_child(nd, c, first, cnt);
-                S.push(sp, leaf_entry(first, cnt));
-            }
-            if (direct) cur = next;
-            else if (sp == 0) live = false;
-            else cur = S.pop(sp);
+            wave_sync();
         }
     }
-    return h;
+}
+
+// Ray slot of this lane for walk().
+__device__ __forceinline__ void walk_load(WaveLds& W, uint32_t lane, d3 p, d3 d, int32_t skip, double tmax) {
+    const Ray32 r = make_ray32(p, d);
+    W.ra[lane] = make_float4(r.ox, r.oy, r.oz, widen(tmax));
+    W.rb[lane] = make_float4(r.ix, r.iy, r.iz, __int_as_float(skip));
+    W.p01[lane] = make_double2(p.x, p.y);
+    W.p2d0[lane] = make_double2(p.z, d.x);
+    W.d12[lane] = make_double2(d.y, d.z);
+    W.t[lane] = (unsigned long long)__double_as_longlong(tmax);
+    W.facet[lane] = -1;
+}
+
+// (u,v) of a hit at distance t on a facet: the operations of facet_test.
+__device__ __forceinline__ void hit_uv(const DFacet* __restrict__ F, d3 P, d3 D, double t, double& u, double& v) {
+    d3 X = mk(fma(t, D.x, P.x), fma(t, D.y, P.y), fma(t, D.z, P.z));
+    d3 r = sub(X, ld3(F->O));
+    u = fdot(r, ld3(F->U)) * F->invU2;
+    v = fdot(r, ld3(F->V)) * F->invV2;
 }
 
 // ------------------------------------------------------------------ tracer
 template <uint32_t FEAT>
 struct Tracer {
     const TraceParams& P;
-    LaneStack S;
+    WaveLds& W;                       // this wave's walk area
+    int32_t* spill;                   // this lane's stack entries beyond the LDS part (second walk)
     // particle state (reference Particle.h:95-122)
     d3 pos, dir;
     double time, vel, ori, gen_time, dist, decay_t, scatter_path, hu, hv;
@@ -722,7 +807,7 @@ struct Tracer {
     uint32_t pend_hits;
     double pend_he, pend_abs, pend_s1v, pend_svo, pend_s1pv;
 
-    __device__ Tracer(const TraceParams& p, const LaneStack& s) : P(p), S(s) {
+    __device__ Tracer(const TraceParams& p, WaveLds& w, int32_t* sp) : P(p), W(w), spill(sp) {
         acc_hits = acc_des = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
         acc_leak = acc_decay = 0;
@@ -1500,14 +1585,27 @@ struct Tracer {
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
     }
 
-    // One event of an alive particle (one SimulationMCStep iteration).
+    // One event of an alive particle (one SimulationMCStep iteration): its
+    // ray goes into the wave's walk, which all lanes run together (also
+    // those without a particle), then finish() treats what it met.
+    __device__ void trace_ray(uint32_t lane, bool alive) {
+        int32_t root = -1;
+        if (alive) {
+            ++nb_events;
+            root = P.roots[var->root_base + (uint32_t)structure];
+            walk_load(W, lane, pos, dir, last_hit, 1e300);
+        }
+        const CoinState cs{rng.k0, rng.k1, rng.p0, rng.p1, nb_events, time, var};
+        walk<(FEAT & FEAT_TRANSPARENT) != 0>(P, W, lnodes, lane, alive, root, cs);
+        // the ray is read back from its slot: not held in registers meanwhile
+        const double2 a = W.p01[lane], b = W.p2d0[lane], c = W.d12[lane];
+        pos = mk(a.x, a.y, b.x);
+        dir = mk(b.y, c.x, c.y);
+    }
     // Returns false when the particle ends.
-    __device__ bool step() {
+    __device__ bool finish(uint32_t lane) {
         constexpr bool TR = (FEAT & FEAT_TRANSPARENT) != 0;
-        ++nb_events;
-        int32_t root = P.roots[var->root_base + (uint32_t)structure];
-        HitRec h = traverse<TR>(P, root, pos, dir, last_hit, 1e300, S, &rng, nb_events, var,
-                                time, false, lnodes);
+        HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
         if (h.facet < 0) {  // leak
             ++acc_leak;
             unsigned long long at = atomicAdd(P.leak_count, 1ull);
@@ -1528,6 +1626,8 @@ struct Tracer {
         if constexpr (TR) {
             if (var->flags & FEAT_TRANSPARENT) {
                 // second walk: every transparent pass closer than `travel`
+                const int32_t root = P.roots[var->root_base + (uint32_t)structure];
+                const LaneStack S{W.nodes + lane, MFG_LANE_STACK, P.stack_total, spill};
                 Ray32 r = make_ray32(pos, dir);
                 float tbf = widen(travel);
                 uint32_t sp = 0;
@@ -1566,6 +1666,7 @@ struct Tracer {
                 hu = save_u; hv = save_v;
             }
         }
+        if (ev == 0) hit_uv(P.facets + h.facet, pos, dir, h.t, h.u, h.v);
         pos = add(pos, scl(travel, dir));
         time += travel / 100.0 / vel;
         if (ev == 0) {
@@ -1624,15 +1725,14 @@ __device__ __forceinline__ uint32_t find_variant(const uint64_t* prefix, uint32_
 
 template <uint32_t FEAT>
 __device__ __forceinline__ void trace_body(const TraceParams& P) {
-    extern __shared__ int32_t lds_stack[];
+    extern __shared__ __align__(16) unsigned char lds_base[];
     const uint32_t lane = __lane_id();
+    WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     const size_t gl = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const LaneStack lane_stack{lds_stack + threadIdx.x, blockDim.x, P.stack_size, P.stack_total,
-                               P.stack_spill ? P.stack_spill + gl * (P.stack_total - P.stack_size)
-                                             : lds_stack + threadIdx.x};
-    Tracer<FEAT> T(P, lane_stack);
-    // hot-facet counters after the stacks (stack bytes are a multiple of 8)
-    double* hot = reinterpret_cast<double*>(lds_stack + (size_t)blockDim.x * P.stack_size);
+    int32_t* spill = P.stack_spill ? P.stack_spill + gl * (P.stack_total - MFG_LANE_STACK) : nullptr;
+    Tracer<FEAT> T(P, W, spill);
+    // hot-facet counters after the waves' walk areas
+    double* hot = reinterpret_cast<double*>(lds_base + (blockDim.x >> 6) * sizeof(WaveLds));
     for (uint32_t i = threadIdx.x; i < 8u * P.n_hot; i += blockDim.x) hot[i] = 0.0;
     // then the block's copy of the top of the tree (128 B per node; the
     // offsets above are multiples of 64 B)
@@ -1649,7 +1749,9 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
         T.seg_t = P.adj_seg_t + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * MFG_ADJ_SEG;
         T.seg_x = P.adj_seg_x + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * MFG_ADJ_SEG;
     }
-    bool alive = false, done = false;
+    // few work items are spread over all waves: lanes beyond the quota stay
+    // without a particle and help with the others' walks
+    bool alive = false, done = lane >= P.lane_quota;
     uint32_t vi = 0;
     uint64_t events_left = 0;
     // work items: first the particles the previous launch left in flight,
@@ -1776,8 +1878,9 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
             break;
         }
         if (!__ballot(!done)) break;
+        T.trace_ray(lane, alive);
         if (alive) {
-            alive = T.step();
+            alive = T.finish(lane);
             if (alive && --events_left == 0) alive = false;
         }
         // slot-0 facet counters of this iteration: lanes that updated the
@@ -1898,23 +2001,34 @@ __global__ void k_carry_flip(unsigned long long* ctl, const unsigned long long* 
     }
 }
 
+// Fixed ray batches: a wave takes p.rays_per_wave rays at a time.
 __global__ void __launch_bounds__(256) k_intersect(IsectParams p) {
-    extern __shared__ int32_t lds_stack[];
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= p.n) return;
+    extern __shared__ __align__(16) unsigned char lds_base[];
+    const uint32_t lane = __lane_id();
+    WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     TraceParams tp{};
-    tp.facets = p.facets; tp.poly = p.poly; tp.nodes = p.nodes; tp.leaves = p.leaves; tp.leaf_uv = p.leaf_uv;
-    d3 P = ld3(p.origins + 3 * i), D = ld3(p.dirs + 3 * i);
-    int32_t skip = p.last_hit ? p.last_hit[i] : -1;
-    if (skip >= 0) skip += (int32_t)p.facet_base;
-    // the whole stack is in LDS here (cap == lds_cap): the spill pointer is never used
-    const LaneStack S{lds_stack + threadIdx.x, blockDim.x, p.stack_size, p.stack_size, lds_stack + threadIdx.x};
-    HitRec h = traverse<false>(tp, p.root, P, D, skip, 1e300, S,
-                               nullptr, 0, nullptr, 0.0, true, nullptr);
-    p.out_facet[i] = h.facet >= 0 ? h.facet - (int32_t)p.facet_base : -1;
-    p.out_t[i] = h.facet >= 0 ? h.t : 0.0;
-    p.out_u[i] = h.u;
-    p.out_v[i] = h.v;
+    tp.poly = p.poly; tp.nodes = p.nodes; tp.leaves = p.leaves; tp.leaf_uv = p.leaf_uv; tp.task_bits = p.task_bits;
+    const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const uint64_t i = wave * p.rays_per_wave + lane;
+    const bool live = lane < p.rays_per_wave && i < p.n;
+    d3 P = mk(0, 0, 0), D = mk(0, 0, 1);
+    if (live) {
+        P = ld3(p.origins + 3 * i);
+        D = ld3(p.dirs + 3 * i);
+        int32_t skip = p.last_hit ? p.last_hit[i] : -1;
+        if (skip >= 0) skip += (int32_t)p.facet_base;
+        walk_load(W, lane, P, D, skip, 1e300);
+    }
+    walk<false>(tp, W, nullptr, lane, live, p.root, CoinState{});
+    if (!live) return;
+    const int32_t f = W.facet[lane];
+    const double t = __longlong_as_double((long long)W.t[lane]);
+    double u = 0.0, v = 0.0;
+    if (f >= 0) hit_uv(p.facets + f, P, D, t, u, v);
+    p.out_facet[i] = f >= 0 ? f - (int32_t)p.facet_base : -1;
+    p.out_t[i] = f >= 0 ? t : 0.0;
+    p.out_u[i] = u;
+    p.out_v[i] = v;
 }
 
 __global__ void k_zero(uint64_t* p, uint64_t n) {
@@ -2011,7 +2125,7 @@ int mfg_trace_occupancy(uint32_t features, int waves, int block, size_t lds) {
 }
 
 int mfg_launch_trace(const TraceParams& p, uint32_t features, int waves, int grid, int block, void* stream) {
-    size_t lds = (size_t)block * p.stack_size * sizeof(int32_t) + (size_t)p.n_hot * 8 * sizeof(double) +
+    size_t lds = (size_t)(block / 64) * sizeof(WaveLds) + (size_t)p.n_hot * 8 * sizeof(double) +
                  (size_t)p.lds_nodes * sizeof(BvhNode);
     const uint32_t f = mfg_trace_kernel_features(features);
     TraceKernel k = block > 256 ? kernel_cu(f, block / 256) : kernel_for(f, waves);
@@ -2034,10 +2148,10 @@ int mfg_launch_carry_flip(unsigned long long* ctl, const unsigned long long* cla
 
 int mfg_launch_intersect(const IsectParams& p, void* stream) {
     const int block = 256;
-    uint64_t grid = (p.n + block - 1) / block;
+    const uint64_t waves = (p.n + p.rays_per_wave - 1) / p.rays_per_wave;
+    const uint64_t grid = (waves + block / 64 - 1) / (block / 64);
     if (grid == 0) return 0;
-    size_t lds = (size_t)block * p.stack_size * sizeof(int32_t);
-    hipLaunchKernelGGL(k_intersect, dim3((uint32_t)grid), dim3(block), lds, (hipStream_t)stream, p);
+    hipLaunchKernelGGL(k_intersect, dim3((uint32_t)grid), dim3(block), (block / 64) * sizeof(WaveLds), (hipStream_t)stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

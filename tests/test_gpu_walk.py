@@ -1,0 +1,64 @@
+"""The wave's shared ray walk: batches at the edges of a wave and models
+whose boxes nearly all overlap, so that a node step hits most of its
+children and the task stack and the facet list run into their capacities.
+First hits against the oracle's brute force, bit for bit. Needs an MI355X."""
+import numpy as np
+import pytest
+
+from helpers import random_rays
+from molflow_sources_amd import geometry
+from molflow_sources_amd.model import Model, default_facets
+from oracle.mfcpu import CpuModel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sim():
+    from molflow_sources_amd.simulation import GpuSimulation
+    s = GpuSimulation(0)
+    yield s
+    s.close()
+
+
+def triangle_soup(n, seed=3):
+    """n large random 2-sided triangles through the middle of a 10 cm cube."""
+    rng = np.random.default_rng(seed)
+    V = rng.uniform(0.0, 10.0, (3 * n, 3))
+    F = default_facets(n)
+    F["is_2sided"] = 1
+    F["sticking"] = 0.5
+    F["desorb_type"][0], F["outgassing"][0] = 2, 1.0
+    return Model(V, np.arange(3 * n).reshape(n, 3).tolist(), F, name="soup")
+
+
+@pytest.mark.parametrize("width,leaf", [(8, 1), (8, 2), (8, 16), (4, 2)])
+@pytest.mark.parametrize("n_rays", [1, 63, 65, 140_000])
+def test_overlapping_boxes_first_hits(sim, width, leaf, n_rays):
+    m = triangle_soup(1500)
+    sim.load(m)
+    sim.rebuild_accel(width, leaf)
+    o, d = random_rays(n_rays, [-1] * 3, [11] * 3, seed=5)
+    last = np.random.default_rng(6).integers(-1, m.n_facets, n_rays).astype(np.int32)
+    got = sim.intersect(o, d, last)
+    ref = CpuModel(m).intersect(o, d, last, brute=True)
+    assert np.array_equal(got[0], ref[0]), f"{int((got[0] != ref[0]).sum())} first-hit facets differ"
+    hit = ref[0] >= 0
+    for a, b in zip(got[1:], ref[1:]):
+        assert np.allclose(a[hit], b[hit], rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("n_des", [1, 64, 3071, 3073, 200_001])
+def test_lane_quota_same_seed_tallies(sim, n_des):
+    """Runs of fewer particles than waves, of about one per wave and of more
+    than lanes (lane quota 1, 1, 2, 64) count what the oracle counts."""
+    m = geometry.tube_model(1.0, 3.0, 16, 6)
+    sim.load(m)
+    sim.rebuild_accel()
+    sim.reset(seed=9)
+    sim.run(n_des)
+    t, c = sim.read(), CpuModel(m).run(n_des, seed=9)
+    assert t.desorbed == n_des
+    a, b = t.facets[0]["nb_mc_hit"].astype(np.int64), c.facets[0]["nb_mc_hit"].astype(np.int64)
+    # a few long trajectories may part by FP64 rounding of the math library
+    assert np.abs(a - b).sum() <= 2e-4 * b.sum()
