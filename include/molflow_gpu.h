@@ -423,10 +423,10 @@ int mfg_read_variant_tallies(mfg_context* ctx, uint32_t variant, const mfg_tally
 /* Launch shape used by runs: threads per block (a multiple of 64 up to
  * 256, 768 or 1024) and blocks per CU (0 = defaults / autotuned). 768 and
  * 1024 run one block per CU at 3 and 4 waves per SIMD, whose LDS copy of
- * the top of the BVH is then shared by the whole CU; they apply to models
- * without transparency, moments, volume events and the other features of
- * the full kernel (those runs take 256-thread blocks). MFG_ERR_INVALID for
- * other sizes. */
+ * the top of the BVH is then shared by the whole CU; they apply to a single
+ * model without transparency, moments, volume events and the other features
+ * of the full kernel (other runs take 256-thread blocks). MFG_ERR_INVALID
+ * for other sizes. */
 int mfg_set_launch(mfg_context* ctx, uint32_t block_threads, uint32_t blocks_per_cu);
 /* Particles kept in flight between runs (the particle state that persists
  * between SimulationMCStep calls, reference Particle.h:95-122 and
@@ -445,8 +445,9 @@ int mfg_set_carry(mfg_context* ctx, int enable);
 /* Number of particles parked on the device after the last run. */
 int mfg_in_flight(const mfg_context* ctx, uint64_t* n);
 
-/* Occupancy bound of the trace kernel: waves per SIMD (1..5; 0 = default).
- * Higher bounds cap registers (cold state spills) to hide more latency. */
+/* Occupancy bound of the trace kernel: waves per SIMD (1..5; 0 = default;
+ * the highest built is 4, and 5 runs as 4). Higher bounds cap registers
+ * (cold state spills) to hide more latency. */
 int mfg_set_kernel_variant(mfg_context* ctx, uint32_t waves_per_simd);
 
 /* Launch autotuner: times short probe runs of n_probe desorptions for every

@@ -890,6 +890,7 @@ struct mfg_context {
     // device data
     DevBuf<DFacet> facets;
     DevBuf<DPhys> phys;
+    DevBuf<DHit> hits;                   // derived from facets and phys (upload_phys)
     DevBuf<double> poly, src_cum, og_cdf, tab_x, tab_y, mom_start, mom_end, tex_inc, am_src;
     DevBuf<int32_t> src_facet, roots;
     DevBuf<LeafFacet> leaves;
@@ -976,6 +977,24 @@ void reset_graph(mfg_context* c) {
     c->graph_key.clear();
 }
 
+// Uploads the physics records and the wall-event records made from them.
+void upload_phys(mfg_context* c) {
+    std::vector<DHit> hits(c->h_phys.size());
+    for (size_t f = 0; f < hits.size(); ++f) {
+        const DFacet& F = c->h_facets[f];
+        const DPhys& ph = c->h_phys[f];
+        DHit& h = hits[f];
+        for (int k = 0; k < 3; ++k) { h.N[k] = F.N[k]; h.nU[k] = ph.nU[k]; h.nV[k] = ph.nV[k]; }
+        h.sticking = ph.sticking; h.sqrt_temp = ph.sqrt_temp;
+        h.flags = ph.flags | (ph.sticking_param >= 0 ? FF_TD_STICKING : 0u) | (ph.temperature_param >= 0 ? FF_TD_TEMP : 0u);
+        h.hot_idx = ph.hot_idx; h.adj_group = ph.adj_group; h.adj_target = ph.adj_target;
+        h.accomodation = ph.accomodation; h.diffuse = ph.diffuse; h.specular = ph.specular;
+    }
+    c->phys.upload(c->h_phys, c->stream);
+    c->hits.upload(hits, c->stream);
+    HIPCHK(hipStreamSynchronize(c->stream));
+}
+
 // Marks the hot facets in the physics records and stores the index of each
 // one's slot-0 counter record.
 void set_hot_facets(mfg_context* c, const std::vector<int32_t>& hot, bool upload) {
@@ -990,7 +1009,7 @@ void set_hot_facets(mfg_context* c, const std::vector<int32_t>& hot, bool upload
         idx.push_back(c->dvars[vi].fc_base + (uint64_t)(uint32_t)ph.local_id);
     }
     c->hot_fc.upload(idx, c->stream);
-    if (upload) c->phys.upload(c->h_phys, c->stream);
+    if (upload) upload_phys(c);
     HIPCHK(hipStreamSynchronize(c->stream));
     reset_graph(c);
 }
@@ -1119,8 +1138,9 @@ void upload_models(mfg_context* c) {
     }
     c->hot.clear();
     set_hot_facets(c, hot, false);
-    c->facets.upload(facets, s); c->phys.upload(c->h_phys, s); c->poly.upload(poly, s);
     c->h_facets = facets;
+    c->facets.upload(facets, s); c->poly.upload(poly, s);
+    upload_phys(c);
     c->h_poly = poly;
     c->src_cum.upload(src_cum, s); c->src_facet.upload(src_facet, s); c->og_cdf.upload(og_cdf, s);
     c->am_src.upload(am_src, s);
@@ -1318,6 +1338,9 @@ uint32_t lds_node_count(const mfg_context* c, int block, int waves) {
 
 TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     TraceParams p{};
+    p.one = c->dvars[0];
+    p.one_root = c->dvars.size() == 1 && c->dvars[0].n_struct == 1 ? c->h_roots.at(c->dvars[0].root_base) : -2;
+    p.hits = c->hits.p;
     p.facets = c->facets.p; p.phys = c->phys.p; p.poly = c->poly.p; p.nodes = c->nodes.p;
     p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p; p.roots = c->roots.p; p.variants = c->variants.p;
     p.var_prefix = c->prefix.p; p.n_variants = (uint32_t)c->dvars.size();
@@ -1360,14 +1383,14 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
         // the one-block-per-CU kernels exist for the lean and low-flux
         // feature sets (768 lanes: 3 waves per SIMD, 1024: 4); other runs
         // take 256-lane blocks
-        if (mfg_trace_has_cu_block(feats, block)) waves = block / 256;
+        if (mfg_trace_has_cu_block(feats, c->dvars.size() == 1, block)) waves = block / 256;
         else block = 256;
     }
     auto lds_bytes = [&](int b) {
         return (size_t)(b / 64) * MFG_WAVE_LDS + c->hot.size() * 8 * sizeof(double) +
                (size_t)lds_node_count(c, b, waves) * sizeof(BvhNode);
     };
-    if (block > 256 && mfg_trace_occupancy(feats, waves, block, lds_bytes(block)) < 1) {
+    if (block > 256 && mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block)) < 1) {
         block = 256;   // the block's LDS does not fit
         waves = c->waves ? c->waves : default_waves(feats);
     }
@@ -1375,7 +1398,7 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
     if (block > 256) per_cu = 1;
     if (per_cu == 0) {
         // fill every CU to its occupancy limit (persistent launch)
-        int occ = mfg_trace_occupancy(feats, waves, block, lds_bytes(block));
+        int occ = mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block));
         per_cu = (uint32_t)std::max(1, occ);
     }
     grid = (int)(per_cu * (uint32_t)c->n_cu);
@@ -1464,7 +1487,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
             (c->adj_groups && mfg_launch_zero(c->counters.p + 8, sizeof(unsigned long long), s)))
             throw Err(MFG_ERR_DEVICE, "zero kernel launch failed");
         if (events) HIPCHK(hipEventRecord(c->ev0, s));
-        if (mfg_launch_trace(p, feats, waves, grid, block, s)) throw Err(MFG_ERR_DEVICE, std::string("trace launch failed: ") + hipGetErrorString(hipGetLastError()));
+        if (mfg_launch_trace(p, feats, nv == 1, waves, grid, block, s)) throw Err(MFG_ERR_DEVICE, std::string("trace launch failed: ") + hipGetErrorString(hipGetLastError()));
         if (p.carry && mfg_launch_carry_flip(p.carry_ctl, p.next_particle, p.carry, p.carry_cap, c->counters.p + 7, s))
             throw Err(MFG_ERR_DEVICE, "carry flip launch failed");
     };
@@ -2065,7 +2088,7 @@ int mfg_autotune(mfg_context* c, uint64_t n_probe, mfg_tune_result* out) {
                 for (uint32_t b : blocks) {
                     // last: one block per CU of 768 and of 1024 lanes, where the kernel exists
                     const uint32_t cu_block = i == nw ? 768u : 1024u;
-                    if (i >= nw && (b != blocks[0] || !mfg_trace_has_cu_block(feats, (int)cu_block))) continue;
+                    if (i >= nw && (b != blocks[0] || !mfg_trace_has_cu_block(feats, nv == 1, (int)cu_block))) continue;
                     c->waves = i < nw ? wl[i] : (int)cu_block / 256; c->block = i < nw ? b : cu_block; c->blocks_per_cu = 0;
                     mfg_step_result sr{};
                     run_variants(c, nd.data(), seeds.data(), 0, &sr);
@@ -2139,7 +2162,7 @@ int mfg_adjoint_setup(mfg_context* c, const int32_t* group_of_facet, uint32_t G,
             if (targets[t] < 0 || (uint32_t)targets[t] >= nF) throw Err(MFG_ERR_INVALID, "target facet out of range");
             phys[targets[t]].adj_target = (int32_t)t;
         }
-        c->phys.upload(phys, c->stream);
+        upload_phys(c);
         c->adj_groups = G; c->adj_targets = T;
         c->adj_j0.alloc(T); c->adj_jac.alloc((size_t)T * G); c->adj_s.alloc(G);
         c->adj_up.alloc(T); c->adj_grad.alloc(G);

@@ -70,6 +70,8 @@ enum : uint32_t {
     FF_DIFFUSE = 1u << 17,      // diffuse_part > 0.999999
     FF_FULL_ACC = 1u << 18,     // accomodation > 0.9999
     FF_OGMAP = 1u << 19,
+    FF_TD_STICKING = 1u << 20,  // DHit::flags only: sticking / temperature from a
+    FF_TD_TEMP = 1u << 21,      // time-dependent parameter (DPhys names it)
 };
 
 struct alignas(16) DFacet {
@@ -118,6 +120,20 @@ struct alignas(16) DPhys {
     int32_t hot_idx;                // slot in the per-block hot-facet counter table, -1
     int32_t pad2_;
 };
+
+// What a wall event always needs of its facet, in one line: loaded as six
+// 16 B loads issued together (the last three words only by facets that are
+// not purely diffuse or thermalising). DFacet and DPhys are read beyond it
+// only for what the flags name (recordings, teleports, parameters).
+struct alignas(128) DHit {
+    double N[3], nU[3], nV[3];
+    double sticking, sqrt_temp;
+    uint32_t flags;                 // DPhys::flags + FF_TD_*
+    int32_t hot_idx;                // as in DPhys
+    int32_t adj_group, adj_target;
+    double accomodation, diffuse, specular;
+};
+static_assert(sizeof(DHit) == 128, "DHit must be one 128-byte line");
 
 // One BVH node of up to 8 children in one 128 B line. Child boxes are
 // quantised to 8-bit steps per plane relative to the node's origin with a
@@ -252,6 +268,12 @@ struct CarryRec {
 static_assert(sizeof(CarryRec) == 200, "CarryRec layout");
 
 struct TraceParams {
+    // a launch of one variant (the kernels built for it): its constants,
+    // read as scalars; seed and pid_base change between replays of a captured
+    // launch and are read from `variants`
+    DVariant one;
+    int32_t one_root;                 // root of its only structure, or -2: look it up
+    const DHit* hits;
     const DFacet* facets;
     const DPhys* phys;
     const double* poly;               // (u,v) pairs
@@ -373,7 +395,8 @@ struct StaticRays {
 int mfg_scratch_address(int device, StaticRays** out);
 
 // kernel launchers (mfg_trace.hip)
-int mfg_launch_trace(const TraceParams& p, uint32_t features, int waves, int grid, int block, void* stream);
+// (single: the launch has one variant, whose constants are in p.one)
+int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int waves, int grid, int block, void* stream);
 int mfg_launch_intersect(const IsectParams& p, void* stream);
 // after a carry launch: append the parked particles the launch did not
 // claim (time limit) to the output half, then swap the halves
@@ -383,8 +406,8 @@ int mfg_launch_zero(void* ptr, uint64_t bytes, void* stream);
 int mfg_launch_backward(const double* jac, const double* up, double* grad, uint32_t n_targets, uint32_t n_groups,
                         double scale, void* stream);
 uint32_t mfg_trace_kernel_features(uint32_t model_features);
-int mfg_trace_occupancy(uint32_t features, int waves, int block, size_t lds_bytes);
+int mfg_trace_occupancy(uint32_t features, bool single, int waves, int block, size_t lds_bytes);
 int mfg_trace_variants(uint32_t features, int* waves_out, int cap);
 // 1 when the feature set has a one-block-per-CU kernel of `block` lanes
-// (768: 3 waves per SIMD, 1024: 4)
-int mfg_trace_has_cu_block(uint32_t features, int block);
+// (768: 3 waves per SIMD, 1024: 4); only for launches of one variant
+int mfg_trace_has_cu_block(uint32_t features, bool single, int block);

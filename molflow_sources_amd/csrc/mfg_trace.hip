@@ -105,7 +105,7 @@ __device__ __forceinline__ unsigned long long wave_sum_u(unsigned long long v) {
 // ------------------------------------------------------------------ tables
 struct XYRef { const double* x; const double* y; uint32_t n; };
 
-__device__ double interp_y(double x, XYRef t, bool logx, bool logy, bool extrapolate) {
+__device__ __forceinline__ double interp_y(double x, XYRef t, bool logx, bool logy, bool extrapolate) {
     uint32_t n = t.n;
     if (n == 0) return 0.0;
     if (n == 1) return t.y[0];
@@ -148,7 +148,7 @@ __device__ double interp_x_guided(double y, XYRef t, const uint32_t* guide, uint
     return x0 + (y - y0) * (x1 - x0) / (y1 - y0);
 }
 
-__device__ double interp_x(double y, XYRef t) {
+__device__ __forceinline__ double interp_x(double y, XYRef t) {
     uint32_t n = t.n;
     if (n == 1) return t.x[0];
     uint32_t i;
@@ -777,9 +777,38 @@ __device__ __forceinline__ void hit_uv(const DFacet* __restrict__ F, d3 P, d3 D,
     v = fdot(r, ld3(F->V)) * F->invV2;
 }
 
+// A wall event's facet in registers (DHit without its rarely used words).
+struct HitRegs {
+    d3 N, nU, nV;
+    double sticking, sqrt_temp;
+    uint32_t flags;
+    int32_t hot;
+};
+__device__ __forceinline__ HitRegs load_hit(const DHit* __restrict__ h) {
+    const double2* q = reinterpret_cast<const double2*>(h);
+    const double2 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3], q4 = q[4];
+    const uint4 q5 = reinterpret_cast<const uint4*>(h)[5];
+    return {mk(q0.x, q0.y, q1.x), mk(q1.y, q2.x, q2.y), mk(q3.x, q3.y, q4.x), q4.y,
+            __longlong_as_double((long long)(((unsigned long long)q5.y << 32) | q5.x)), q5.z, (int32_t)q5.w};
+}
+
+#define MFG_IN __device__ __forceinline__
+
 // ------------------------------------------------------------------ tracer
-template <uint32_t FEAT>
+// ONE: the launch has a single variant, whose constants come with the kernel
+// arguments (scalar loads, no round trip on the event's path); otherwise
+// every lane follows its own variant's record.
+// Without a feature that reads them, a particle has no clock, path length,
+// decay time, hit position or bounce count (CLOCKED false: they would be
+// live across every walk), and its weight is 1 without low flux. With one
+// line read per event and these constants at hand, the event of a lone
+// particle took 10,000 instead of 21,000 cycles (most of it serial loads),
+// that of a full wave on the beam pipe 54,000 instead of 86,000; beam-pipe
+// launch 91.3 -> 72.5 ms, textured tube 18.2 -> 14.5 ms, low flux 165 -> 120.
+template <uint32_t FEAT, bool ONE>
 struct Tracer {
+    static constexpr bool CLOCKED = (FEAT & FEAT_ALL & ~(uint32_t)FEAT_LOWFLUX) != 0;
+    static constexpr bool WEIGHTED = (FEAT & FEAT_LOWFLUX) != 0;
     const TraceParams& P;
     WaveLds& W;                       // this wave's walk area
     int32_t* spill;                   // this lane's stack entries beyond the LDS part (second walk)
@@ -788,11 +817,12 @@ struct Tracer {
     double time, vel, ori, gen_time, dist, decay_t, scatter_path, hu, hv;
     int32_t structure, last_hit, tele_from;
     uint32_t nb_bounces, nb_events;
-    uint64_t pid;
     Rng rng;
     const DVariant* var;
-    // lane accumulators (flushed once per wave)
-    uint32_t acc_hits, acc_des;
+    // lane accumulators (flushed once per wave); unweighted particles need
+    // neither weight sum, and without a clock every path ends on a facet, so
+    // the two path sums are one
+    uint32_t acc_hits, acc_des, acc_absorbed;
     double acc_hit_equiv, acc_abs_equiv, acc_dist_total, acc_dist_full;
     uint32_t acc_leak, acc_decay;
     uint32_t tr_n;
@@ -803,12 +833,12 @@ struct Tracer {
     double* hot;                      // LDS table of the hot facets' slot-0 counters (8 words each)
     const uint4* lnodes;              // LDS copy of the first P.lds_nodes BVH nodes
     // pending slot-0 facet counter update of this lane
-    int32_t pend_f;
+    int32_t pend_f, pend_hot;
     uint32_t pend_hits;
     double pend_he, pend_abs, pend_s1v, pend_svo, pend_s1pv;
 
-    __device__ Tracer(const TraceParams& p, WaveLds& w, int32_t* sp) : P(p), W(w), spill(sp) {
-        acc_hits = acc_des = 0;
+    MFG_IN Tracer(const TraceParams& p, WaveLds& w, int32_t* sp) : P(p), W(w), spill(sp) {
+        acc_hits = acc_des = acc_absorbed = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
         acc_leak = acc_decay = 0;
         tr_n = 0;
@@ -819,15 +849,34 @@ struct Tracer {
         var = nullptr;
         hot = nullptr;
         lnodes = nullptr;
+        ori = 1.0;
+        time = gen_time = dist = hu = hv = 0.0;
+        decay_t = scatter_path = 1e100;
+        tele_from = -1;
+        nb_bounces = nb_events = 0;
         clear_pending();
     }
 
-    __device__ int32_t local(int32_t f) const { return f - (int32_t)var->facet_base; }
+    MFG_IN const DVariant& vc() const {
+        if constexpr (ONE) return P.one;
+        else return *var;
+    }
+    MFG_IN uint64_t pid() const { return ((uint64_t)rng.p1 << 32) | rng.p0; }
+    MFG_IN double w() const {         // the particle's weight
+        if constexpr (WEIGHTED) return ori;
+        else return 1.0;
+    }
+    MFG_IN void add_hit() {
+        ++acc_hits;
+        if constexpr (WEIGHTED) acc_hit_equiv += ori;
+    }
 
-    __device__ void trace(int32_t f, int32_t kind) {
+    MFG_IN int32_t local(int32_t f) const { return f - (int32_t)vc().facet_base; }
+
+    MFG_IN void trace(int32_t f, int32_t kind) {
         if constexpr ((FEAT & FEAT_TRACE) != 0) {
-            if (pid < P.trace_n && tr_n < P.trace_k) {
-                size_t at = (size_t)pid * P.trace_k + tr_n;
+            if (pid() < P.trace_n && tr_n < P.trace_k) {
+                size_t at = (size_t)pid() * P.trace_k + tr_n;
                 P.trace_facet[at] = f < 0 ? f : local(f);
                 P.trace_kind[at] = kind;
                 ++tr_n;
@@ -835,60 +884,64 @@ struct Tracer {
         }
         (void)f; (void)kind;
     }
-    __device__ int moment(double t) const {
+    MFG_IN int moment(double t) const {
         if constexpr ((FEAT & FEAT_MOMENTS) != 0) {
-            uint32_t n = var->n_moments;
+            uint32_t n = vc().n_moments;
             if (n == 0) return -1;
-            const double* S = P.mom_start + var->mom_base;
+            const double* S = P.mom_start + vc().mom_base;
             uint32_t lo = 0, hi = n;  // first start >= t
             while (lo < hi) { uint32_t mid = (lo + hi) / 2; if (S[mid] < t) lo = mid + 1; else hi = mid; }
             uint32_t lb = lo;
             if (lb != 0) --lb;
-            if (S[lb] <= t && t < P.mom_end[var->mom_base + lb]) return (int)lb + 1;
+            if (S[lb] <= t && t < P.mom_end[vc().mom_base + lb]) return (int)lb + 1;
         }
         (void)t;
         return -1;
     }
-    __device__ double param_at(int32_t id, double t, double c) const {
+    MFG_IN double param_at(int32_t id, double t, double c) const {
         if constexpr ((FEAT & FEAT_TDPARAM) != 0) {
             if (id >= 0) {
-                const DTable tb = P.params[var->param_base + id];
+                const DTable tb = P.params[vc().param_base + id];
                 return interp_y(t, XYRef{P.tab_x + tb.off, P.tab_y + tb.off, tb.n}, tb.log_x, tb.log_y, false);
             }
         }
         (void)id; (void)t;
         return c;
     }
-    __device__ double sticking(const DPhys& ph) const {
+    MFG_IN double sticking(const HitRegs& H, int32_t f) const {
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
-            if (ph.adj_group >= 0) return P.adj_sticking[ph.adj_group];
+            const int32_t g = P.hits[f].adj_group;
+            if (g >= 0) return P.adj_sticking[g];
         }
-        return param_at(ph.sticking_param, time, ph.sticking);
+        if constexpr ((FEAT & FEAT_TDPARAM) != 0) {
+            if (H.flags & FF_TD_STICKING) return param_at(P.phys[f].sticking_param, time, H.sticking);
+        }
+        return H.sticking;
     }
-    __device__ double temperature(const DPhys& ph) const { return param_at(ph.temperature_param, time, ph.temperature); }
+    MFG_IN double temperature(const DPhys& ph) const { return param_at(ph.temperature_param, time, ph.temperature); }
 
-    __device__ mfg_facet_counters* fc(const DPhys& ph, int slot) const {
-        return P.fc + var->fc_base + (size_t)slot * var->n_facets + (uint32_t)ph.local_id;
+    MFG_IN mfg_facet_counters* fc(int32_t f, int slot) const {
+        return P.fc + vc().fc_base + (size_t)slot * vc().n_facets + (uint32_t)local(f);
     }
 
     // IncreaseFacetCounter (Particle.cpp:1193-1230). Slot 0 goes to the
     // lane's pending record (summed across the wave before the atomics);
     // moment slots and force terms go straight to memory.
-    __device__ void counter(const DPhys& ph, int m, uint32_t hit, uint32_t des, uint32_t abs_, double s1v, double svo,
+    MFG_IN void counter(const HitRegs& H, int32_t f, int m, uint32_t hit, uint32_t des, uint32_t abs_, double s1v, double svo,
                             d3 imp, d3 imp2, d3 impm) {
-        double he = (double)hit * ori;
+        double he = (double)hit * w();
         double s1pv = (hit || des) ? (he + (double)des) / vel : 0.0;
         bool force = false;
-        if constexpr ((FEAT & FEAT_FORCE) != 0) force = var->enable_force != 0;
-        int32_t gf = ph.local_id + (int32_t)var->facet_base;
+        if constexpr ((FEAT & FEAT_FORCE) != 0) force = vc().enable_force != 0;
         if (!force && des == 0) {
-            if (pend_f >= 0 && pend_f != gf) flush_pending_direct();
-            pend_f = gf;
+            if constexpr (CLOCKED) { if (pend_f >= 0 && pend_f != f) flush_pending_direct(); }
+            pend_f = f;
+            pend_hot = H.hot;
             pend_hits += hit;
             pend_he += he;
-            pend_abs += (double)abs_ * ori;
-            pend_s1v += ori * s1v;
-            pend_svo += ori * svo;
+            pend_abs += (double)abs_ * w();
+            pend_s1v += w() * s1v;
+            pend_svo += w() * svo;
             pend_s1pv += s1pv;
         }
 #pragma unroll
@@ -896,16 +949,16 @@ struct Tracer {
             int slot = k == 0 ? 0 : m;
             if (k == 1 && m <= 0) break;
             if (k == 0 && !force && des == 0) continue;
-            mfg_facet_counters* c = fc(ph, slot);
+            mfg_facet_counters* c = fc(f, slot);
             if (hit) { atomic_addu(&c->nb_mc_hit, hit); atomic_addd(&c->nb_hit_equiv, he); }
             if (des) atomic_addu(&c->nb_desorbed, des);
-            if (abs_) atomic_addd(&c->nb_abs_equiv, (double)abs_ * ori);
-            if (s1v != 0.0) atomic_addd(&c->sum_1_per_ort_velocity, ori * s1v);
-            if (svo != 0.0) atomic_addd(&c->sum_v_ort, ori * svo);
+            if (abs_) atomic_addd(&c->nb_abs_equiv, (double)abs_ * w());
+            if (s1v != 0.0) atomic_addd(&c->sum_1_per_ort_velocity, w() * s1v);
+            if (svo != 0.0) atomic_addd(&c->sum_v_ort, w() * svo);
             if (hit || des) atomic_addd(&c->sum_1_per_velocity, s1pv);
             if constexpr ((FEAT & FEAT_FORCE) != 0) {
                 if (force) {
-                    double* fo = P.force + var->force_base + ((size_t)slot * var->n_facets + (uint32_t)ph.local_id) * 9;
+                    double* fo = P.force + vc().force_base + ((size_t)slot * vc().n_facets + (uint32_t)local(f)) * 9;
                     atomic_addd(fo + 0, ori * imp.x); atomic_addd(fo + 1, ori * imp.y); atomic_addd(fo + 2, ori * imp.z);
                     atomic_addd(fo + 3, ori * imp2.x); atomic_addd(fo + 4, ori * imp2.y); atomic_addd(fo + 5, ori * imp2.z);
                     atomic_addd(fo + 6, ori * impm.x); atomic_addd(fo + 7, ori * impm.y); atomic_addd(fo + 8, ori * impm.z);
@@ -913,24 +966,24 @@ struct Tracer {
             }
         }
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
-            if (hit && ph.adj_target >= 0) adjoint_score(ph, he, false);
+            const int32_t at = P.hits[f].adj_target;
+            if (hit && at >= 0) adjoint_score(at, P.hits[f].adj_group, he, false);
         }
         (void)imp; (void)imp2; (void)impm;
     }
     // Without low-flux weighting every particle weighs 1, so the slot-0
     // nb_hit_equiv equals nb_mc_hit: it is not added here (one atomic less
     // per hit) and the host fills it in when it reads the counters.
-    __device__ bool weighted() const {
-        if constexpr ((FEAT & FEAT_LOWFLUX) != 0) return var->low_flux != 0;
+    MFG_IN bool weighted() const {
+        if constexpr (WEIGHTED) return vc().low_flux != 0;
         return false;
     }
     // Atomics of this lane's pending slot-0 record, then clear it.
-    __device__ void flush_pending_direct() {
+    MFG_IN void flush_pending_direct() {
         if (pend_f < 0) return;
-        const DPhys& ph = P.phys[pend_f];
         const bool w = weighted();
-        if (ph.hot_idx >= 0) {
-            double* h = hot + 8 * ph.hot_idx;   // same field order as mfg_facet_counters
+        if (pend_hot >= 0) {
+            double* h = hot + 8 * pend_hot;   // same field order as mfg_facet_counters
             if (pend_hits) {
                 atomicAdd(reinterpret_cast<unsigned long long*>(h), (unsigned long long)pend_hits);
                 if (w) atomic_addd(h + 1, pend_he);
@@ -942,7 +995,7 @@ struct Tracer {
             clear_pending();
             return;
         }
-        mfg_facet_counters* cc = P.fc + var->fc_base + (uint32_t)ph.local_id;
+        mfg_facet_counters* cc = P.fc + vc().fc_base + (uint32_t)local(pend_f);
         if (pend_hits) {
             atomic_addu(&cc->nb_mc_hit, pend_hits);
             if (w) atomic_addd(&cc->nb_hit_equiv, pend_he);
@@ -953,28 +1006,27 @@ struct Tracer {
         if (pend_s1pv != 0.0) atomic_addd(&cc->sum_1_per_velocity, pend_s1pv);
         clear_pending();
     }
-    __device__ void clear_pending() {
-        pend_f = -1; pend_hits = 0;
+    MFG_IN void clear_pending() {
+        pend_f = pend_hot = -1; pend_hits = 0;
         pend_he = pend_abs = pend_s1v = pend_svo = pend_s1pv = 0.0;
     }
     // Path score of a hit-equivalent x on a target:
     // d x / d s_g = x * (-n_g / (1 - s_g)) (+ x / s_t for the absorbed part).
-    __device__ void adjoint_score(const DPhys& ph, double x, bool absorbed_part) {
+    MFG_IN void adjoint_score(int t, int group, double x, bool absorbed_part) {
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
-            int t = ph.adj_target;
             atomic_addd(P.adj_j0 + t, x);
             uint32_t G = P.adj_groups;
             for (uint32_t g = 0; g < G; ++g) {
                 double s = P.adj_sticking[g];
                 double d = -x * (double)adj_cnt[g] / (1.0 - s);
-                if (absorbed_part && ph.adj_group == (int)g) d += x / s;
+                if (absorbed_part && group == (int)g) d += x / s;
                 if (d != 0.0) atomic_addd(P.adj_jac + (size_t)t * G + g, d);
             }
             // kept for the cutoff term until the particle survives a sticky collision
             if (seg_n < MFG_ADJ_SEG) { seg_t[seg_n] = t; seg_x[seg_n] = x; }
             ++seg_n;
         }
-        (void)ph; (void)x; (void)absorbed_part;
+        (void)t; (void)group; (void)x; (void)absorbed_part;
     }
     // The low-flux cutoff's term of dE[J]/ds_g (not a derivative of any
     // single path): the particle ends at collision K, W_{K-1} (1 - s_K) <=
@@ -984,7 +1036,7 @@ struct Tracer {
     // it survived K-1. In the renewal limit ln(W_{K-1}/c) is uniform on
     // (0, -ln(1 - s_K)] given K, so the term is
     //   dJ_t/ds_g += -sum x_t n_g / ((1 - s_g)(-ln(1 - s_K))).
-    __device__ void cutoff_boundary(const DPhys& ph, double sK) {
+    MFG_IN void cutoff_boundary(int group, double sK) {
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
             if (seg_n > MFG_ADJ_SEG) atomicOr(P.adj_seg_overflow, 1ull);
             const double dK = -log1p(-sK);
@@ -995,27 +1047,27 @@ struct Tracer {
                 const int t = seg_t[i];
                 const double x = seg_x[i];
                 for (uint32_t g = 0; g < G; ++g) {
-                    const double n = (double)adj_cnt[g] - (ph.adj_group == (int)g ? 1.0 : 0.0);
+                    const double n = (double)adj_cnt[g] - (group == (int)g ? 1.0 : 0.0);
                     if (n > 0.0) atomic_addd(P.adj_jac + (size_t)t * G + g, -x * n / ((1.0 - P.adj_sticking[g]) * dK));
                 }
             }
         }
-        (void)ph; (void)sK;
+        (void)group; (void)sK;
     }
-    __device__ void counter_force(const DPhys& ph, int m, uint32_t hit, uint32_t des, uint32_t abs_, double s1v,
+    MFG_IN void counter_force(const HitRegs& H, int32_t f, int m, uint32_t hit, uint32_t des, uint32_t abs_, double s1v,
                                   double svo, double sign) {
         d3 z = mk(0, 0, 0), v2 = z, mom = z, vv = z;
         if constexpr ((FEAT & FEAT_FORCE) != 0) {
-            if (var->enable_force) {
+            if (vc().enable_force) {
                 vv = scl(sign * vel, dir);
                 v2 = mk(vv.x * vv.x, vv.y * vv.y, vv.z * vv.z);
-                mom = cross(sub(pos, ld3(var->torque)), vv);
+                mom = cross(sub(pos, ld3(vc().torque)), vv);
             }
         }
         (void)sign;
-        counter(ph, m, hit, des, abs_, s1v, svo, vv, v2, mom);
+        counter(H, f, m, hit, des, abs_, s1v, svo, vv, v2, mom);
     }
-    __device__ bool cell(const DPhys& ph, uint32_t& add) const {
+    MFG_IN bool cell(const DPhys& ph, uint32_t& add) const {
         int tu = (int)(hu * ph.tex_wp), tv = (int)(hv * ph.tex_hp);
         tu = tu > ph.tex_w - 1 ? ph.tex_w - 1 : tu;
         tv = tv > ph.tex_h - 1 ? ph.tex_h - 1 : tv;
@@ -1023,25 +1075,27 @@ struct Tracer {
         add = (uint32_t)tu + (uint32_t)tv * (uint32_t)ph.tex_w;
         return true;
     }
-    __device__ double ort(const DFacet* F) const { return fabs(dot(dir, ld3(F->N))); }
+    MFG_IN double ort(const HitRegs& H) const { return fabs(dot(dir, H.N)); }
     // RecordHitOnTexture (Particle.cpp:977-1004)
-    __device__ void texture(const DFacet* F, const DPhys& ph, int m, bool count, double vf, double of) {
+    MFG_IN void texture(const HitRegs& H, int32_t f, int m, bool count, double vf, double of) {
+        const DPhys& ph = P.phys[f];
         uint32_t add;
         if (!cell(ph, add)) return;
-        double ov = var->c_factor * vel * ort(F);
-        double inc = P.tex_inc[var->tex_base + (size_t)ph.tex_off + add];
+        double ov = vc().c_factor * vel * ort(H);
+        double inc = P.tex_inc[vc().tex_base + (size_t)ph.tex_off + add];
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             int slot = k == 0 ? 0 : m;
             if (k == 1 && m <= 0) break;
-            mfg_texture_cell* c = P.tex + var->tex_base + (size_t)slot * var->n_tex + (size_t)ph.tex_off + add;
+            mfg_texture_cell* c = P.tex + vc().tex_base + (size_t)slot * vc().n_tex + (size_t)ph.tex_off + add;
             if (count) atomic_addd(&c->count_equiv, ori);
             atomic_addd(&c->sum_1_per_ort_velocity, ori * vf / ov);
             atomic_addd(&c->sum_v_ort_per_area, ori * of * ov * inc);
         }
     }
     // RecordDirectionVector (Particle.cpp:1006-1023)
-    __device__ void direction(const DPhys& ph, int m) {
+    MFG_IN void direction(int32_t f, int m) {
+        const DPhys& ph = P.phys[f];
         if (ph.dir_off < 0) return;
         uint32_t add;
         if (!cell(ph, add)) return;
@@ -1049,7 +1103,7 @@ struct Tracer {
         for (int k = 0; k < 2; ++k) {
             int slot = k == 0 ? 0 : m;
             if (k == 1 && m <= 0) break;
-            mfg_direction_cell* c = P.dir + var->dir_base + (size_t)slot * var->n_dir + (size_t)ph.dir_off + add;
+            mfg_direction_cell* c = P.dir + vc().dir_base + (size_t)slot * vc().n_dir + (size_t)ph.dir_off + add;
             atomic_addd(&c->dir[0], ori * dir.x * vel);
             atomic_addd(&c->dir[1], ori * dir.y * vel);
             atomic_addd(&c->dir[2], ori * dir.z * vel);
@@ -1057,11 +1111,12 @@ struct Tracer {
         }
     }
     // ProfileFacet (Particle.cpp:1025-1085)
-    __device__ void profile(const DFacet* F, const DPhys& ph, int m, bool count, double vf, double of) {
-        if (ph.prof_off < 0) return;
+    MFG_IN void profile(const HitRegs& H, int32_t f, int m, bool count, double vf, double of) {
+        if (!(H.flags & FF_PROFILE)) return;
+        const DPhys& ph = P.phys[f];
         int pt = ph.profile_type;
-        double a = ort(F);
-        mfg_profile_slice* base = P.prof + var->prof_base + (size_t)ph.prof_off;
+        double a = ort(H);
+        mfg_profile_slice* base = P.prof + vc().prof_base + (size_t)ph.prof_off;
         if (count && pt == MFG_PROFILE_ANGULAR) {
             double th = acos(fmin(1.0, a));
             long p = (long)(th / (kPi / 2) * (double)MFG_PROFILE_SIZE);
@@ -1069,7 +1124,7 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                atomic_addd(&base[(size_t)slot * var->n_prof + p].count_equiv, ori);
+                atomic_addd(&base[(size_t)slot * vc().n_prof + p].count_equiv, ori);
             }
         } else if (pt == MFG_PROFILE_U || pt == MFG_PROFILE_V) {
             double c = pt == MFG_PROFILE_U ? hu : hv;
@@ -1081,10 +1136,10 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                mfg_profile_slice* s = &base[(size_t)slot * var->n_prof + p];
+                mfg_profile_slice* s = &base[(size_t)slot * vc().n_prof + p];
                 if (count) atomic_addd(&s->count_equiv, ori);
                 atomic_addd(&s->sum_1_per_ort_velocity, ori * vf / ov);
-                atomic_addd(&s->sum_v_ort, ori * of * var->c_factor * ov);
+                atomic_addd(&s->sum_v_ort, ori * of * vc().c_factor * ov);
             }
         } else if (count && (pt == MFG_PROFILE_VELOCITY || pt == MFG_PROFILE_ORT_VELOCITY || pt == MFG_PROFILE_TAN_VELOCITY)) {
             double d = pt == MFG_PROFILE_VELOCITY ? 1.0 : (pt == MFG_PROFILE_ORT_VELOCITY ? a : sqrt(fmax(0.0, 1 - a * a)));
@@ -1094,20 +1149,22 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                atomic_addd(&base[(size_t)slot * var->n_prof + p].count_equiv, ori);
+                atomic_addd(&base[(size_t)slot * vc().n_prof + p].count_equiv, ori);
             }
         }
     }
-    __device__ void polar(const DFacet* F, const DPhys& ph, double& th, double& phv) const {
-        double lu = dot(dir, ld3(ph.nU)), lv = dot(dir, ld3(ph.nV)), ln = dot(dir, ld3(F->N));
+    MFG_IN void polar(const HitRegs& H, double& th, double& phv) const {
+        double lu = dot(dir, H.nU), lv = dot(dir, H.nV), ln = dot(dir, H.N);
         th = acos(fmax(-1.0, fmin(1.0, ln)));
         phv = atan2(lv, lu);
     }
     // RecordAngleMap (Particle.cpp:1104-1136). The angles only select a bin,
     // so they are evaluated in FP32.
-    __device__ void angle_map(const DFacet* F, const DPhys& ph) {
-        if (!(ph.flags & FF_ANGLEMAP) || ph.am_off < 0) return;
-        double lu = dot(dir, ld3(ph.nU)), lv = dot(dir, ld3(ph.nV)), ln = dot(dir, ld3(F->N));
+    MFG_IN void angle_map(const HitRegs& H, int32_t f) {
+        if (!(H.flags & FF_ANGLEMAP)) return;
+        const DPhys& ph = P.phys[f];
+        if (ph.am_off < 0) return;
+        double lu = dot(dir, H.nU), lv = dot(dir, H.nV), ln = dot(dir, H.N);
         double th = (double)acosf((float)fmax(-1.0, fmin(1.0, ln)));
         double phv = (double)atan2f((float)lv, (float)lu);
         if (th > kPi / 2.0) th = fabs(kPi - th);
@@ -1123,25 +1180,25 @@ struct Tracer {
         ti = ti < 0 ? 0 : (ti > nt - 1 ? nt - 1 : ti);
         long pi_ = (long)((phv + 3.1415926) / (2.0 * kPi) * (double)ph.am_phi);
         pi_ = pi_ < 0 ? 0 : (pi_ > (long)ph.am_phi - 1 ? (long)ph.am_phi - 1 : pi_);
-        atomic_addu(P.am + var->am_base + (size_t)ph.am_off + (size_t)ti * ph.am_phi + pi_, 1ull);
+        atomic_addu(P.am + vc().am_base + (size_t)ph.am_off + (size_t)ti * ph.am_phi + pi_, 1ull);
     }
     // LogHit (Particle.cpp:1087-1102)
-    __device__ void log_hit(const DFacet* F, const DPhys& ph, int32_t f) {
+    MFG_IN void log_hit(const HitRegs& H, int32_t f) {
         if constexpr ((FEAT & FEAT_LOG) != 0) {
-            if (var->log_facet == f) {
+            if (vc().log_facet == f) {
                 unsigned long long at = atomicAdd(P.log_count, 1ull);
-                if (at < var->log_limit) {
+                if (at < vc().log_limit) {
                     mfg_log_entry e;
                     e.u = hu; e.v = hv;
-                    polar(F, ph, e.hit_theta, e.hit_phi);
+                    polar(H, e.hit_theta, e.hit_phi);
                     e.ori_ratio = ori; e.particle_decay_moment = decay_t; e.time = time; e.velocity = vel;
                     P.log[at] = e;
                 }
             }
         }
-        (void)F; (void)ph; (void)f;
+        (void)H; (void)f;
     }
-    __device__ void hist_add(double* g, uint32_t nb, uint32_t nd, uint32_t nt, uint32_t bbin, double dbin, double tbin) {
+    MFG_IN void hist_add(double* g, uint32_t nb, uint32_t nd, uint32_t nt, uint32_t bbin, double dbin, double tbin) {
         uint32_t off = 0;
         if (nb) { uint32_t b = nb_bounces / bbin; atomic_addd(g + off + (b < nb - 1 ? b : nb - 1), ori); off += nb; }
         if (nd) {
@@ -1156,51 +1213,52 @@ struct Tracer {
         }
     }
     // RecordHistograms (Particle.cpp:926-975), called on absorption
-    __device__ void histograms(const DPhys& ph, int m) {
+    MFG_IN void histograms(int32_t f, int m) {
         if constexpr ((FEAT & FEAT_HIST) != 0) {
+            const DPhys& ph = P.phys[f];
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                if (var->n_gh)
-                    hist_add(P.gh + var->gh_base + (size_t)slot * var->n_gh, var->gh_nb_bounce, var->gh_nb_dist,
-                             var->gh_nb_time, var->gh_bounce_bin, var->gh_dist_bin, var->gh_time_bin);
+                if (vc().n_gh)
+                    hist_add(P.gh + vc().gh_base + (size_t)slot * vc().n_gh, vc().gh_nb_bounce, vc().gh_nb_dist,
+                             vc().gh_nb_time, vc().gh_bounce_bin, vc().gh_dist_bin, vc().gh_time_bin);
                 if (ph.fh_off >= 0)
-                    hist_add(P.fh + var->fh_base + (size_t)slot * var->n_fh + ph.fh_off, ph.fh_nb_bounce, ph.fh_nb_dist,
+                    hist_add(P.fh + vc().fh_base + (size_t)slot * vc().n_fh + ph.fh_off, ph.fh_nb_bounce, ph.fh_nb_dist,
                              ph.fh_nb_time, ph.fh_bounce_bin, ph.fh_dist_bin, ph.fh_time_bin);
             }
         }
-        (void)ph; (void)m;
+        (void)f; (void)m;
     }
-    __device__ d3 polar_to_cart(const DFacet* F, const DPhys& ph, double cos_t, double sin_t, double phv, bool reverse) const {
+    MFG_IN d3 polar_to_cart(const HitRegs& H, double cos_t, double sin_t, double phv, bool reverse) const {
         double s, c;
         sincos(phv, &s, &c);
         double n = reverse ? -cos_t : cos_t;
-        return add(add(scl(sin_t * c, ld3(ph.nU)), scl(sin_t * s, ld3(ph.nV))), scl(n, ld3(F->N)));
+        return add(add(scl(sin_t * c, H.nU), scl(sin_t * s, H.nV)), scl(n, H.N));
     }
     // TreatMovingFacet (Physics.cpp:22-39)
-    __device__ void moving(d3& d, double& v) const {
+    MFG_IN void moving(d3& d, double& v) const {
         if constexpr ((FEAT & FEAT_MOVING) != 0) {
             d3 a = mk(0, 0, 0);
-            if (var->motion_type == 1) a = ld3(var->motion2);
-            else if (var->motion_type == 2) a = cross(ld3(var->motion2), scl(0.01, sub(pos, ld3(var->motion1))));
+            if (vc().motion_type == 1) a = ld3(vc().motion2);
+            else if (vc().motion_type == 2) a = cross(ld3(vc().motion2), scl(0.01, sub(pos, ld3(vc().motion1))));
             d3 nv = add(scl(v, d), a);
             v = nrm(nv);
             d = unitv(nv);
         }
         (void)d; (void)v;
     }
-    __device__ double maxwell_speed(double sq) {
-        XYRef t{P.tab_x + var->maxwell_base, P.tab_y + var->maxwell_base, 100};
-        return interp_x_guided(rng.rnd(), t, P.guides + var->maxwell_guide, MFG_MAXWELL_GUIDE) * sq;
+    MFG_IN double maxwell_speed(double sq) {
+        XYRef t{P.tab_x + vc().maxwell_base, P.tab_y + vc().maxwell_base, 100};
+        return interp_x_guided(rng.rnd(), t, P.guides + vc().maxwell_guide, MFG_MAXWELL_GUIDE) * sq;
     }
-    __device__ d3 emit(const DFacet* F, const DPhys& ph, int type, double n_exp, bool reverse) {
+    MFG_IN d3 emit(const HitRegs& H, const DPhys& ph, int type, double n_exp, bool reverse) {
         if (type == MFG_DES_UNIFORM) {
             double c = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
-            return polar_to_cart(F, ph, c, sqrt(1 - c * c), phv, reverse);
+            return polar_to_cart(H, c, sqrt(1 - c * c), phv, reverse);
         }
         if (type == MFG_DES_COSINE_N) {
             double c = pow(rng.rnd(), 1.0 / (n_exp + 1.0)); double phv = rng.rnd() * 2.0 * kPi;
-            return polar_to_cart(F, ph, c, sqrt(1 - c * c), phv, reverse);
+            return polar_to_cart(H, c, sqrt(1 - c * c), phv, reverse);
         }
         if constexpr ((FEAT & FEAT_AMSRC) != 0) {
             if (type == MFG_DES_ANGLEMAP) {   // Particle.cpp:599-621: the map holds incident angles
@@ -1210,40 +1268,40 @@ struct Tracer {
                 am_generate_theta(A, rng.rnd(), th, tlo, ov);
                 double phv = am_generate_phi(A, tlo, ov, rng.rnd());
                 double t2 = kPi - th;
-                return polar_to_cart(F, ph, cos(t2), sin(t2), phv, false);
+                return polar_to_cart(H, cos(t2), sin(t2), phv, false);
             }
         }
         double a = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
-        return polar_to_cart(F, ph, sqrt(a), sqrt(1 - a), phv, reverse);
+        return polar_to_cart(H, sqrt(a), sqrt(1 - a), phv, reverse);
     }
 
     // StartFromSource (Particle.cpp:407-685) without the source-facet
     // counter, which the caller adds (summed across the wave).
-    __device__ int32_t start(uint64_t local_pid) {
-        pid = local_pid;
-        rng.init(var->seed, pid);
+    MFG_IN int32_t start(uint64_t local_pid) {
+        rng.init(var->seed, local_pid);
         nb_events = 0;
         tr_n = 0;
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
             for (uint32_t g = 0; g < P.adj_groups; ++g) adj_cnt[g] = 0;
             seg_n = 0;
         }
-        double r = rng.rnd() * var->total_des;
-        const double* cum = P.src_cum + var->src_base;
-        uint32_t n = var->src_n;
+        double r = rng.rnd() * vc().total_des;
+        const double* cum = P.src_cum + vc().src_base;
+        uint32_t n = vc().src_n;
         uint32_t lo = 0, hi = n;  // first cum > r
         while (lo < hi) { uint32_t mid = (lo + hi) / 2; if (cum[mid] <= r) lo = mid + 1; else hi = mid; }
         uint32_t k = lo < n ? lo : n - 1;
-        int32_t src = P.src_facet[var->src_base + k];
+        int32_t src = P.src_facet[vc().src_base + k];
         const DFacet* F = P.facets + src;
         const DPhys& ph = P.phys[src];
+        const HitRegs H = load_hit(P.hits + src);
         bool reverse = false;
-        if (F->flags & FF_2SIDED) reverse = rng.rnd() > 0.5;
+        if (H.flags & FF_2SIDED) reverse = rng.rnd() > 0.5;
         long map_w = -1, map_h = -1;
         if constexpr ((FEAT & FEAT_OGMAP) != 0) {
             if (ph.flags & FF_OGMAP) {
                 double base = k ? cum[k - 1] : 0.0;
-                double rem = (r - base) / var->latest * (1.38E-23 * ph.temperature);
+                double rem = (r - base) / vc().latest * (1.38E-23 * ph.temperature);
                 const double* oc = P.og_cdf + ph.og_off;
                 uint32_t nc = ph.og_w * ph.og_h, a = 0, b = nc;
                 while (a < b) { uint32_t mid = (a + b) / 2; if (oc[mid] <= rem) a = mid + 1; else b = mid; }
@@ -1254,23 +1312,23 @@ struct Tracer {
         }
         last_hit = src;
         double rt = rng.rnd();
-        time = rt * var->latest;
+        if constexpr (CLOCKED) time = rt * vc().latest;
         if constexpr ((FEAT & FEAT_TDPARAM) != 0) {
             if (ph.id_index >= 0) {
-                const DTable tb = P.ids[var->id_base + ph.id_index];
+                const DTable tb = P.ids[vc().id_base + ph.id_index];
                 XYRef t{P.tab_x + tb.off, P.tab_y + tb.off, tb.n};
                 time = interp_x(rt * t.y[t.n - 1], t);
             }
         }
         gen_time = time;
-        if (var->use_maxwell) vel = maxwell_speed(ph.sqrt_temp);
-        else vel = 145.469 * sqrt(ph.temperature / var->gas_mass);
+        if (vc().use_maxwell) vel = maxwell_speed(H.sqrt_temp);
+        else vel = 145.469 * sqrt(ph.temperature / vc().gas_mass);
         ori = 1.0;
         decay_t = 1e100;
         scatter_path = 1e100;
         if constexpr ((FEAT & FEAT_VOLUME) != 0) {
-            if (var->enable_decay) decay_t = time + (1.44269 * var->half_life) * -log(rng.rnd());
-            if (var->scatter_enabled) scatter_path = var->scatter_mfp * -log(rng.rnd());
+            if (vc().enable_decay) decay_t = time + (1.44269 * vc().half_life) * -log(rng.rnd());
+            if (vc().scatter_enabled) scatter_path = vc().scatter_mfp * -log(rng.rnd());
         }
         nb_bounces = 0;
         dist = 0.0;
@@ -1305,42 +1363,41 @@ struct Tracer {
                 pos = ld3(ph.centre);
             }
         }
-        dir = emit(F, ph, ph.desorb_type, ph.des_exp, reverse);
+        dir = emit(H, ph, ph.desorb_type, ph.des_exp, reverse);
         structure = ph.super_idx;
         tele_from = -1;
         if constexpr ((FEAT & FEAT_MOVING) != 0) {
-            if ((ph.flags & FF_MOVING) && var->motion_type) moving(dir, vel);
+            if ((ph.flags & FF_MOVING) && vc().motion_type) moving(dir, vel);
         }
         return src;
     }
 
     // Records of a desorption other than the facet counter of slot 0.
-    __device__ void desorption_records(int32_t src, int m, double ov) {
-        const DFacet* F = P.facets + src;
-        const DPhys& ph = P.phys[src];
-        if (m > 0 || ((FEAT & FEAT_FORCE) != 0 && var->enable_force)) {
+    MFG_IN void desorption_records(int32_t src, int m, double ov) {
+        const HitRegs H = load_hit(P.hits + src);
+        if (m > 0 || ((FEAT & FEAT_FORCE) != 0 && vc().enable_force)) {
             // moment slot (and force terms) per lane
             d3 z = mk(0, 0, 0), v2 = z, mom = z, vv = z;
             if constexpr ((FEAT & FEAT_FORCE) != 0) {
-                if (var->enable_force) {
+                if (vc().enable_force) {
                     vv = scl(vel, dir);
                     v2 = mk(vv.x * vv.x, vv.y * vv.y, vv.z * vv.z);
-                    mom = cross(sub(pos, ld3(var->torque)), vv);
-                    double* fo = P.force + var->force_base + (size_t)(uint32_t)ph.local_id * 9;
+                    mom = cross(sub(pos, ld3(vc().torque)), vv);
+                    double* fo = P.force + vc().force_base + (size_t)(uint32_t)local(src) * 9;
                     atomic_addd(fo + 0, vv.x); atomic_addd(fo + 1, vv.y); atomic_addd(fo + 2, vv.z);
                     atomic_addd(fo + 3, v2.x); atomic_addd(fo + 4, v2.y); atomic_addd(fo + 5, v2.z);
                     atomic_addd(fo + 6, mom.x); atomic_addd(fo + 7, mom.y); atomic_addd(fo + 8, mom.z);
                 }
             }
             if (m > 0) {
-                mfg_facet_counters* c = fc(ph, m);
+                mfg_facet_counters* c = fc(src, m);
                 atomic_addu(&c->nb_desorbed, 1ull);
                 atomic_addd(&c->sum_1_per_ort_velocity, 2.0 / ov);
-                atomic_addd(&c->sum_v_ort, var->c_factor * ov);
+                atomic_addd(&c->sum_v_ort, vc().c_factor * ov);
                 atomic_addd(&c->sum_1_per_velocity, 1.0 / vel);
                 if constexpr ((FEAT & FEAT_FORCE) != 0) {
-                    if (var->enable_force) {
-                        double* fo = P.force + var->force_base + ((size_t)m * var->n_facets + (uint32_t)ph.local_id) * 9;
+                    if (vc().enable_force) {
+                        double* fo = P.force + vc().force_base + ((size_t)m * vc().n_facets + (uint32_t)local(src)) * 9;
                         atomic_addd(fo + 0, vv.x); atomic_addd(fo + 1, vv.y); atomic_addd(fo + 2, vv.z);
                         atomic_addd(fo + 3, v2.x); atomic_addd(fo + 4, v2.y); atomic_addd(fo + 5, v2.z);
                         atomic_addd(fo + 6, mom.x); atomic_addd(fo + 7, mom.y); atomic_addd(fo + 8, mom.z);
@@ -1348,138 +1405,137 @@ struct Tracer {
                 }
             }
         }
-        profile(F, ph, m, false, 2.0, 1.0);
-        log_hit(F, ph, src);
-        if ((ph.flags & FF_COUNT_DES) && ph.tex_off >= 0) texture(F, ph, m, true, 2.0, 1.0);
+        profile(H, src, m, false, 2.0, 1.0);
+        log_hit(H, src);
+        if ((H.flags & FF_COUNT_DES) && (H.flags & FF_TEXTURE)) texture(H, src, m, true, 2.0, 1.0);
         trace(src, 0);
     }
 
     // RegisterTransparentPass (Particle.cpp:1232-1257)
-    __device__ void transparent_pass(int32_t f, double tp) {
-        const DFacet* F = P.facets + f;
-        const DPhys& ph = P.phys[f];
-        double df = ort(F);
+    MFG_IN void transparent_pass(int32_t f, double tp) {
+        const HitRegs H = load_hit(P.hits + f);
+        double df = ort(H);
         int m = moment(time + tp / 100.0 / vel);
         d3 z = mk(0, 0, 0);
-        counter(ph, m, 1, 0, 0, 2.0 / (vel * df), 2.0 * var->c_factor * vel * df, z, z, z);
-        if ((ph.flags & FF_COUNT_TRANS) && ph.tex_off >= 0) texture(F, ph, m, true, 2.0, 2.0);
-        if (ph.flags & FF_COUNT_DIR) direction(ph, m);
-        log_hit(F, ph, f);
-        profile(F, ph, m, true, 2.0, 2.0);
-        angle_map(F, ph);
+        counter(H, f, m, 1, 0, 0, 2.0 / (vel * df), 2.0 * vc().c_factor * vel * df, z, z, z);
+        if ((H.flags & FF_COUNT_TRANS) && (H.flags & FF_TEXTURE)) texture(H, f, m, true, 2.0, 2.0);
+        if (H.flags & FF_COUNT_DIR) direction(f, m);
+        log_hit(H, f);
+        profile(H, f, m, true, 2.0, 2.0);
+        angle_map(H, f);
         trace(f, 3);
     }
     // RecordAbsorb (Particle.cpp:888-924)
-    __device__ void record_absorb(int32_t f) {
-        const DFacet* F = P.facets + f;
-        const DPhys& ph = P.phys[f];
-        ++acc_hits; acc_hit_equiv += ori; acc_abs_equiv += ori;
+    MFG_IN void record_absorb(const HitRegs& H, int32_t f) {
+        add_hit();
+        if constexpr (WEIGHTED) acc_abs_equiv += ori;
+        else ++acc_absorbed;
         int m = moment(time);
-        histograms(ph, m);
-        double ov = vel * ort(F);
+        histograms(f, m);
+        double ov = vel * ort(H);
         bool scored = false;
         if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
-            if (ph.adj_target >= 0) {
+            const int32_t at = P.hits[f].adj_target;
+            if (at >= 0) {
                 // the absorbed part carries its own d/ds_t term
                 for (int k = 0; k < 2; ++k) {
                     int slot = k == 0 ? 0 : m;
                     if (k == 1 && m <= 0) break;
-                    mfg_facet_counters* c = fc(ph, slot);
+                    mfg_facet_counters* c = fc(f, slot);
                     atomic_addu(&c->nb_mc_hit, 1ull);
                     atomic_addd(&c->nb_hit_equiv, ori);
                     atomic_addd(&c->nb_abs_equiv, ori);
                     atomic_addd(&c->sum_1_per_ort_velocity, ori * 2.0 / ov);
-                    atomic_addd(&c->sum_v_ort, ori * var->c_factor * ov);
+                    atomic_addd(&c->sum_v_ort, ori * vc().c_factor * ov);
                     atomic_addd(&c->sum_1_per_velocity, ori / vel);
                 }
-                adjoint_score(ph, ori, true);
+                adjoint_score(at, P.hits[f].adj_group, ori, true);
                 scored = true;
             }
         }
-        if (!scored) counter_force(ph, m, 1, 0, 1, 2.0 / ov, var->c_factor * ov, 1.0);
-        log_hit(F, ph, f);
-        profile(F, ph, m, true, 2.0, 1.0);
-        angle_map(F, ph);
-        if ((ph.flags & FF_COUNT_ABS) && ph.tex_off >= 0) texture(F, ph, m, true, 2.0, 1.0);
-        if (ph.flags & FF_COUNT_DIR) direction(ph, m);
+        if (!scored) counter_force(H, f, m, 1, 0, 1, 2.0 / ov, vc().c_factor * ov, 1.0);
+        log_hit(H, f);
+        profile(H, f, m, true, 2.0, 1.0);
+        angle_map(H, f);
+        if ((H.flags & FF_COUNT_ABS) && (H.flags & FF_TEXTURE)) texture(H, f, m, true, 2.0, 1.0);
+        if (H.flags & FF_COUNT_DIR) direction(f, m);
     }
     // UpdateVelocity (Particle.cpp:1138-1163)
-    __device__ void update_velocity(const DPhys& ph) {
-        double T = temperature(ph);
-        double sq = ph.temperature_param == -1 ? ph.sqrt_temp : sqrt(T);
-        if (ph.flags & FF_FULL_ACC) {
-            vel = var->use_maxwell ? maxwell_speed(sq) : 145.469 * sq / var->gas_mass;
+    MFG_IN void update_velocity(const HitRegs& H, int32_t f) {
+        double sq = H.sqrt_temp;
+        if constexpr ((FEAT & FEAT_TDPARAM) != 0) { if (H.flags & FF_TD_TEMP) sq = sqrt(temperature(P.phys[f])); }
+        if (H.flags & FF_FULL_ACC) {
+            vel = vc().use_maxwell ? maxwell_speed(sq) : 145.469 * sq / vc().gas_mass;
         } else {
             double o2 = vel * vel, n2;
-            if (var->use_maxwell) { double vv = maxwell_speed(sq); n2 = vv * vv; }
-            else n2 = 29369.939 * (T / var->gas_mass);
-            vel = sqrt(o2 + (n2 - o2) * ph.accomodation);
+            if (vc().use_maxwell) { double vv = maxwell_speed(sq); n2 = vv * vv; }
+            else n2 = 29369.939 * (temperature(P.phys[f]) / vc().gas_mass);
+            vel = sqrt(o2 + (n2 - o2) * P.hits[f].accomodation);
         }
     }
     // PerformBounce (Particle.cpp:691-838)
-    __device__ void bounce(int32_t f) {
-        const DFacet* F = P.facets + f;
-        const DPhys& ph = P.phys[f];
-        ++acc_hits; acc_hit_equiv += ori;
+    MFG_IN void bounce(const HitRegs& H, int32_t f) {
+        add_hit();
         if constexpr ((FEAT & FEAT_TELEPORT) != 0) {
-            if (ph.super_dest) {
+            if (H.flags & FF_LINK) {
                 int m = moment(time);
                 d3 z = mk(0, 0, 0);
-                counter(ph, m, 1, 0, 0, 0.0, 0.0, z, z, z);
-                structure = ph.super_dest - 1;
-                if constexpr ((FEAT & FEAT_MOVING) != 0) { if (ph.flags & FF_MOVING) moving(dir, vel); }
-                log_hit(F, ph, f);
-                profile(F, ph, m, true, 2.0, 2.0);
-                angle_map(F, ph);
-                if ((ph.flags & FF_COUNT_TRANS) && ph.tex_off >= 0) texture(F, ph, m, true, 2.0, 2.0);
-                if (ph.flags & FF_COUNT_DIR) direction(ph, m);
+                counter(H, f, m, 1, 0, 0, 0.0, 0.0, z, z, z);
+                structure = P.phys[f].super_dest - 1;
+                if constexpr ((FEAT & FEAT_MOVING) != 0) { if (H.flags & FF_MOVING) moving(dir, vel); }
+                log_hit(H, f);
+                profile(H, f, m, true, 2.0, 2.0);
+                angle_map(H, f);
+                if ((H.flags & FF_COUNT_TRANS) && (H.flags & FF_TEXTURE)) texture(H, f, m, true, 2.0, 2.0);
+                if (H.flags & FF_COUNT_DIR) direction(f, m);
                 trace(f, 5);
                 return;
             }
         }
-        d3 N = ld3(F->N);
-        double dn = dot(dir, N);
-        bool revert = (F->flags & FF_2SIDED) && dn > 0.0;
+        double dn = dot(dir, H.N);
+        bool revert = (H.flags & FF_2SIDED) && dn > 0.0;
         double ov_in = vel * fabs(dn);
         int m = moment(time);
-        counter_force(ph, m, 1, 0, 0, 1.0 / ov_in, var->c_factor * ov_in, 1.0);
-        ++nb_bounces;
-        if ((ph.flags & FF_COUNT_REFL) && ph.tex_off >= 0) texture(F, ph, m, true, 1.0, 1.0);
-        if (ph.flags & FF_COUNT_DIR) direction(ph, m);
-        log_hit(F, ph, f);
-        profile(F, ph, m, true, 1.0, 1.0);
-        angle_map(F, ph);
-        update_velocity(ph);
+        counter_force(H, f, m, 1, 0, 0, 1.0 / ov_in, vc().c_factor * ov_in, 1.0);
+        if constexpr (CLOCKED) ++nb_bounces;
+        if ((H.flags & FF_COUNT_REFL) && (H.flags & FF_TEXTURE)) texture(H, f, m, true, 1.0, 1.0);
+        if (H.flags & FF_COUNT_DIR) direction(f, m);
+        log_hit(H, f);
+        profile(H, f, m, true, 1.0, 1.0);
+        angle_map(H, f);
+        update_velocity(H, f);
         int m_out = m;
         if constexpr ((FEAT & FEAT_SOJOURN) != 0) {
-            if (ph.flags & FF_SOJOURN) {
+            if (H.flags & FF_SOJOURN) {
+                const DPhys& ph = P.phys[f];
                 double A = exp(-ph.sojourn_e / (8.31 * temperature(ph)));
                 time += -log(rng.rnd()) / (A * ph.sojourn_freq);
                 m_out = moment(time);
             }
         }
-        if (ph.flags & FF_DIFFUSE) {
+        if (H.flags & FF_DIFFUSE) {
             double a = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
-            dir = polar_to_cart(F, ph, sqrt(a), sqrt(1 - a), phv, revert);
+            dir = polar_to_cart(H, sqrt(a), sqrt(1 - a), phv, revert);
         } else {
+            const DHit& C = P.hits[f];
             double rt = rng.rnd();
-            if (rt < ph.diffuse) {
+            if (rt < C.diffuse) {
                 double a = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
-                dir = polar_to_cart(F, ph, sqrt(a), sqrt(1 - a), phv, revert);
-            } else if (rt < ph.diffuse + ph.specular) {
-                dir = sub(dir, scl(2.0 * dot(dir, N), N));
+                dir = polar_to_cart(H, sqrt(a), sqrt(1 - a), phv, revert);
+            } else if (rt < C.diffuse + C.specular) {
+                dir = sub(dir, scl(2.0 * dot(dir, H.N), H.N));
             } else {
-                double c = pow(rng.rnd(), 1.0 / (ph.cos_exp + 1.0)); double phv = rng.rnd() * 2.0 * kPi;
-                dir = polar_to_cart(F, ph, c, sqrt(1 - c * c), phv, revert);
+                double c = pow(rng.rnd(), 1.0 / (P.phys[f].cos_exp + 1.0)); double phv = rng.rnd() * 2.0 * kPi;
+                dir = polar_to_cart(H, c, sqrt(1 - c * c), phv, revert);
             }
         }
         if constexpr ((FEAT & FEAT_MOVING) != 0) {
-            if ((ph.flags & FF_MOVING) && var->motion_type) moving(dir, vel);
+            if ((H.flags & FF_MOVING) && vc().motion_type) moving(dir, vel);
         }
-        double ov_out = vel * ort(F);
-        counter_force(ph, m_out, 0, 0, 0, 1.0 / ov_out, var->c_factor * ov_out, -1.0);
-        if ((ph.flags & FF_COUNT_REFL) && ph.tex_off >= 0) texture(F, ph, m_out, false, 1.0, 1.0);
-        profile(F, ph, m_out, false, 1.0, 1.0);
+        double ov_out = vel * ort(H);
+        counter_force(H, f, m_out, 0, 0, 0, 1.0 / ov_out, vc().c_factor * ov_out, -1.0);
+        if ((H.flags & FF_COUNT_REFL) && (H.flags & FF_TEXTURE)) texture(H, f, m_out, false, 1.0, 1.0);
+        profile(H, f, m_out, false, 1.0, 1.0);
         last_hit = f;
         trace(f, 1);
     }
@@ -1488,24 +1544,23 @@ struct Tracer {
     // the reference records teleportedFrom = destIndex (:122). A destination
     // in every structure (super_idx -1) keeps the particle's structure; the
     // reference would index its structure list with -1 there (:121, :245).
-    __device__ void teleport(int32_t f) {
-        const DFacet* F = P.facets + f;
+    MFG_IN void teleport(const HitRegs& H, int32_t f) {
         const DPhys& ph = P.phys[f];
         trace(f, 4);
         int32_t dest = ph.teleport_dest == -1 ? tele_from : ph.teleport_dest - 1;
-        if (dest < 0 || dest >= (int32_t)var->n_facets) { last_hit = f; return; }
-        int32_t dg = dest + (int32_t)var->facet_base;
+        if (dest < 0 || dest >= (int32_t)vc().n_facets) { last_hit = f; return; }
+        int32_t dg = dest + (int32_t)vc().facet_base;
         const DFacet* D = P.facets + dg;
         const DPhys& dph = P.phys[dg];
         if (dph.super_idx >= 0) structure = dph.super_idx;
         tele_from = dest;
         int m = moment(time);
-        if ((ph.flags & FF_COUNT_TRANS) && ph.tex_off >= 0) texture(F, ph, m, true, 2.0, 2.0);
-        if (ph.flags & FF_COUNT_DIR) direction(ph, m);
-        profile(F, ph, m, true, 2.0, 2.0);
-        log_hit(F, ph, f);
-        angle_map(F, ph);
-        double lu = dot(dir, ld3(ph.nU)), lv = dot(dir, ld3(ph.nV)), ln = dot(dir, ld3(F->N));
+        if ((H.flags & FF_COUNT_TRANS) && (H.flags & FF_TEXTURE)) texture(H, f, m, true, 2.0, 2.0);
+        if (H.flags & FF_COUNT_DIR) direction(f, m);
+        profile(H, f, m, true, 2.0, 2.0);
+        log_hit(H, f);
+        angle_map(H, f);
+        double lu = dot(dir, H.nU), lv = dot(dir, H.nV), ln = dot(dir, H.N);
         dir = add(add(scl(lu, ld3(dph.nU)), scl(lv, ld3(dph.nV))), scl(ln, ld3(D->N)));
         double u = hu, v = hv;
         d3 O = ld3(D->O), U = ld3(D->U), V = ld3(D->V);
@@ -1518,15 +1573,15 @@ struct Tracer {
             }
         }
         last_hit = dg;
-        double ov = vel * ort(F);
+        double ov = vel * ort(H);
         d3 z = mk(0, 0, 0);
-        counter(ph, m, 1, 0, 0, 2.0 / ov, 2.0 * var->c_factor * ov, z, z, z);
+        counter(H, f, m, 1, 0, 0, 2.0 / ov, 2.0 * vc().c_factor * ov, z, z, z);
     }
     // PerformScatter (Particle.cpp:840-886, Physics.cpp:41-63)
-    __device__ bool scatter() {
-        ++acc_hits; acc_hit_equiv += ori;
+    MFG_IN bool scatter() {
+        add_hit();
         ++nb_bounces;
-        double rho = var->scatter_rho, mr = var->scatter_mr;
+        double rho = vc().scatter_rho, mr = vc().scatter_mr;
         double b = rho * sqrt(rng.rnd());
         double a = sqrt(rho * rho - b * b);
         double ctg = 1.0 / (2.0 * a * b) * (rho * rho * mr + b * b - a * a);
@@ -1539,60 +1594,70 @@ struct Tracer {
         dir = add(add(scl(st * ca, un), scl(st * sa, vn)), scl(ct, dir));
         double q = mr * rho / b * st;
         vel = sqrt(vel * vel / (1.0 + q * q));
-        scatter_path = dist + var->scatter_mfp * -log(rng.rnd());
+        scatter_path = dist + vc().scatter_mfp * -log(rng.rnd());
         trace(-1, 8);
-        return !(var->scatter_cutoff && vel < var->scatter_cut);
+        return !(vc().scatter_cutoff && vel < vc().scatter_cut);
     }
 
     // Add this lane's global counters to its variant and clear them.
     // ---- particles kept between launches
-    __device__ void save(CarryRec& r, uint64_t events_left, uint32_t vi) const {
+    MFG_IN void save(CarryRec& r, uint64_t events_left, uint32_t vi) const {
         r.pos[0] = pos.x; r.pos[1] = pos.y; r.pos[2] = pos.z;
         r.dir[0] = dir.x; r.dir[1] = dir.y; r.dir[2] = dir.z;
-        r.time = time; r.vel = vel; r.ori = ori; r.gen_time = gen_time; r.dist = dist;
+        r.time = time; r.vel = vel; r.ori = w(); r.gen_time = gen_time; r.dist = dist;
         r.decay_t = decay_t; r.scatter_path = scatter_path; r.hu = hu; r.hv = hv;
-        r.pid = pid; r.events_left = events_left;
+        r.pid = pid(); r.events_left = events_left;
         r.k0 = rng.k0; r.k1 = rng.k1; r.blk = rng.blk;
         r.b0 = rng.b0; r.b1 = rng.b1; r.b2 = rng.b2; r.b3 = rng.b3; r.avail = rng.avail;
         r.structure = structure; r.last_hit = last_hit; r.tele_from = tele_from;
         r.nb_bounces = nb_bounces; r.nb_events = nb_events; r.variant = vi; r.tr_n = tr_n;
     }
-    __device__ uint64_t restore(const CarryRec& r) {
+    MFG_IN uint64_t restore(const CarryRec& r) {
         pos = mk(r.pos[0], r.pos[1], r.pos[2]);
         dir = mk(r.dir[0], r.dir[1], r.dir[2]);
-        time = r.time; vel = r.vel; ori = r.ori; gen_time = r.gen_time; dist = r.dist;
-        decay_t = r.decay_t; scatter_path = r.scatter_path; hu = r.hu; hv = r.hv;
-        pid = r.pid;
+        vel = r.vel;
+        if constexpr (WEIGHTED) ori = r.ori;
+        if constexpr (CLOCKED) {
+            time = r.time; gen_time = r.gen_time; dist = r.dist;
+            decay_t = r.decay_t; scatter_path = r.scatter_path; hu = r.hu; hv = r.hv;
+            tele_from = r.tele_from; nb_bounces = r.nb_bounces; nb_events = r.nb_events; tr_n = r.tr_n;
+        }
         rng.k0 = r.k0; rng.k1 = r.k1; rng.p0 = (uint32_t)r.pid; rng.p1 = (uint32_t)(r.pid >> 32);
         rng.blk = r.blk; rng.b0 = r.b0; rng.b1 = r.b1; rng.b2 = r.b2; rng.b3 = r.b3; rng.avail = r.avail;
-        structure = r.structure; last_hit = r.last_hit; tele_from = r.tele_from;
-        nb_bounces = r.nb_bounces; nb_events = r.nb_events; tr_n = r.tr_n;
+        structure = r.structure; last_hit = r.last_hit;
         return r.events_left;
     }
 
-    __device__ void flush_lane() {
+    MFG_IN double hit_equiv() const { return WEIGHTED ? acc_hit_equiv : (double)acc_hits; }
+    MFG_IN double abs_equiv() const { return WEIGHTED ? acc_abs_equiv : (double)acc_absorbed; }
+    MFG_IN double dist_full() const { return CLOCKED ? acc_dist_full : acc_dist_total; }
+    MFG_IN void flush_lane() {
         if (var == nullptr) return;
-        DGlobal* gl = P.glob + var->glob_index;
+        DGlobal* gl = P.glob + vc().glob_index;
         if (acc_hits) atomic_addu(&gl->nb_mc_hit, acc_hits);
         if (acc_des) atomic_addu(&gl->nb_desorbed, acc_des);
-        if (acc_hit_equiv != 0.0) atomic_addd(&gl->nb_hit_equiv, acc_hit_equiv);
-        if (acc_abs_equiv != 0.0) atomic_addd(&gl->nb_abs_equiv, acc_abs_equiv);
+        if (hit_equiv() != 0.0) atomic_addd(&gl->nb_hit_equiv, hit_equiv());
+        if (abs_equiv() != 0.0) atomic_addd(&gl->nb_abs_equiv, abs_equiv());
         if (acc_leak) atomic_addu(&gl->nb_leak, acc_leak);
         if (acc_dist_total != 0.0) atomic_addd(&gl->dist_total, acc_dist_total);
-        if (acc_dist_full != 0.0) atomic_addd(&gl->dist_full, acc_dist_full);
+        if (dist_full() != 0.0) atomic_addd(&gl->dist_full, dist_full());
         if (acc_decay) atomic_addu(&gl->nb_decayed, acc_decay);
-        acc_hits = acc_des = acc_leak = acc_decay = 0;
+        acc_hits = acc_des = acc_absorbed = acc_leak = acc_decay = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
     }
 
+    MFG_IN int32_t find_root() const {
+        if constexpr (ONE) { if (P.one_root != -2) return P.one_root; }
+        return P.roots[vc().root_base + (uint32_t)structure];
+    }
     // One event of an alive particle (one SimulationMCStep iteration): its
     // ray goes into the wave's walk, which all lanes run together (also
     // those without a particle), then finish() treats what it met.
-    __device__ void trace_ray(uint32_t lane, bool alive) {
+    MFG_IN void trace_ray(uint32_t lane, bool alive) {
         int32_t root = -1;
         if (alive) {
-            ++nb_events;
-            root = P.roots[var->root_base + (uint32_t)structure];
+            if constexpr (CLOCKED) ++nb_events;
+            root = find_root();
             walk_load(W, lane, pos, dir, last_hit, 1e300);
         }
         const CoinState cs{rng.k0, rng.k1, rng.p0, rng.p1, nb_events, time, var};
@@ -1603,7 +1668,7 @@ struct Tracer {
         dir = mk(b.y, c.x, c.y);
     }
     // Returns false when the particle ends.
-    __device__ bool finish(uint32_t lane) {
+    MFG_IN bool finish(uint32_t lane) {
         constexpr bool TR = (FEAT & FEAT_TRANSPARENT) != 0;
         HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
         if (h.facet < 0) {  // leak
@@ -1619,14 +1684,14 @@ struct Tracer {
         double travel = h.t;
         int ev = 0;
         if constexpr ((FEAT & FEAT_VOLUME) != 0) {
-            if (!var->calc_const_flow) { double dl = vel * 100.0 * (var->latest - time); if (dl < travel) { travel = dl; ev = 1; } }
-            if (var->enable_decay) { double dd = vel * 100.0 * (decay_t - time); if (dd < travel) { travel = dd; ev = 2; } }
-            if (var->scatter_enabled) { double ds = scatter_path - dist; if (ds < travel) { travel = ds; ev = 3; } }
+            if (!vc().calc_const_flow) { double dl = vel * 100.0 * (vc().latest - time); if (dl < travel) { travel = dl; ev = 1; } }
+            if (vc().enable_decay) { double dd = vel * 100.0 * (decay_t - time); if (dd < travel) { travel = dd; ev = 2; } }
+            if (vc().scatter_enabled) { double ds = scatter_path - dist; if (ds < travel) { travel = ds; ev = 3; } }
         }
         if constexpr (TR) {
-            if (var->flags & FEAT_TRANSPARENT) {
+            if (vc().flags & FEAT_TRANSPARENT) {
                 // second walk: every transparent pass closer than `travel`
-                const int32_t root = P.roots[var->root_base + (uint32_t)structure];
+                const int32_t root = find_root();
                 const LaneStack S{W.nodes + lane, MFG_LANE_STACK, P.stack_total, spill};
                 Ray32 r = make_ray32(pos, dir);
                 float tbf = widen(travel);
@@ -1666,42 +1731,47 @@ struct Tracer {
                 hu = save_u; hv = save_v;
             }
         }
-        if (ev == 0) hit_uv(P.facets + h.facet, pos, dir, h.t, h.u, h.v);
+        const int32_t f = h.facet;
+        const HitRegs H = load_hit(P.hits + f);
+        // the hit's facet coordinates, for the recordings that use them
+        if (ev == 0 && (CLOCKED || (H.flags & (FF_TEXTURE | FF_PROFILE)))) hit_uv(P.facets + f, pos, dir, h.t, hu, hv);
         pos = add(pos, scl(travel, dir));
-        time += travel / 100.0 / vel;
+        if constexpr (CLOCKED) time += travel / 100.0 / vel;
         if (ev == 0) {
-            int32_t f = h.facet;
-            const DPhys& ph = P.phys[f];
-            hu = h.u; hv = h.v;
-            acc_dist_total += travel; acc_dist_full += travel; dist += travel;
+            acc_dist_total += travel;
+            if constexpr (CLOCKED) { acc_dist_full += travel; dist += travel; }
             if constexpr ((FEAT & FEAT_TELEPORT) != 0) {
-                if (ph.teleport_dest != 0) { teleport(f); return true; }
+                if (H.flags & FF_TELEPORT) { teleport(H, f); return true; }
             }
-            double s = sticking(ph);
-            bool lowflux = false;
-            if constexpr ((FEAT & FEAT_LOWFLUX) != 0) lowflux = var->low_flux != 0;
+            // absorption, or the weight's absorbed part (low flux), then the
+            // bounce of what is left
+            const double s = sticking(H, f);
+            bool rec, go, lowflux = false;
+            double w0 = 1.0;
+            if constexpr (WEIGHTED) { lowflux = vc().low_flux != 0; w0 = ori; }
             if (!lowflux) {
-                if (s == 1.0 || (s > 0.0 && rng.rnd() < s)) { record_absorb(f); trace(f, 2); return false; }
-                bounce(f);
-                return true;
-            }
-            if (s > 0.0) {
-                double w0 = ori;
-                ori *= s;
-                record_absorb(f);
-                ori = w0 * (1.0 - s);
-                if constexpr ((FEAT & FEAT_ADJOINT) != 0) { if (ph.adj_group >= 0) adj_cnt[ph.adj_group] += 1; }
+                rec = s == 1.0 || (s > 0.0 && rng.rnd() < s);
+                go = !rec;
             } else {
-                ori *= (1.0 - s);
+                rec = s > 0.0;
+                go = true;
+                if constexpr (WEIGHTED) { if (rec) ori *= s; }
             }
-            if (ori > var->low_flux_cutoff) {
-                if constexpr ((FEAT & FEAT_ADJOINT) != 0) { if (s > 0.0) seg_n = 0; }
-                bounce(f);
-                return true;
+            if (rec) record_absorb(H, f);
+            if constexpr (WEIGHTED) {
+                if (lowflux) {
+                    ori = w0 * (1.0 - s);
+                    if constexpr ((FEAT & FEAT_ADJOINT) != 0) { const int32_t g = P.hits[f].adj_group; if (rec && g >= 0) adj_cnt[g] += 1; }
+                    go = ori > vc().low_flux_cutoff;
+                    if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
+                        if (rec && go) seg_n = 0;
+                        if (rec && !go) cutoff_boundary(P.hits[f].adj_group, s);
+                    }
+                }
             }
-            if constexpr ((FEAT & FEAT_ADJOINT) != 0) { if (s > 0.0) cutoff_boundary(ph, s); }
-            trace(f, 2);
-            return false;
+            if (go) bounce(H, f);
+            else trace(f, 2);
+            return go;
         }
         if (ev == 1 || ev == 2) {
             acc_dist_total += travel;
@@ -1723,14 +1793,14 @@ __device__ __forceinline__ uint32_t find_variant(const uint64_t* prefix, uint32_
     return lo;
 }
 
-template <uint32_t FEAT>
+template <uint32_t FEAT, bool ONE>
 __device__ __forceinline__ void trace_body(const TraceParams& P) {
     extern __shared__ __align__(16) unsigned char lds_base[];
     const uint32_t lane = __lane_id();
     WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     const size_t gl = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     int32_t* spill = P.stack_spill ? P.stack_spill + gl * (P.stack_total - MFG_LANE_STACK) : nullptr;
-    Tracer<FEAT> T(P, W, spill);
+    Tracer<FEAT, ONE> T(P, W, spill);
     // hot-facet counters after the waves' walk areas
     double* hot = reinterpret_cast<double*>(lds_base + (blockDim.x >> 6) * sizeof(WaveLds));
     for (uint32_t i = threadIdx.x; i < 8u * P.n_hot; i += blockDim.x) hot[i] = 0.0;
@@ -1800,18 +1870,22 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                 uint64_t g = base + mbcnt(mask);
                 if (g < n_in) {
                     const CarryRec& r = carry_in[g];
-                    vi = r.variant;
-                    if (T.var != P.variants + vi) T.flush_lane();
+                    if constexpr (!ONE) {
+                        vi = r.variant;
+                        if (T.var != P.variants + vi) T.flush_lane();
+                    }
                     T.var = P.variants + vi;
                     events_left = T.restore(r);
                     alive = true;
                 } else if (g < limit) {
                     uint64_t d = g - n_in;
-                    vi = P.n_variants > 1 ? find_variant(P.var_prefix, P.n_variants, d) : 0;
-                    if (T.var != P.variants + vi) T.flush_lane();
+                    if constexpr (!ONE) {
+                        vi = find_variant(P.var_prefix, P.n_variants, d);
+                        if (T.var != P.variants + vi) T.flush_lane();
+                    }
                     T.var = P.variants + vi;
                     ++T.acc_des;
-                    uint64_t lp = d - P.var_prefix[vi] + T.var->pid_base;
+                    uint64_t lp = (ONE ? d : d - P.var_prefix[vi]) + T.var->pid_base;
                     src = T.start(lp);
                     started = true;
                     alive = true;
@@ -1825,12 +1899,11 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
             // add through one set of atomics
             uint64_t smask = __ballot(started);
             if (smask) {
-                const DPhys* ph = started ? &P.phys[src] : nullptr;
                 double ov = 0.0, w1 = 0.0, w2 = 0.0, w3 = 0.0;
                 int m = -1;
                 if (started) {
-                    ov = T.vel * fabs(dot(T.dir, ld3(P.facets[src].N)));
-                    w1 = 2.0 / ov; w2 = T.var->c_factor * ov; w3 = 1.0 / T.vel;
+                    ov = T.vel * fabs(dot(T.dir, ld3(P.hits[src].N)));
+                    w1 = 2.0 / ov; w2 = T.vc().c_factor * ov; w3 = 1.0 / T.vel;
                     m = T.moment(T.time);
                 }
                 uint32_t sl = (uint32_t)__ffsll((unsigned long long)smask) - 1;
@@ -1839,14 +1912,15 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                 uint64_t gmask = __ballot(grp);
                 double s1 = wave_sum(grp ? w1 : 0.0), s2 = wave_sum(grp ? w2 : 0.0), s3 = wave_sum(grp ? w3 : 0.0);
                 if (grp && lane == sl) {
-                    if (ph->hot_idx >= 0) {
-                        double* h = hot + 8 * ph->hot_idx;
+                    const int32_t hi = P.hits[src].hot_idx;
+                    if (hi >= 0) {
+                        double* h = hot + 8 * hi;
                         atomicAdd(reinterpret_cast<unsigned long long*>(h + 2), (unsigned long long)__popcll(gmask));
                         atomic_addd(h + 4, s1);
                         atomic_addd(h + 5, s2);
                         atomic_addd(h + 6, s3);
                     } else {
-                        mfg_facet_counters* c = T.fc(*ph, 0);
+                        mfg_facet_counters* c = T.fc(src, 0);
                         atomic_addu(&c->nb_desorbed, (unsigned long long)__popcll(gmask));
                         atomic_addd(&c->sum_1_per_ort_velocity, s1);
                         atomic_addd(&c->sum_v_ort, s2);
@@ -1854,7 +1928,7 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                     }
                 }
                 if (started && !grp) {
-                    mfg_facet_counters* c = T.fc(*ph, 0);
+                    mfg_facet_counters* c = T.fc(src, 0);
                     atomic_addu(&c->nb_desorbed, 1ull);
                     atomic_addd(&c->sum_1_per_ort_velocity, w1);
                     atomic_addd(&c->sum_v_ort, w2);
@@ -1910,13 +1984,13 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     }
     // flush lane accumulators: one set of atomics per wave for a single
     // variant, per lane otherwise
-    if (P.n_variants == 1) {
-        double he = wave_sum(T.acc_hit_equiv), ae = wave_sum(T.acc_abs_equiv);
-        double d1 = wave_sum(T.acc_dist_total), d2 = wave_sum(T.acc_dist_full);
+    if constexpr (ONE) {
+        double he = wave_sum(T.hit_equiv()), ae = wave_sum(T.abs_equiv());
+        double d1 = wave_sum(T.acc_dist_total), d2 = wave_sum(T.dist_full());
         unsigned long long hits = wave_sum_u(T.acc_hits), des = wave_sum_u(T.acc_des);
         unsigned long long lk = wave_sum_u(T.acc_leak), dc = wave_sum_u(T.acc_decay);
         if (lane == 0) {
-            DGlobal* gl = P.glob + P.variants[0].glob_index;
+            DGlobal* gl = P.glob + P.one.glob_index;
             if (hits) atomic_addu(&gl->nb_mc_hit, hits);
             if (des) atomic_addu(&gl->nb_desorbed, des);
             if (he != 0.0) atomic_addd(&gl->nb_hit_equiv, he);
@@ -1948,18 +2022,18 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
 // One instantiation per occupancy bound: WAVES waves per SIMD caps the
 // VGPR budget (cold per-particle state spills to scratch at the higher
 // bounds); the host autotuner picks the fastest for a model.
-template <uint32_t FEAT, int WAVES>
+template <uint32_t FEAT, int WAVES, bool ONE>
 __global__ void __launch_bounds__(256, WAVES) k_trace(TraceParams P) {
-    trace_body<FEAT>(P);
+    trace_body<FEAT, ONE>(P);
 }
 
 // One block per CU of 256 lanes per wave slot (768 lanes at 3 waves per
 // SIMD, 1024 at 4): all waves of a CU share one LDS copy of the top of the
 // tree, which can then hold several times the nodes of a 256-lane block's
-// copy (same per-lane LDS budget).
+// copy (single-variant launches: the others keep no copy).
 template <uint32_t FEAT, int WAVES>
 __global__ void __launch_bounds__(256 * WAVES, WAVES) k_trace_cu(TraceParams P) {
-    trace_body<FEAT>(P);
+    trace_body<FEAT, true>(P);
 }
 
 // Parked particles that a launch did not claim: the queue hands out items
@@ -2079,56 +2153,61 @@ TraceKernel kernel_cu(uint32_t features, int waves) {
     return nullptr;
 }
 
-TraceKernel kernel_for(uint32_t features, int waves) {
-    constexpr int N = 5;   // occupancy bounds 1..5 waves per SIMD
-    static TraceKernel lean[N] = {nullptr, k_trace<kLean, 2>, k_trace<kLean, 3>, k_trace<kLean, 4>, k_trace<kLean, 5>};
-    static TraceKernel full[N] = {k_trace<kFull, 1>, k_trace<kFull, 2>, k_trace<kFull, 3>, nullptr, nullptr};
-    static TraceKernel adj[N] = {k_trace<kFullAdj, 1>, k_trace<kFullAdj, 2>, nullptr, nullptr, nullptr};
-    static TraceKernel lowflux[N] = {nullptr, k_trace<kLowFlux, 2>, k_trace<kLowFlux, 3>, k_trace<kLowFlux, 4>,
-                                     k_trace<kLowFlux, 5>};
-    static TraceKernel lowflux_adj[N] = {nullptr, k_trace<kLowFluxAdj, 2>, k_trace<kLowFluxAdj, 3>,
-                                         k_trace<kLowFluxAdj, 4>, nullptr};
-    TraceKernel* t = features == kLean ? lean
-                   : features == kFull ? full
-                   : features == kLowFlux ? lowflux
-                   : features == kLowFluxAdj ? lowflux_adj : adj;
+template <bool ONE>
+TraceKernel kernel_of(uint32_t features, int waves) {
+    constexpr int N = 4;   // occupancy bounds 1..4 waves per SIMD (a fifth's walk areas do not fit the LDS)
+    static TraceKernel lean[N] = {nullptr, k_trace<kLean, 2, ONE>, k_trace<kLean, 3, ONE>, k_trace<kLean, 4, ONE>};
+    static TraceKernel full[N] = {k_trace<kFull, 1, ONE>, k_trace<kFull, 2, ONE>, k_trace<kFull, 3, ONE>, nullptr};
+    static TraceKernel lowflux[N] = {nullptr, k_trace<kLowFlux, 2, ONE>, k_trace<kLowFlux, 3, ONE>, k_trace<kLowFlux, 4, ONE>};
+    TraceKernel* t = features == kLean ? lean : features == kFull ? full : features == kLowFlux ? lowflux : nullptr;
+    if constexpr (ONE) {
+        // the adjoint takes one model
+        static TraceKernel adj[N] = {k_trace<kFullAdj, 1, true>, k_trace<kFullAdj, 2, true>, nullptr, nullptr};
+        static TraceKernel lowflux_adj[N] = {nullptr, k_trace<kLowFluxAdj, 2, true>, k_trace<kLowFluxAdj, 3, true>,
+                                             k_trace<kLowFluxAdj, 4, true>};
+        if (!t) t = features == kLowFluxAdj ? lowflux_adj : adj;
+    }
+    if (!t) return nullptr;
     if (waves < 1) waves = 1;
     if (waves > N) waves = N;
     for (int w = waves; w >= 1; --w) if (t[w - 1]) return t[w - 1];
     for (int w = waves; w <= N; ++w) if (t[w - 1]) return t[w - 1];
-    return t[0];
+    return nullptr;
+}
+TraceKernel kernel_for(uint32_t features, bool single, int waves, int block) {
+    if (block > 256) return single ? kernel_cu(features, block / 256) : nullptr;
+    return single ? kernel_of<true>(features, waves) : kernel_of<false>(features, waves);
 }
 }  // namespace
 
 int mfg_trace_variants(uint32_t features, int* waves_out, int cap) {
     uint32_t f = mfg_trace_kernel_features(features);
     int lo = 1, hi = 2;
-    if (f == kLean || f == kLowFlux) { lo = 2; hi = 5; }
-    else if (f == kLowFluxAdj) { lo = 2; hi = 4; }
+    if (f == kLean || f == kLowFlux || f == kLowFluxAdj) { lo = 2; hi = 4; }
     else if (f == kFull) hi = 3;
     int n = 0;
     for (int w = lo; w <= hi && n < cap; ++w) waves_out[n++] = w;
     return n;
 }
 
-int mfg_trace_has_cu_block(uint32_t features, int block) {
-    return block % 256 == 0 && kernel_cu(mfg_trace_kernel_features(features), block / 256) != nullptr;
+int mfg_trace_has_cu_block(uint32_t features, bool single, int block) {
+    return single && block % 256 == 0 && kernel_cu(mfg_trace_kernel_features(features), block / 256) != nullptr;
 }
 
-int mfg_trace_occupancy(uint32_t features, int waves, int block, size_t lds) {
+int mfg_trace_occupancy(uint32_t features, bool single, int waves, int block, size_t lds) {
     int n = 0;
     const uint32_t f = mfg_trace_kernel_features(features);
-    TraceKernel k = block > 256 ? kernel_cu(f, block / 256) : kernel_for(f, waves);
+    TraceKernel k = kernel_for(f, single, waves, block);
     if (!k) return 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, block, lds);
     return e == hipSuccess ? n : 1;
 }
 
-int mfg_launch_trace(const TraceParams& p, uint32_t features, int waves, int grid, int block, void* stream) {
+int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int waves, int grid, int block, void* stream) {
     size_t lds = (size_t)(block / 64) * sizeof(WaveLds) + (size_t)p.n_hot * 8 * sizeof(double) +
                  (size_t)p.lds_nodes * sizeof(BvhNode);
     const uint32_t f = mfg_trace_kernel_features(features);
-    TraceKernel k = block > 256 ? kernel_cu(f, block / 256) : kernel_for(f, waves);
+    TraceKernel k = kernel_for(f, single, waves, block);
     if (!k) return -1;
     hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, (hipStream_t)stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -1;

@@ -62,3 +62,31 @@ def test_lane_quota_same_seed_tallies(sim, n_des):
     a, b = t.facets[0]["nb_mc_hit"].astype(np.int64), c.facets[0]["nb_mc_hit"].astype(np.int64)
     # a few long trajectories may part by FP64 rounding of the math library
     assert np.abs(a - b).sum() <= 2e-4 * b.sum()
+
+
+def test_parked_lean_particles_resume_in_the_full_kernel(sim):
+    """Particles parked by the kernel without a clock and resumed by the one
+    with it (event tracing switches kernels) end as in one run."""
+    m = geometry.tube_model(1.0, 6.0, 16, 8)
+    n = 200_000
+    sim.load(m)
+    sim.rebuild_accel()
+    sim.set_carry(False)
+    sim.reset(seed=4)
+    sim.run(n)
+    one = sim.read()
+    sim.reset(seed=4)
+    sim.set_carry(True)
+    sim.run(n)
+    parked = sim.in_flight()
+    sim.set_trace(8, 16)
+    sim.drain()
+    sim.set_trace(0, 0)
+    two = sim.read()
+    assert parked > 1000
+    for fld in ("nb_mc_hit", "nb_desorbed"):
+        assert np.array_equal(one.facets[fld], two.facets[fld])
+    for fld in ("nb_abs_equiv", "sum_1_per_ort_velocity", "sum_v_ort", "sum_1_per_velocity"):
+        assert np.allclose(one.facets[fld], two.facets[fld], rtol=1e-9, atol=0)
+    assert one.glob[0]["nb_mc_hit"] == two.glob[0]["nb_mc_hit"]
+    assert np.isclose(one.glob[0]["dist_traveled_total"], two.glob[0]["dist_traveled_total"], rtol=1e-12)
