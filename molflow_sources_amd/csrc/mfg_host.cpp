@@ -897,7 +897,31 @@ struct mfg_context {
     DevBuf<LeafUV> leaf_uv;
     std::vector<DPhys> h_phys;           // host copy of the uploaded physics records
     std::vector<int32_t> hot;            // hot facets (global index), their counters summed in LDS
-    DevBuf<uint64_t> hot_fc;
+    // slots of each kept there: all that fit 24 KB (at two blocks of 256
+    // lanes a CU that leaves the walks their LDS and some of the tree), one
+    // model only. Device-scope atomics on one record are served one after
+    // the other: the time-dependent tube (101 slots; 3 facets and 100 profile
+    // slices take most updates) went from 160 to 14.6 ms a launch with these
+    // slots in LDS and, the transparent passes coming from the walk, from
+    // 12.4 to 5.9 ms with the profile's first 5 slots beside them.
+    uint32_t hot_slots() const {
+        if (dvars.size() != 1 || hot.empty()) return 1;
+        return std::max<uint32_t>(1, std::min<uint32_t>(dvars[0].n_slots, (uint32_t)(24576 / (64 * hot.size()))));
+    }
+    // profiles summed in LDS: those of a model (one variant) that has at most
+    // MFG_MAX_PROF_HOT, all slots that fit 12 KB (at least the steady state)
+    uint32_t n_prof_hot = 0;
+    uint32_t prof_slots() const {
+        if (n_prof_hot == 0) return 1;
+        const uint32_t per = (uint32_t)(MFG_PROFILE_SIZE * sizeof(mfg_profile_slice)) * n_prof_hot;
+        return std::max<uint32_t>(1, std::min<uint32_t>(dvars[0].n_slots, 12288 / per));
+    }
+    // LDS of a block's hot counters and profiles
+    size_t hot_bytes() const {
+        return hot.size() * hot_slots() * sizeof(mfg_facet_counters) +
+               (size_t)n_prof_hot * prof_slots() * MFG_PROFILE_SIZE * sizeof(mfg_profile_slice);
+    }
+    DevBuf<uint64_t> hot_fc, hot_prof;
     std::vector<DFacet> h_facets;        // host copies of the concatenated facets and polygons
     std::vector<double> h_poly;
     DevBuf<uint32_t> guides;
@@ -1119,25 +1143,42 @@ void upload_models(mfg_context* c) {
     }
     hipStream_t s = c->stream;
     c->h_phys = phys;
-    // default hot facets of each variant: its sources and absorbers when
-    // there are only a few of them (the autotuner refines the choice from
+    // default hot facets of each variant: its sources, absorbers and
+    // transparent facets when there are only a few of them (the autotuner refines the choice from
     // measured counts)
     std::vector<int32_t> hot;
     for (size_t vi = 0; vi < c->models.size(); ++vi) {
         const HostModel& M = *c->models[vi];
         const uint32_t fb = c->dvars[vi].facet_base;
-        std::vector<int32_t> src(M.src_facet.begin(), M.src_facet.end()), ab;
-        for (size_t f = 0; f < M.phys.size(); ++f)
+        std::vector<int32_t> src(M.src_facet.begin(), M.src_facet.end()), ab, tr;
+        for (size_t f = 0; f < M.phys.size(); ++f) {
             if (M.phys[f].sticking > 0.0 || M.phys[f].sticking_param >= 0) ab.push_back((int32_t)f);
+            if (M.phys[f].opacity < 1.0 || M.phys[f].opacity_param >= 0) tr.push_back((int32_t)f);
+        }
         std::vector<int32_t> pick;
         if (src.size() <= 4) pick.insert(pick.end(), src.begin(), src.end());
         if (ab.size() <= 8) pick.insert(pick.end(), ab.begin(), ab.end());
+        if (tr.size() <= 4) pick.insert(pick.end(), tr.begin(), tr.end());
         std::sort(pick.begin(), pick.end());
         pick.erase(std::unique(pick.begin(), pick.end()), pick.end());
         for (int32_t f : pick) if (hot.size() < MFG_MAX_HOT) hot.push_back(f + (int32_t)fb);
     }
     c->hot.clear();
     set_hot_facets(c, hot, false);
+    // profiles kept in LDS
+    std::vector<uint64_t> hot_prof;
+    for (size_t f = 0; f < c->h_phys.size(); ++f) {
+        c->h_phys[f].prof_hot = -1;
+        if (c->models.size() == 1 && c->h_phys[f].prof_off >= 0) hot_prof.push_back(f);
+    }
+    if (hot_prof.size() > MFG_MAX_PROF_HOT) hot_prof.clear();
+    c->n_prof_hot = (uint32_t)hot_prof.size();
+    for (size_t k = 0; k < hot_prof.size(); ++k) {
+        DPhys& ph = c->h_phys[hot_prof[k]];
+        ph.prof_hot = (int32_t)k;
+        hot_prof[k] = c->dvars[0].prof_base + (uint64_t)ph.prof_off;
+    }
+    c->hot_prof.upload(hot_prof, s);
     c->h_facets = facets;
     c->facets.upload(facets, s); c->poly.upload(poly, s);
     upload_phys(c);
@@ -1327,10 +1368,10 @@ void build_accel(mfg_context* c, int width, int leaf) {
 // many as fit beside the waves' walk areas and the hot facets in a block's
 // share of the CU's LDS (all of it for a block of 768 or 1024 lanes, else a
 // 1 / waves part for every 256 lanes).
-uint32_t lds_node_count(const mfg_context* c, int block, int waves) {
+uint32_t lds_node_count(const mfg_context* c, uint32_t feats, int block, int waves) {
     if (c->dvars.size() != 1) return 0;
     const size_t share = block > 256 ? c->lds_per_block : c->lds_per_block * (size_t)block / 256 / (size_t)std::max(1, waves);
-    const size_t used = (size_t)(block / 64) * MFG_WAVE_LDS + c->hot.size() * 8 * sizeof(double) + 256;
+    const size_t used = (size_t)(block / 64) * mfg_wave_lds(feats) + c->hot_bytes() + 256;
     size_t n = share > used ? (share - used) / sizeof(BvhNode) : 0;
     if (block <= 256) n = std::min<size_t>(n, c->node_cache);
     return (uint32_t)std::min<size_t>(n, c->nodes.n);
@@ -1348,7 +1389,8 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     p.stack_total = c->stack_size;
     p.stack_spill = p.stack_total > MFG_LANE_STACK ? c->stack_spill.p : nullptr;
     p.src_cum = c->src_cum.p; p.src_facet = c->src_facet.p; p.og_cdf = c->og_cdf.p; p.am_src = c->am_src.p;
-    p.hot_fc = c->hot_fc.p; p.n_hot = (uint32_t)c->hot.size();
+    p.hot_fc = c->hot_fc.p; p.n_hot = (uint32_t)c->hot.size(); p.hot_slots = c->hot_slots();
+    p.hot_prof = c->hot_prof.p; p.n_prof_hot = c->n_prof_hot; p.prof_slots = c->prof_slots();
     p.guides = c->guides.p; p.tab_x = c->tab_x.p; p.tab_y = c->tab_y.p; p.params = c->params.p; p.ids = c->ids.p;
     p.mom_start = c->mom_start.p; p.mom_end = c->mom_end.p;
     p.fc = c->fc.p; p.force = c->force.p; p.tex = c->tex.p; p.tex_inc = c->tex_inc.p; p.dir = c->dir.p;
@@ -1387,8 +1429,8 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
         else block = 256;
     }
     auto lds_bytes = [&](int b) {
-        return (size_t)(b / 64) * MFG_WAVE_LDS + c->hot.size() * 8 * sizeof(double) +
-               (size_t)lds_node_count(c, b, waves) * sizeof(BvhNode);
+        return (size_t)(b / 64) * mfg_wave_lds(feats) + c->hot_bytes() +
+               (size_t)lds_node_count(c, feats, b, waves) * sizeof(BvhNode);
     };
     if (block > 256 && mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block)) < 1) {
         block = 256;   // the block's LDS does not fit
@@ -1462,7 +1504,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     HIPCHK(hipMemcpyAsync(before.data(), c->glob.p, nv * sizeof(DGlobal), hipMemcpyDeviceToHost, s));
     *c->stop_host = 0;
     TraceParams p = make_params(c, total, max_events);
-    p.lds_nodes = lds_node_count(c, block, waves);
+    p.lds_nodes = lds_node_count(c, feats, block, waves);
     // lanes of a wave that take particles: all once there is one for every
     // lane, else the items are spread over all waves, whose other lanes then
     // help with the walks (a wave's step gets shorter the fewer rays it has:
@@ -1562,10 +1604,10 @@ void add_tallies(mfg_context* c, uint32_t vi, const mfg_tally_view* o) {
     uint64_t S = L.n_slots;
     if (o->facets) {
         auto h = fetch(c->fc.p, L.fc, S * L.n_facets);
-        // without low-flux weighting the kernel leaves the slot-0 hit
-        // equivalents to this read: every hit weighs 1
+        // without low-flux weighting the kernel leaves the hit equivalents
+        // to this read: every hit weighs 1
         if (!c->dvars[vi].low_flux)
-            for (uint64_t i = 0; i < L.n_facets; ++i) h[i].nb_hit_equiv = (double)h[i].nb_mc_hit;
+            for (uint64_t i = 0; i < h.size(); ++i) h[i].nb_hit_equiv = (double)h[i].nb_mc_hit;
         for (size_t i = 0; i < h.size(); ++i) {
             auto& a = o->facets[i]; const auto& b = h[i];
             a.nb_mc_hit += b.nb_mc_hit; a.nb_hit_equiv += b.nb_hit_equiv; a.nb_desorbed += b.nb_desorbed;

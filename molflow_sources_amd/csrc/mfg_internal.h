@@ -27,6 +27,7 @@
 #define MFG_MAX_GROUPS 64
 #define MFG_MAXWELL_GUIDE 128
 #define MFG_MAX_HOT 32           // facets whose counters are privatised per block
+#define MFG_MAX_PROF_HOT 4       // profiles privatised per block
 
 // feature bits of a trace-kernel instantiation / of a loaded model
 enum : uint32_t {
@@ -118,7 +119,7 @@ struct alignas(16) DPhys {
     int32_t pad_;
     int64_t am_src_off;             // DES_ANGLEMAP source table in the pool (global), -1
     int32_t hot_idx;                // slot in the per-block hot-facet counter table, -1
-    int32_t pad2_;
+    int32_t prof_hot;               // index among the profiles summed in LDS, -1
 };
 
 // What a wall event always needs of its facet, in one line: loaded as six
@@ -192,10 +193,13 @@ struct alignas(16) WaveLds {
     uint32_t leaves[MFG_WALK_LEAVES];  // ray << task_bits | facet record
 };
 #endif
-#define MFG_WAVE_LDS 8960
-#ifdef __HIPCC__
-static_assert(sizeof(WaveLds) == MFG_WAVE_LDS, "MFG_WAVE_LDS is the size of WaveLds");
-#endif
+// Transparent facets each ray of a wave met on its walk (more than
+// MFG_PASSES: only counted), beside WaveLds in the kernels that need it.
+#define MFG_PASSES 4
+struct alignas(16) PassLds {
+    uint32_t n[64];
+    uint32_t rec[64][MFG_PASSES];      // facet records
+};
 
 // global counters of one variant (mfg_global_counters)
 struct DGlobal {
@@ -302,10 +306,16 @@ struct TraceParams {
     // [W, L, H, theta limit, lower ratio, total count, line sums (T),
     //  theta CDF (T), phi CDFs (T*W), phi pdfs (T*W)], T = L + H
     const double* am_src;
-    // hot facets: their slot-0 counter updates are summed in LDS per block
+    // hot facets: their counter updates of the first hot_slots slots (0 =
+    // steady state, then the moments) are summed in LDS per block
     // and added to the global records once, when the block ends
     const uint64_t* hot_fc;           // index into fc of each hot facet's slot-0 record
     uint32_t n_hot;
+    uint32_t hot_slots;               // slots of each kept there (1 with several variants)
+    // profiles of a model with few of them: the slices of the first
+    // prof_slots slots are summed in LDS per block, like the hot facets
+    const uint64_t* hot_prof;         // first slice of each in slot 0
+    uint32_t n_prof_hot, prof_slots;
     // tallies
     mfg_facet_counters* fc;
     double* force;
@@ -406,6 +416,8 @@ int mfg_launch_zero(void* ptr, uint64_t bytes, void* stream);
 int mfg_launch_backward(const double* jac, const double* up, double* grad, uint32_t n_targets, uint32_t n_groups,
                         double scale, void* stream);
 uint32_t mfg_trace_kernel_features(uint32_t model_features);
+// LDS of one wave of the kernel that runs these features (its walk areas)
+size_t mfg_wave_lds(uint32_t model_features);
 int mfg_trace_occupancy(uint32_t features, bool single, int waves, int block, size_t lds_bytes);
 int mfg_trace_variants(uint32_t features, int* waves_out, int cap);
 // 1 when the feature set has a one-block-per-CU kernel of `block` lanes

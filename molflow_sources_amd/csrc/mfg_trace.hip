@@ -641,7 +641,7 @@ struct CoinState {
 // that for the deepest tree the host accepts. The list has room for lane
 // 0's facets (8 leaves of 16) whenever a node step runs (below 64 waiting).
 template <bool TRANSP>
-__device__ void walk(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint32_t lane, bool live, int32_t root,
+__device__ void walk(const TraceParams& P, WaveLds& W, PassLds* pass, const uint4* lnodes, uint32_t lane, bool live, int32_t root,
                      const CoinState& cs) {
     const uint32_t bits = P.task_bits, low = (1u << bits) - 1u;
     uint32_t top, waiting = 0;   // wave-uniform
@@ -707,7 +707,7 @@ __device__ void walk(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint
         } else {
             const uint32_t n = waiting < 64u ? waiting : 64u;
             waiting -= n;
-            uint32_t ray = 0;
+            uint32_t ray = 0, rec = 0;
             double t = 0.0, u, v;
             int32_t f = -1;
             uint32_t fl = FF_OPAQUE;
@@ -715,7 +715,7 @@ __device__ void walk(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint
             if (lane < n) {
                 const uint32_t w = W.leaves[waiting + lane];
                 ray = w >> bits;
-                const uint32_t rec = w & low;
+                rec = w & low;
                 const double2 a = W.p01[ray], b = W.p2d0[ray], c = W.d12[ray];
                 hit = leaf_test(P.leaves + rec, P.leaf_uv + rec, P.poly, mk(a.x, a.y, b.x), mk(b.y, c.x, c.y),
                                 __float_as_int(W.rb[ray].w), t, u, v, f, fl);
@@ -733,6 +733,10 @@ __device__ void walk(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint
                     if (coin) {
                         double op = (fl & FF_TD_OPACITY) ? td_opacity(P, var, f, tm) : (double)P.phys[f].opacity;
                         if (op < 1.0) hit = (op > 0.0) && g.coin(ev, (uint32_t)(f - (int32_t)var->facet_base)) < op;
+                        if (!hit) {
+                            const uint32_t k = atomicAdd(&pass->n[ray], 1u);
+                            if (k < MFG_PASSES) pass->rec[ray][k] = rec;
+                        }
                     }
                 }
             }
@@ -811,6 +815,7 @@ struct Tracer {
     static constexpr bool WEIGHTED = (FEAT & FEAT_LOWFLUX) != 0;
     const TraceParams& P;
     WaveLds& W;                       // this wave's walk area
+    PassLds* pass;                    // this wave's transparent passes
     int32_t* spill;                   // this lane's stack entries beyond the LDS part (second walk)
     // particle state (reference Particle.h:95-122)
     d3 pos, dir;
@@ -831,13 +836,14 @@ struct Tracer {
     int32_t* seg_t;
     double* seg_x;
     double* hot;                      // LDS table of the hot facets' slot-0 counters (8 words each)
+    double* profs;                    // LDS slices of the profiles kept there
     const uint4* lnodes;              // LDS copy of the first P.lds_nodes BVH nodes
     // pending slot-0 facet counter update of this lane
     int32_t pend_f, pend_hot;
     uint32_t pend_hits;
     double pend_he, pend_abs, pend_s1v, pend_svo, pend_s1pv;
 
-    MFG_IN Tracer(const TraceParams& p, WaveLds& w, int32_t* sp) : P(p), W(w), spill(sp) {
+    MFG_IN Tracer(const TraceParams& p, WaveLds& w, PassLds* pl, int32_t* sp) : P(p), W(w), pass(pl), spill(sp) {
         acc_hits = acc_des = acc_absorbed = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
         acc_leak = acc_decay = 0;
@@ -847,7 +853,7 @@ struct Tracer {
         seg_t = nullptr;
         seg_x = nullptr;
         var = nullptr;
-        hot = nullptr;
+        hot = profs = nullptr;
         lnodes = nullptr;
         ori = 1.0;
         time = gen_time = dist = hu = hv = 0.0;
@@ -949,8 +955,15 @@ struct Tracer {
             int slot = k == 0 ? 0 : m;
             if (k == 1 && m <= 0) break;
             if (k == 0 && !force && des == 0) continue;
+            if constexpr ((FEAT & FEAT_MOMENTS) != 0) {
+                // a hot facet's moment slots, like its slot 0, in LDS
+                if (k == 1 && !force && des == 0 && H.hot >= 0 && (uint32_t)m < P.hot_slots) {
+                    add_hot(H.hot, m, hit, weighted() ? he : 0.0, (double)abs_ * w(), w() * s1v, w() * svo, s1pv);
+                    continue;
+                }
+            }
             mfg_facet_counters* c = fc(f, slot);
-            if (hit) { atomic_addu(&c->nb_mc_hit, hit); atomic_addd(&c->nb_hit_equiv, he); }
+            if (hit) { atomic_addu(&c->nb_mc_hit, hit); if (weighted()) atomic_addd(&c->nb_hit_equiv, he); }
             if (des) atomic_addu(&c->nb_desorbed, des);
             if (abs_) atomic_addd(&c->nb_abs_equiv, (double)abs_ * w());
             if (s1v != 0.0) atomic_addd(&c->sum_1_per_ort_velocity, w() * s1v);
@@ -971,9 +984,19 @@ struct Tracer {
         }
         (void)imp; (void)imp2; (void)impm;
     }
-    // Without low-flux weighting every particle weighs 1, so the slot-0
-    // nb_hit_equiv equals nb_mc_hit: it is not added here (one atomic less
-    // per hit) and the host fills it in when it reads the counters.
+    // Counter record of a hot facet in LDS (field order of mfg_facet_counters).
+    MFG_IN void add_hot(int32_t idx, int slot, uint32_t hits, double he, double ab, double s1v, double svo, double s1pv) {
+        double* h = hot + 8 * ((uint32_t)idx * P.hot_slots + (uint32_t)slot);
+        if (hits) atomicAdd(reinterpret_cast<unsigned long long*>(h), (unsigned long long)hits);
+        if (he != 0.0) atomic_addd(h + 1, he);
+        if (ab != 0.0) atomic_addd(h + 3, ab);
+        if (s1v != 0.0) atomic_addd(h + 4, s1v);
+        if (svo != 0.0) atomic_addd(h + 5, svo);
+        if (s1pv != 0.0) atomic_addd(h + 6, s1pv);
+    }
+    // Without low-flux weighting every particle weighs 1, so nb_hit_equiv
+    // equals nb_mc_hit: it is not added here (one atomic less per hit) and
+    // the host fills it in when it reads the counters.
     MFG_IN bool weighted() const {
         if constexpr (WEIGHTED) return vc().low_flux != 0;
         return false;
@@ -983,15 +1006,7 @@ struct Tracer {
         if (pend_f < 0) return;
         const bool w = weighted();
         if (pend_hot >= 0) {
-            double* h = hot + 8 * pend_hot;   // same field order as mfg_facet_counters
-            if (pend_hits) {
-                atomicAdd(reinterpret_cast<unsigned long long*>(h), (unsigned long long)pend_hits);
-                if (w) atomic_addd(h + 1, pend_he);
-            }
-            if (pend_abs != 0.0) atomic_addd(h + 3, pend_abs);
-            if (pend_s1v != 0.0) atomic_addd(h + 4, pend_s1v);
-            if (pend_svo != 0.0) atomic_addd(h + 5, pend_svo);
-            if (pend_s1pv != 0.0) atomic_addd(h + 6, pend_s1pv);
+            add_hot(pend_hot, 0, pend_hits, w ? pend_he : 0.0, pend_abs, pend_s1v, pend_svo, pend_s1pv);
             clear_pending();
             return;
         }
@@ -1110,13 +1125,25 @@ struct Tracer {
             atomic_addu(&c->count, 1ull);
         }
     }
+    // Adds to slice p of a facet's profile: in LDS for the profiles and slots
+    // kept there (TraceParams::prof_slots), else in memory.
+    MFG_IN void slice(const DPhys& ph, int slot, size_t p, bool count, double s1, double sv, bool sums) {
+        if (ph.prof_hot >= 0 && (uint32_t)slot < P.prof_slots) {
+            double* s = profs + 3u * (((uint32_t)ph.prof_hot * P.prof_slots + (uint32_t)slot) * MFG_PROFILE_SIZE + (uint32_t)p);
+            if (count) atomic_addd(s, w());
+            if (sums) { atomic_addd(s + 1, sv); atomic_addd(s + 2, s1); }
+            return;
+        }
+        mfg_profile_slice* s = P.prof + vc().prof_base + (size_t)slot * vc().n_prof + (size_t)ph.prof_off + p;
+        if (count) atomic_addd(&s->count_equiv, w());
+        if (sums) { atomic_addd(&s->sum_v_ort, sv); atomic_addd(&s->sum_1_per_ort_velocity, s1); }
+    }
     // ProfileFacet (Particle.cpp:1025-1085)
     MFG_IN void profile(const HitRegs& H, int32_t f, int m, bool count, double vf, double of) {
         if (!(H.flags & FF_PROFILE)) return;
         const DPhys& ph = P.phys[f];
         int pt = ph.profile_type;
         double a = ort(H);
-        mfg_profile_slice* base = P.prof + vc().prof_base + (size_t)ph.prof_off;
         if (count && pt == MFG_PROFILE_ANGULAR) {
             double th = acos(fmin(1.0, a));
             long p = (long)(th / (kPi / 2) * (double)MFG_PROFILE_SIZE);
@@ -1124,7 +1151,7 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                atomic_addd(&base[(size_t)slot * vc().n_prof + p].count_equiv, ori);
+                slice(ph, slot, (size_t)p, true, 0.0, 0.0, false);
             }
         } else if (pt == MFG_PROFILE_U || pt == MFG_PROFILE_V) {
             double c = pt == MFG_PROFILE_U ? hu : hv;
@@ -1136,10 +1163,7 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                mfg_profile_slice* s = &base[(size_t)slot * vc().n_prof + p];
-                if (count) atomic_addd(&s->count_equiv, ori);
-                atomic_addd(&s->sum_1_per_ort_velocity, ori * vf / ov);
-                atomic_addd(&s->sum_v_ort, ori * of * vc().c_factor * ov);
+                slice(ph, slot, p, count, w() * vf / ov, w() * of * vc().c_factor * ov, true);
             }
         } else if (count && (pt == MFG_PROFILE_VELOCITY || pt == MFG_PROFILE_ORT_VELOCITY || pt == MFG_PROFILE_TAN_VELOCITY)) {
             double d = pt == MFG_PROFILE_VELOCITY ? 1.0 : (pt == MFG_PROFILE_ORT_VELOCITY ? a : sqrt(fmax(0.0, 1 - a * a)));
@@ -1149,7 +1173,7 @@ struct Tracer {
             for (int k = 0; k < 2; ++k) {
                 int slot = k == 0 ? 0 : m;
                 if (k == 1 && m <= 0) break;
-                atomic_addd(&base[(size_t)slot * vc().n_prof + p].count_equiv, ori);
+                slice(ph, slot, (size_t)p, true, 0.0, 0.0, false);
             }
         }
     }
@@ -1389,12 +1413,20 @@ struct Tracer {
                     atomic_addd(fo + 6, mom.x); atomic_addd(fo + 7, mom.y); atomic_addd(fo + 8, mom.z);
                 }
             }
-            if (m > 0) {
+            if (m > 0 && H.hot >= 0 && (uint32_t)m < P.hot_slots) {
+                double* h = hot + 8 * ((uint32_t)H.hot * P.hot_slots + (uint32_t)m);
+                atomicAdd(reinterpret_cast<unsigned long long*>(h + 2), 1ull);
+                atomic_addd(h + 4, 2.0 / ov);
+                atomic_addd(h + 5, vc().c_factor * ov);
+                atomic_addd(h + 6, 1.0 / vel);
+            } else if (m > 0) {
                 mfg_facet_counters* c = fc(src, m);
                 atomic_addu(&c->nb_desorbed, 1ull);
                 atomic_addd(&c->sum_1_per_ort_velocity, 2.0 / ov);
                 atomic_addd(&c->sum_v_ort, vc().c_factor * ov);
                 atomic_addd(&c->sum_1_per_velocity, 1.0 / vel);
+            }
+            if (m > 0) {
                 if constexpr ((FEAT & FEAT_FORCE) != 0) {
                     if (vc().enable_force) {
                         double* fo = P.force + vc().force_base + ((size_t)m * vc().n_facets + (uint32_t)local(src)) * 9;
@@ -1659,9 +1691,10 @@ struct Tracer {
             if constexpr (CLOCKED) ++nb_events;
             root = find_root();
             walk_load(W, lane, pos, dir, last_hit, 1e300);
+            if constexpr ((FEAT & FEAT_TRANSPARENT) != 0) pass->n[lane] = 0;
         }
         const CoinState cs{rng.k0, rng.k1, rng.p0, rng.p1, nb_events, time, var};
-        walk<(FEAT & FEAT_TRANSPARENT) != 0>(P, W, lnodes, lane, alive, root, cs);
+        walk<(FEAT & FEAT_TRANSPARENT) != 0>(P, W, pass, lnodes, lane, alive, root, cs);
         // the ray is read back from its slot: not held in registers meanwhile
         const double2 a = W.p01[lane], b = W.p2d0[lane], c = W.d12[lane];
         pos = mk(a.x, a.y, b.x);
@@ -1690,43 +1723,68 @@ struct Tracer {
         }
         if constexpr (TR) {
             if (vc().flags & FEAT_TRANSPARENT) {
-                // second walk: every transparent pass closer than `travel`
-                const int32_t root = find_root();
-                const LaneStack S{W.nodes + lane, MFG_LANE_STACK, P.stack_total, spill};
-                Ray32 r = make_ray32(pos, dir);
-                float tbf = widen(travel);
-                uint32_t sp = 0;
-                int32_t node = root;
-                double save_u = hu, save_v = hv;
-                for (;;) {
-                    const NodeRegs nd = load_node_at(P.nodes, lnodes, P.lds_nodes, node);
-                    uint32_t msk = node_hits(nd, r, tbf);
-                    while (msk) {
-                        uint32_t c = (uint32_t)__builtin_ctz(msk);
-                        msk &= msk - 1u;
-                        if (node_inner(nd) & (1u << c)) {
-                            S.push(sp, node_inner_child(nd, c));
-                            continue;
-                        }
-                        uint32_t first, cnt;
-                        node_leaf_child(nd, c, first, cnt);
-                        for (uint32_t kk = 0; kk < cnt; ++kk) {
-                            double t, u, v;
-                            int32_t f;
-                            uint32_t fl;
-                            bool hit = leaf_test(P.leaves + first + kk, P.leaf_uv + first + kk, P.poly, pos, dir, last_hit,
-                                                 t, u, v, f, fl);
-                            if (!hit || (fl & FF_OPAQUE)) continue;
-                            if (!(t < travel)) continue;
-                            double op = (fl & FF_TD_OPACITY) ? td_opacity(P, var, f, time) : (double)P.phys[f].opacity;
-                            bool hard = op >= 1.0 || (op > 0.0 && rng.coin(nb_events, (uint32_t)local(f)) < op);
-                            if (hard) continue;
-                            hu = u; hv = v;
-                            transparent_pass(f, t);
-                        }
+                // every transparent pass closer than `travel`: the ones the
+                // walk met and noted (in record order, the walk's own order
+                // depending on the wave), or all of them from a second walk
+                // of this lane if there were more than it notes
+                const double save_u = hu, save_v = hv;
+                const uint32_t n_pass = pass->n[lane];
+                if (n_pass != 0 && n_pass <= MFG_PASSES) {
+                    uint32_t q[MFG_PASSES];
+#pragma unroll
+                    for (uint32_t k = 0; k < MFG_PASSES; ++k) q[k] = k < n_pass ? pass->rec[lane][k] : ~0u;
+#pragma unroll
+                    for (uint32_t i = 1; i < MFG_PASSES; ++i)
+#pragma unroll
+                        for (uint32_t k = 0; k + i < MFG_PASSES; ++k)
+                            if (q[k] > q[k + 1]) { const uint32_t x = q[k]; q[k] = q[k + 1]; q[k + 1] = x; }
+                    for (uint32_t k = 0; k < n_pass; ++k) {
+                        const uint32_t rec = k == 0 ? q[0] : k == 1 ? q[1] : k == 2 ? q[2] : q[3];
+                        double t, u, v;
+                        int32_t f;
+                        uint32_t fl;
+                        (void)leaf_test(P.leaves + rec, P.leaf_uv + rec, P.poly, pos, dir, last_hit, t, u, v, f, fl);
+                        if (!(t < travel)) continue;
+                        hu = u; hv = v;
+                        transparent_pass(f, t);
                     }
-                    if (sp == 0) break;
-                    node = S.pop(sp);
+                } else if (n_pass != 0) {
+                    const int32_t root = find_root();
+                    const LaneStack S{W.nodes + lane, MFG_LANE_STACK, P.stack_total, spill};
+                    Ray32 r = make_ray32(pos, dir);
+                    float tbf = widen(travel);
+                    uint32_t sp = 0;
+                    int32_t node = root;
+                    for (;;) {
+                        const NodeRegs nd = load_node_at(P.nodes, lnodes, P.lds_nodes, node);
+                        uint32_t msk = node_hits(nd, r, tbf);
+                        while (msk) {
+                            uint32_t c = (uint32_t)__builtin_ctz(msk);
+                            msk &= msk - 1u;
+                            if (node_inner(nd) & (1u << c)) {
+                                S.push(sp, node_inner_child(nd, c));
+                                continue;
+                            }
+                            uint32_t first, cnt;
+                            node_leaf_child(nd, c, first, cnt);
+                            for (uint32_t kk = 0; kk < cnt; ++kk) {
+                                double t, u, v;
+                                int32_t f;
+                                uint32_t fl;
+                                bool hit = leaf_test(P.leaves + first + kk, P.leaf_uv + first + kk, P.poly, pos, dir, last_hit,
+                                                     t, u, v, f, fl);
+                                if (!hit || (fl & FF_OPAQUE)) continue;
+                                if (!(t < travel)) continue;
+                                double op = (fl & FF_TD_OPACITY) ? td_opacity(P, var, f, time) : (double)P.phys[f].opacity;
+                                bool hard = op >= 1.0 || (op > 0.0 && rng.coin(nb_events, (uint32_t)local(f)) < op);
+                                if (hard) continue;
+                                hu = u; hv = v;
+                                transparent_pass(f, t);
+                            }
+                        }
+                        if (sp == 0) break;
+                        node = S.pop(sp);
+                    }
                 }
                 hu = save_u; hv = save_v;
             }
@@ -1800,19 +1858,31 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     const size_t gl = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     int32_t* spill = P.stack_spill ? P.stack_spill + gl * (P.stack_total - MFG_LANE_STACK) : nullptr;
-    Tracer<FEAT, ONE> T(P, W, spill);
-    // hot-facet counters after the waves' walk areas
-    double* hot = reinterpret_cast<double*>(lds_base + (blockDim.x >> 6) * sizeof(WaveLds));
-    for (uint32_t i = threadIdx.x; i < 8u * P.n_hot; i += blockDim.x) hot[i] = 0.0;
+    // after the waves' walk areas: their pass areas (transparent models),
+    // then the hot-facet counters
+    unsigned char* lds_next = lds_base + (blockDim.x >> 6) * sizeof(WaveLds);
+    PassLds* pass = nullptr;
+    if constexpr ((FEAT & FEAT_TRANSPARENT) != 0) {
+        pass = reinterpret_cast<PassLds*>(lds_next) + (threadIdx.x >> 6);
+        lds_next += (blockDim.x >> 6) * sizeof(PassLds);
+    }
+    Tracer<FEAT, ONE> T(P, W, pass, spill);
+    double* hot = reinterpret_cast<double*>(lds_next);
+    const uint32_t hot_words = 8u * P.n_hot * P.hot_slots;
+    for (uint32_t i = threadIdx.x; i < hot_words; i += blockDim.x) hot[i] = 0.0;
     // then the block's copy of the top of the tree (128 B per node; the
     // offsets above are multiples of 64 B)
-    uint4* lnodes = reinterpret_cast<uint4*>(hot + 8u * P.n_hot);
+    double* profs = hot + hot_words;
+    const uint32_t prof_words = 3u * MFG_PROFILE_SIZE * P.n_prof_hot * P.prof_slots;
+    for (uint32_t i = threadIdx.x; i < prof_words; i += blockDim.x) profs[i] = 0.0;
+    uint4* lnodes = reinterpret_cast<uint4*>(profs + prof_words);
     {
         const uint4* g = reinterpret_cast<const uint4*>(P.nodes);
         for (uint32_t i = threadIdx.x; i < 8u * P.lds_nodes; i += blockDim.x) lnodes[i] = g[i];
     }
     __syncthreads();
     T.hot = hot;
+    T.profs = profs;
     T.lnodes = lnodes;
     if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
         T.adj_cnt = P.adj_counts + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * P.adj_groups;
@@ -1914,7 +1984,7 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                 if (grp && lane == sl) {
                     const int32_t hi = P.hits[src].hot_idx;
                     if (hi >= 0) {
-                        double* h = hot + 8 * hi;
+                        double* h = hot + 8 * ((uint32_t)hi * P.hot_slots);
                         atomicAdd(reinterpret_cast<unsigned long long*>(h + 2), (unsigned long long)__popcll(gmask));
                         atomic_addd(h + 4, s1);
                         atomic_addd(h + 5, s2);
@@ -2006,16 +2076,23 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     // every wave of the block has left the loop: add the block's hot-facet
     // sums to the global records
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < 8u * P.n_hot; i += blockDim.x) {
-        const uint32_t k = i >> 3, fld = i & 7u;
+    for (uint32_t i = threadIdx.x; i < hot_words; i += blockDim.x) {
+        const uint32_t k = (i >> 3) / P.hot_slots, slot = (i >> 3) % P.hot_slots, fld = i & 7u;
         if (fld == 7u) continue;
-        double* g = reinterpret_cast<double*>(P.fc + P.hot_fc[k]) + fld;
+        double* g = reinterpret_cast<double*>(P.fc + P.hot_fc[k] + (size_t)slot * P.one.n_facets) + fld;
         if (fld == 0u || fld == 2u) {
             unsigned long long v = *reinterpret_cast<unsigned long long*>(hot + i);
             if (v) atomic_addu(reinterpret_cast<unsigned long long*>(g), v);
         } else if (hot[i] != 0.0) {
             atomic_addd(g, hot[i]);
         }
+    }
+    // and its profile slices
+    for (uint32_t i = threadIdx.x; i < prof_words; i += blockDim.x) {
+        if (profs[i] == 0.0) continue;
+        const uint32_t per = 3u * MFG_PROFILE_SIZE, k = i / per, slot = k % P.prof_slots;
+        double* g = reinterpret_cast<double*>(P.prof + P.hot_prof[k / P.prof_slots] + (size_t)slot * P.one.n_prof);
+        atomic_addd(g + i % per, profs[i]);
     }
 }
 
@@ -2093,7 +2170,7 @@ __global__ void __launch_bounds__(256) k_intersect(IsectParams p) {
         if (skip >= 0) skip += (int32_t)p.facet_base;
         walk_load(W, lane, P, D, skip, 1e300);
     }
-    walk<false>(tp, W, nullptr, lane, live, p.root, CoinState{});
+    walk<false>(tp, W, nullptr, nullptr, lane, live, p.root, CoinState{});
     if (!live) return;
     const int32_t f = W.facet[lane];
     const double t = __longlong_as_double((long long)W.t[lane]);
@@ -2128,6 +2205,10 @@ constexpr uint32_t kFull = FEAT_ALL;
 constexpr uint32_t kFullAdj = FEAT_ALL | FEAT_ADJOINT;
 
 }  // namespace
+
+size_t mfg_wave_lds(uint32_t model_features) {
+    return sizeof(WaveLds) + ((mfg_trace_kernel_features(model_features) & FEAT_TRANSPARENT) ? sizeof(PassLds) : 0);
+}
 
 uint32_t mfg_trace_kernel_features(uint32_t model_features) {
     const uint32_t rest = model_features & FEAT_ALL & ~FEAT_LOWFLUX;
@@ -2204,7 +2285,7 @@ int mfg_trace_occupancy(uint32_t features, bool single, int waves, int block, si
 }
 
 int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int waves, int grid, int block, void* stream) {
-    size_t lds = (size_t)(block / 64) * sizeof(WaveLds) + (size_t)p.n_hot * 8 * sizeof(double) +
+    size_t lds = (size_t)(block / 64) * mfg_wave_lds(features) + ((size_t)p.n_hot * p.hot_slots * 8 + (size_t)p.n_prof_hot * p.prof_slots * 3 * MFG_PROFILE_SIZE) * sizeof(double) +
                  (size_t)p.lds_nodes * sizeof(BvhNode);
     const uint32_t f = mfg_trace_kernel_features(features);
     TraceKernel k = kernel_for(f, single, waves, block);

@@ -90,3 +90,44 @@ def test_parked_lean_particles_resume_in_the_full_kernel(sim):
         assert np.allclose(one.facets[fld], two.facets[fld], rtol=1e-9, atol=0)
     assert one.glob[0]["nb_mc_hit"] == two.glob[0]["nb_mc_hit"]
     assert np.isclose(one.glob[0]["dist_traveled_total"], two.glob[0]["dist_traveled_total"], rtol=1e-12)
+
+
+@pytest.mark.parametrize("moments,sheets", [(3, 1), (150, 1), (12, 7), (0, 6)])
+def test_moment_and_profile_sums_kept_in_lds(sim, moments, sheets):
+    """Counters and profiles of hot facets with all, some or one of their
+    slots summed in LDS, more profiles than are kept there (more than 4), and
+    rays that cross more transparent sheets than the walk notes (more than
+    4), against the oracle on the same seed."""
+    from molflow_sources_amd import _abi as A
+    m = geometry.time_dependent_tube("0.1e-3,0.2e-3,%g" % (0.2e-3 * (max(moments, 1) - 0.4)), window=0.2e-3)
+    if moments == 0:
+        m.moments = []
+        m.settings.calc_constant_flow = 1
+        m.facets["outgassing_param"][0] = -1
+    V, F = [m.vertices], [m.facets]
+    nv = len(m.vertices)
+    for k in range(sheets - 1):
+        z = 1.0 + 8.0 * k / max(1, sheets - 2)
+        V.append(np.array([[-0.6, -0.6, z], [0.6, -0.6, z], [0.6, 0.6, z], [-0.6, 0.6, z]]))
+        m.polygons.append([nv, nv + 1, nv + 2, nv + 3])
+        nv += 4
+        f = default_facets(1)
+        f["opacity"], f["is_2sided"], f["profile_type"] = 0.25 * (k % 2), 1, A.PROFILE_V
+        F.append(f)
+    m.vertices, m.facets = np.concatenate(V), np.concatenate(F)
+    n = 30_000
+    sim.load(m)
+    sim.rebuild_accel()
+    sim.reset(seed=11)
+    sim.run(n)
+    t, c = sim.read(), CpuModel(m).run(n, seed=11)
+    assert t.n_slots == 1 + moments
+    assert t.desorbed == n
+    # a few long trajectories may part by FP64 rounding of the math library
+    for a, b in ((t.facets["nb_mc_hit"], c.facets["nb_mc_hit"]), (t.facets["nb_desorbed"], c.facets["nb_desorbed"])):
+        a, b = a.astype(np.int64), b.astype(np.int64)
+        assert np.abs(a - b).sum() <= 1e-3 * b.sum()
+    for a, b in [(t.facets[k], c.facets[k]) for k in ("nb_hit_equiv", "nb_abs_equiv", "sum_v_ort", "sum_1_per_ort_velocity")] + \
+                [(t.profiles[k], c.profiles[k]) for k in ("count_equiv", "sum_v_ort", "sum_1_per_ort_velocity")]:
+        assert b.sum() > 0
+        assert np.abs(a - b).sum() <= 2e-3 * b.sum()
