@@ -16,6 +16,12 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function",
          "-Wno-unused-variable", "-Wno-unused-but-set-variable"]
 SOURCES = ["mfg_trace.hip", "mfg_host.cpp"]
+# No machine LICM for the trace kernels: their persistent loop contains the
+# whole event, and hoisting the FP64 constants of sincos, pow, acos and log
+# out of it kept some 80 VGPRs live across the walk, which then spilled (336 B
+# of scratch a lane at 3 waves per SIMD, 0 without; the full kernel at 2
+# waves: 628 B and 44 B).
+SOURCE_FLAGS = {"mfg_trace.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def build(verbose: bool = False) -> str:
@@ -23,7 +29,7 @@ def build(verbose: bool = False) -> str:
     for src in SOURCES:
         obj = os.path.join(CSRC, src.rsplit(".", 1)[0] + ".o")
         lang = ["-x", "hip"] if src.endswith(".hip") else []
-        cmd = [HIPCC, *FLAGS, *lang, "-c", os.path.join(CSRC, src), "-o", obj]
+        cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), *lang, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd))
         subprocess.run(cmd, check=True)
