@@ -916,9 +916,10 @@ struct mfg_context {
         const uint32_t per = (uint32_t)(MFG_PROFILE_SIZE * sizeof(mfg_profile_slice)) * n_prof_hot;
         return std::max<uint32_t>(1, std::min<uint32_t>(dvars[0].n_slots, 12288 / per));
     }
-    // LDS of a block's hot counters and profiles
+    double maxwell_scale = 0.0;          // TraceParams::maxwell_scale
+    // LDS of a block's hot counters, profiles and Maxwell table
     size_t hot_bytes() const {
-        return hot.size() * hot_slots() * sizeof(mfg_facet_counters) +
+        return (maxwell_scale > 0.0 ? MFG_MAXWELL_LDS : 0) + hot.size() * hot_slots() * sizeof(mfg_facet_counters) +
                (size_t)n_prof_hot * prof_slots() * MFG_PROFILE_SIZE * sizeof(mfg_profile_slice);
     }
     DevBuf<uint64_t> hot_fc, hot_prof;
@@ -1143,6 +1144,12 @@ void upload_models(mfg_context* c) {
     }
     hipStream_t s = c->stream;
     c->h_phys = phys;
+    // one gas in all variants (a gas' CDF depends on its mass alone): the
+    // kernel's blocks keep that table in LDS
+    static_assert(kMaxwellPoints == MFG_MAXWELL_POINTS, "points of a Maxwell table");
+    c->maxwell_scale = (double)MFG_MAXWELL_GUIDE / c->models[0]->maxwell.back().y;
+    for (auto& M : c->models)
+        if (M->s.gas_mass != c->models[0]->s.gas_mass) c->maxwell_scale = 0.0;
     // default hot facets of each variant: its sources, absorbers and
     // transparent facets when there are only a few of them (the autotuner refines the choice from
     // measured counts)
@@ -1364,14 +1371,20 @@ void build_accel(mfg_context* c, int width, int leaf) {
     reset_graph(c);
 }
 
+// LDS is allocated in units of 1280 B on gfx950; the occupancy query does
+// not round to them, and a grid of blocks that do not all fit would run its
+// last ones after the first have ended.
+constexpr size_t kLdsGrain = 1280;
+
 // Nodes read from LDS: the top of the tree of a single-variant model, as
 // many as fit beside the waves' walk areas and the hot facets in a block's
 // share of the CU's LDS (all of it for a block of 768 or 1024 lanes, else a
 // 1 / waves part for every 256 lanes).
 uint32_t lds_node_count(const mfg_context* c, uint32_t feats, int block, int waves) {
     if (c->dvars.size() != 1) return 0;
-    const size_t share = block > 256 ? c->lds_per_block : c->lds_per_block * (size_t)block / 256 / (size_t)std::max(1, waves);
-    const size_t used = (size_t)(block / 64) * mfg_wave_lds(feats) + c->hot_bytes() + 256;
+    size_t share = block > 256 ? c->lds_per_block : c->lds_per_block * (size_t)block / 256 / (size_t)std::max(1, waves);
+    share = share / kLdsGrain * kLdsGrain;
+    const size_t used = (size_t)(block / 64) * mfg_wave_lds(feats) + c->hot_bytes();
     size_t n = share > used ? (share - used) / sizeof(BvhNode) : 0;
     if (block <= 256) n = std::min<size_t>(n, c->node_cache);
     return (uint32_t)std::min<size_t>(n, c->nodes.n);
@@ -1389,7 +1402,7 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     p.stack_total = c->stack_size;
     p.stack_spill = p.stack_total > MFG_LANE_STACK ? c->stack_spill.p : nullptr;
     p.src_cum = c->src_cum.p; p.src_facet = c->src_facet.p; p.og_cdf = c->og_cdf.p; p.am_src = c->am_src.p;
-    p.hot_fc = c->hot_fc.p; p.n_hot = (uint32_t)c->hot.size(); p.hot_slots = c->hot_slots();
+    p.hot_fc = c->hot_fc.p; p.n_hot = (uint32_t)c->hot.size(); p.hot_slots = c->hot_slots(); p.maxwell_scale = c->maxwell_scale;
     p.hot_prof = c->hot_prof.p; p.n_prof_hot = c->n_prof_hot; p.prof_slots = c->prof_slots();
     p.guides = c->guides.p; p.tab_x = c->tab_x.p; p.tab_y = c->tab_y.p; p.params = c->params.p; p.ids = c->ids.p;
     p.mom_start = c->mom_start.p; p.mom_end = c->mom_end.p;
@@ -1441,6 +1454,8 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
     if (per_cu == 0) {
         // fill every CU to its occupancy limit (persistent launch)
         int occ = mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block));
+        const size_t lds = (lds_bytes(block) + kLdsGrain - 1) / kLdsGrain * kLdsGrain;
+        occ = std::min(occ, (int)(c->lds_per_block / lds));
         per_cu = (uint32_t)std::max(1, occ);
     }
     grid = (int)(per_cu * (uint32_t)c->n_cu);

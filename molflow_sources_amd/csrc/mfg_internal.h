@@ -25,7 +25,9 @@
 #define MFG_WALK_LEAVES 256      // (ray, facet record) tasks waiting: below 64 plus one node's 8 leaves of 16
 #define MFG_LANE_STACK ((MFG_WALK_NODES + MFG_WALK_LEAVES) / 64)   // entries of a lane's own stack in the same LDS
 #define MFG_MAX_GROUPS 64
+#define MFG_MAXWELL_POINTS 100
 #define MFG_MAXWELL_GUIDE 128
+#define MFG_MAXWELL_LDS (16 * MFG_MAXWELL_POINTS + MFG_MAXWELL_GUIDE)
 #define MFG_MAX_HOT 32           // facets whose counters are privatised per block
 #define MFG_MAX_PROF_HOT 4       // profiles privatised per block
 
@@ -296,6 +298,8 @@ struct TraceParams {
     const int32_t* src_facet;
     const double* og_cdf;
     const uint32_t* guides;           // guide tables of the Maxwell CDFs
+    double maxwell_scale;             // > 0: all variants share one gas, whose CDF the blocks copy
+                                      // to LDS (guide entries per unit of probability)
     const double* tab_x;              // table pool (maxwell CDFs, params, IDs)
     const double* tab_y;
     const DTable* params;

@@ -69,6 +69,46 @@ struct Rng {
     }
 };
 
+// The draws of one wall event: what the particle's block has left and the
+// next block, so that the block function runs once per event for the whole
+// wave; called at each draw that finds its lane's block empty, it ran at
+// nearly every draw of every event for some lane (3 draws a bounce, 4 words
+// a block). Rng's own state is unchanged until done().
+struct EventDraws {
+    Rng& g;
+    uint32_t w0, w1, w2, w3, w4, w5, w6, w7, left;
+    __device__ __forceinline__ EventDraws(Rng& r) : g(r) {
+        philox10(g.p0, g.p1, g.blk, 0u, g.k0, g.k1, w4, w5, w6, w7);
+        // the next block's words follow the `avail` words left
+        const bool a1 = (g.avail & 1u) != 0, a2 = (g.avail & 2u) != 0, a4 = (g.avail & 4u) != 0;
+        w0 = g.avail ? g.b0 : w4;
+        w1 = g.avail > 1u ? g.b1 : (a1 ? w4 : w5);
+        w2 = g.avail > 2u ? g.b2 : (a2 ? w4 : a1 ? w5 : w6);
+        w3 = a4 ? g.b3 : (a2 ? (a1 ? w4 : w5) : a1 ? w6 : w7);
+        const uint32_t x4 = a4 ? w4 : (a2 ? (a1 ? w5 : w6) : w7);   // avail 1..4 (0: past the end)
+        const uint32_t x5 = a4 ? w5 : (a1 ? w6 : w7), x6 = a4 ? w6 : w7;
+        w4 = x4; w5 = x5; w6 = x6;
+        left = g.avail + 4u;
+    }
+    __device__ __forceinline__ double rnd() {
+        if (left == 0) {
+            // an event of more than 4 draws
+            ++g.blk;
+            philox10(g.p0, g.p1, g.blk, 0u, g.k0, g.k1, w0, w1, w2, w3);
+            left = 4;
+        }
+        const uint32_t r = w0;
+        w0 = w1; w1 = w2; w2 = w3; w3 = w4; w4 = w5; w5 = w6; w6 = w7;
+        --left;
+        return u2d(r);
+    }
+    __device__ __forceinline__ void done() {
+        g.b0 = w0; g.b1 = w1; g.b2 = w2; g.b3 = w3;
+        if (left >= 4u) g.avail = left - 4u;   // the next block untouched: drawn again later
+        else { g.avail = left; ++g.blk; }
+    }
+};
+
 // ------------------------------------------------------------------ math helpers
 struct d3 { double x, y, z; };
 __device__ __forceinline__ d3 mk(double x, double y, double z) { return {x, y, z}; }
@@ -146,6 +186,24 @@ __device__ double interp_x_guided(double y, XYRef t, const uint32_t* guide, uint
     double y0 = t.y[i], y1 = t.y[i + 1], x0 = t.x[i], x1 = t.x[i + 1];
     if (y1 == y0) return x0;
     return x0 + (y - y0) * (x1 - x0) / (y1 - y0);
+}
+
+// The same interval and value from the block's LDS copy of a Maxwell CDF:
+// (speed, cumulative) points and one byte per guide entry. The guide only
+// says where the search starts, so the scale K / last y may be rounded.
+struct MaxwellLds {
+    double2 p[MFG_MAXWELL_POINTS];
+    uint8_t guide[MFG_MAXWELL_GUIDE];
+};
+static_assert(sizeof(MaxwellLds) == MFG_MAXWELL_LDS, "MFG_MAXWELL_LDS is the size of MaxwellLds");
+__device__ __forceinline__ double maxwell_lds(const MaxwellLds* M, double y, double scale) {
+    constexpr uint32_t n = MFG_MAXWELL_POINTS;
+    uint32_t i = M->guide[(uint32_t)fmin((double)(MFG_MAXWELL_GUIDE - 1), y * scale)];
+    double2 a = M->p[i], b = M->p[i + 1];
+    while (i > 0 && a.y > y) { --i; b = a; a = M->p[i]; }
+    while (i + 1 < n - 1 && b.y <= y) { ++i; a = b; b = M->p[i + 1]; }
+    if (b.y == a.y) return a.x;
+    return a.x + (y - a.y) * (b.x - a.x) / (b.y - a.y);
 }
 
 __device__ __forceinline__ double interp_x(double y, XYRef t) {
@@ -838,6 +896,7 @@ struct Tracer {
     double* hot;                      // LDS table of the hot facets' slot-0 counters (8 words each)
     double* profs;                    // LDS slices of the profiles kept there
     const uint4* lnodes;              // LDS copy of the first P.lds_nodes BVH nodes
+    const MaxwellLds* maxwell;        // LDS copy of the Maxwell CDF (P.maxwell_scale > 0)
     // pending slot-0 facet counter update of this lane
     int32_t pend_f, pend_hot;
     uint32_t pend_hits;
@@ -855,6 +914,7 @@ struct Tracer {
         var = nullptr;
         hot = profs = nullptr;
         lnodes = nullptr;
+        maxwell = nullptr;
         ori = 1.0;
         time = gen_time = dist = hu = hv = 0.0;
         decay_t = scatter_path = 1e100;
@@ -1271,9 +1331,12 @@ struct Tracer {
         }
         (void)d; (void)v;
     }
-    MFG_IN double maxwell_speed(double sq) {
-        XYRef t{P.tab_x + vc().maxwell_base, P.tab_y + vc().maxwell_base, 100};
-        return interp_x_guided(rng.rnd(), t, P.guides + vc().maxwell_guide, MFG_MAXWELL_GUIDE) * sq;
+    template <typename G>
+    MFG_IN double maxwell_speed(G& g, double sq) {
+        const double r = g.rnd();
+        if (P.maxwell_scale > 0.0) return maxwell_lds(maxwell, r, P.maxwell_scale) * sq;
+        XYRef t{P.tab_x + vc().maxwell_base, P.tab_y + vc().maxwell_base, MFG_MAXWELL_POINTS};
+        return interp_x_guided(r, t, P.guides + vc().maxwell_guide, MFG_MAXWELL_GUIDE) * sq;
     }
     MFG_IN d3 emit(const HitRegs& H, const DPhys& ph, int type, double n_exp, bool reverse) {
         if (type == MFG_DES_UNIFORM) {
@@ -1345,7 +1408,7 @@ struct Tracer {
             }
         }
         gen_time = time;
-        if (vc().use_maxwell) vel = maxwell_speed(H.sqrt_temp);
+        if (vc().use_maxwell) vel = maxwell_speed(rng, H.sqrt_temp);
         else vel = 145.469 * sqrt(ph.temperature / vc().gas_mass);
         ori = 1.0;
         decay_t = 1e100;
@@ -1493,20 +1556,20 @@ struct Tracer {
         if (H.flags & FF_COUNT_DIR) direction(f, m);
     }
     // UpdateVelocity (Particle.cpp:1138-1163)
-    MFG_IN void update_velocity(const HitRegs& H, int32_t f) {
+    MFG_IN void update_velocity(EventDraws& g, const HitRegs& H, int32_t f) {
         double sq = H.sqrt_temp;
         if constexpr ((FEAT & FEAT_TDPARAM) != 0) { if (H.flags & FF_TD_TEMP) sq = sqrt(temperature(P.phys[f])); }
         if (H.flags & FF_FULL_ACC) {
-            vel = vc().use_maxwell ? maxwell_speed(sq) : 145.469 * sq / vc().gas_mass;
+            vel = vc().use_maxwell ? maxwell_speed(g, sq) : 145.469 * sq / vc().gas_mass;
         } else {
             double o2 = vel * vel, n2;
-            if (vc().use_maxwell) { double vv = maxwell_speed(sq); n2 = vv * vv; }
+            if (vc().use_maxwell) { double vv = maxwell_speed(g, sq); n2 = vv * vv; }
             else n2 = 29369.939 * (temperature(P.phys[f]) / vc().gas_mass);
             vel = sqrt(o2 + (n2 - o2) * P.hits[f].accomodation);
         }
     }
     // PerformBounce (Particle.cpp:691-838)
-    MFG_IN void bounce(const HitRegs& H, int32_t f) {
+    MFG_IN void bounce(EventDraws& g, const HitRegs& H, int32_t f) {
         add_hit();
         if constexpr ((FEAT & FEAT_TELEPORT) != 0) {
             if (H.flags & FF_LINK) {
@@ -1535,29 +1598,29 @@ struct Tracer {
         log_hit(H, f);
         profile(H, f, m, true, 1.0, 1.0);
         angle_map(H, f);
-        update_velocity(H, f);
+        update_velocity(g, H, f);
         int m_out = m;
         if constexpr ((FEAT & FEAT_SOJOURN) != 0) {
             if (H.flags & FF_SOJOURN) {
                 const DPhys& ph = P.phys[f];
                 double A = exp(-ph.sojourn_e / (8.31 * temperature(ph)));
-                time += -log(rng.rnd()) / (A * ph.sojourn_freq);
+                time += -log(g.rnd()) / (A * ph.sojourn_freq);
                 m_out = moment(time);
             }
         }
         if (H.flags & FF_DIFFUSE) {
-            double a = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
+            double a = g.rnd(); double phv = g.rnd() * 2.0 * kPi;
             dir = polar_to_cart(H, sqrt(a), sqrt(1 - a), phv, revert);
         } else {
             const DHit& C = P.hits[f];
-            double rt = rng.rnd();
+            double rt = g.rnd();
             if (rt < C.diffuse) {
-                double a = rng.rnd(); double phv = rng.rnd() * 2.0 * kPi;
+                double a = g.rnd(); double phv = g.rnd() * 2.0 * kPi;
                 dir = polar_to_cart(H, sqrt(a), sqrt(1 - a), phv, revert);
             } else if (rt < C.diffuse + C.specular) {
                 dir = sub(dir, scl(2.0 * dot(dir, H.N), H.N));
             } else {
-                double c = pow(rng.rnd(), 1.0 / (P.phys[f].cos_exp + 1.0)); double phv = rng.rnd() * 2.0 * kPi;
+                double c = pow(g.rnd(), 1.0 / (P.phys[f].cos_exp + 1.0)); double phv = g.rnd() * 2.0 * kPi;
                 dir = polar_to_cart(H, c, sqrt(1 - c * c), phv, revert);
             }
         }
@@ -1804,11 +1867,12 @@ struct Tracer {
             // absorption, or the weight's absorbed part (low flux), then the
             // bounce of what is left
             const double s = sticking(H, f);
+            EventDraws g(rng);
             bool rec, go, lowflux = false;
             double w0 = 1.0;
             if constexpr (WEIGHTED) { lowflux = vc().low_flux != 0; w0 = ori; }
             if (!lowflux) {
-                rec = s == 1.0 || (s > 0.0 && rng.rnd() < s);
+                rec = s == 1.0 || (s > 0.0 && g.rnd() < s);
                 go = !rec;
             } else {
                 rec = s > 0.0;
@@ -1827,8 +1891,9 @@ struct Tracer {
                     }
                 }
             }
-            if (go) bounce(H, f);
+            if (go) bounce(g, H, f);
             else trace(f, 2);
+            g.done();
             return go;
         }
         if (ev == 1 || ev == 2) {
@@ -1875,7 +1940,15 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     double* profs = hot + hot_words;
     const uint32_t prof_words = 3u * MFG_PROFILE_SIZE * P.n_prof_hot * P.prof_slots;
     for (uint32_t i = threadIdx.x; i < prof_words; i += blockDim.x) profs[i] = 0.0;
-    uint4* lnodes = reinterpret_cast<uint4*>(profs + prof_words);
+    MaxwellLds* maxwell = reinterpret_cast<MaxwellLds*>(profs + prof_words);
+    if (P.maxwell_scale > 0.0) {
+        const DVariant& v = ONE ? P.one : P.variants[0];
+        for (uint32_t i = threadIdx.x; i < MFG_MAXWELL_POINTS; i += blockDim.x)
+            maxwell->p[i] = make_double2(P.tab_x[v.maxwell_base + i], P.tab_y[v.maxwell_base + i]);
+        for (uint32_t i = threadIdx.x; i < MFG_MAXWELL_GUIDE; i += blockDim.x)
+            maxwell->guide[i] = (uint8_t)P.guides[v.maxwell_guide + i];
+    }
+    uint4* lnodes = reinterpret_cast<uint4*>(maxwell + (P.maxwell_scale > 0.0 ? 1 : 0));
     {
         const uint4* g = reinterpret_cast<const uint4*>(P.nodes);
         for (uint32_t i = threadIdx.x; i < 8u * P.lds_nodes; i += blockDim.x) lnodes[i] = g[i];
@@ -1883,6 +1956,7 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     __syncthreads();
     T.hot = hot;
     T.profs = profs;
+    T.maxwell = maxwell;
     T.lnodes = lnodes;
     if constexpr ((FEAT & FEAT_ADJOINT) != 0) {
         T.adj_cnt = P.adj_counts + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * P.adj_groups;
@@ -2286,7 +2360,7 @@ int mfg_trace_occupancy(uint32_t features, bool single, int waves, int block, si
 
 int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int waves, int grid, int block, void* stream) {
     size_t lds = (size_t)(block / 64) * mfg_wave_lds(features) + ((size_t)p.n_hot * p.hot_slots * 8 + (size_t)p.n_prof_hot * p.prof_slots * 3 * MFG_PROFILE_SIZE) * sizeof(double) +
-                 (size_t)p.lds_nodes * sizeof(BvhNode);
+                 (p.maxwell_scale > 0.0 ? sizeof(MaxwellLds) : 0) + (size_t)p.lds_nodes * sizeof(BvhNode);
     const uint32_t f = mfg_trace_kernel_features(features);
     TraceKernel k = kernel_for(f, single, waves, block);
     if (!k) return -1;
