@@ -1425,9 +1425,14 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     return p;
 }
 
+// Waves per SIMD without a choice by the caller or the autotuner. The lean
+// kernel runs 3 without scratch. The weighted ones spill at 3 (100 B a lane),
+// and their runs are mostly long thin tails: 2 waves took 2e4 low-flux
+// particles from 97 to 78 ms and the adjoint from 80 to 65. The full kernel
+// fits 2; with the adjoint it takes 1.
 int default_waves(uint32_t feats) {
     uint32_t k = mfg_trace_kernel_features(feats);
-    if ((k & FEAT_ALL & ~FEAT_LOWFLUX) == 0) return 3;   // lean and low-flux sets
+    if ((k & FEAT_ALL & ~(uint32_t)FEAT_LOWFLUX) == 0) return (k & FEAT_LOWFLUX) ? 2 : 3;
     return (k & FEAT_ADJOINT) ? 1 : 2;
 }
 
