@@ -23,6 +23,7 @@
 #define MFG_WALK_NODES 512       // (ray, node) tasks of one wave's walk
 #define MFG_WALK_RESERVE 72      // of these for the depth-first tail: width - 1 entries a level, + width
 #define MFG_WALK_LEAVES 256      // (ray, facet record) tasks waiting: below 64 plus one node's 8 leaves of 16
+static_assert(MFG_WALK_LEAVES >= 63 + 64 * 3, "a step of 8 nodes with leaves of 3 facets fits the list");
 #define MFG_LANE_STACK ((MFG_WALK_NODES + MFG_WALK_LEAVES) / 64)   // entries of a lane's own stack in the same LDS
 #define MFG_MAX_GROUPS 64
 #define MFG_MAXWELL_POINTS 100
@@ -291,6 +292,7 @@ struct TraceParams {
     const uint64_t* var_prefix;       // n_variants+1 prefix of this run's desorptions
     uint32_t n_variants;
     uint32_t task_bits;               // bits of a walk task's node or record index (the rest: its ray)
+    uint32_t child_lanes;             // 1: leaves so small (at most 3 facets) that 8 nodes' facets fit the list
     uint32_t lane_quota;              // lanes of a wave that take particles
     uint32_t stack_total;             // entries a lane's own walk may need; the ones past MFG_LANE_STACK
     int32_t* stack_spill;             // live in this per-lane global area (lane-major)
@@ -381,7 +383,7 @@ struct IsectParams {
     const LeafFacet* leaves;
     const LeafUV* leaf_uv;
     int32_t root;
-    uint32_t task_bits;
+    uint32_t task_bits, child_lanes;
     uint32_t rays_per_wave;
     uint64_t n;
     const double* origins;

@@ -354,7 +354,7 @@ struct Ray32 { float ox, oy, oz, ix, iy, iz; };
 __device__ __forceinline__ float safe_inv(double d) {
     float f = (float)d;
     if (fabsf(f) < 1e-30f) f = (f < 0.0f) ? -1e-30f : 1e-30f;
-    return 1.0f / f;
+    return __builtin_amdgcn_rcpf(f);   // within 1 ulp, as the boxes' padding allows
 }
 
 __device__ __forceinline__ Ray32 make_ray32(d3 P, d3 D) {
@@ -663,6 +663,35 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
     return v;
 }
 
+// One child of a node against a ray: the test of node_hits for slot c alone,
+// from the node's header and that slot's six plane steps.
+struct ChildRegs {
+    uint4 c0, c1;
+    uint16_t lx, ly, lz, hx, hy, hz;
+};
+template <typename Q>
+__device__ __forceinline__ ChildRegs load_child(const Q* nd, uint32_t c) {
+    const uint4* q = reinterpret_cast<const uint4*>(nd);
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(nd) + 16 + c;
+    return {q[0], q[1], h[0], h[8], h[16], h[24], h[32], h[40]};
+}
+__device__ __forceinline__ float half_bits(uint16_t v) { return (float)__builtin_bit_cast(_Float16, v); }
+__device__ __forceinline__ bool child_hit(const ChildRegs& n, const Ray32& r, float tmax) {
+    const uint32_t ew = n.c0.w;
+    const float ax = exp2i((int)(int8_t)(ew & 0xffu)) * r.ix, ay = exp2i((int)(int8_t)((ew >> 8) & 0xffu)) * r.iy;
+    const float az = exp2i((int)(int8_t)((ew >> 16) & 0xffu)) * r.iz;
+    const float bx = (__uint_as_float(n.c0.x) - r.ox) * r.ix, by = (__uint_as_float(n.c0.y) - r.oy) * r.iy;
+    const float bz = (__uint_as_float(n.c0.z) - r.oz) * r.iz;
+    const float x0 = fmaf(half_bits(n.lx), ax, bx), x1 = fmaf(half_bits(n.hx), ax, bx);
+    const float y0 = fmaf(half_bits(n.ly), ay, by), y1 = fmaf(half_bits(n.hy), ay, by);
+    const float z0 = fmaf(half_bits(n.lz), az, bz), z1 = fmaf(half_bits(n.hz), az, bz);
+    // low planes first along +axis rays; a slot without a child is masked by the caller
+    const bool px = r.ix >= 0.0f, py = r.iy >= 0.0f, pz = r.iz >= 0.0f;
+    const float a = fmaxf(fmaxf(px ? x0 : x1, py ? y0 : y1), fmaxf(pz ? z0 : z1, 0.0f));
+    const float b = fminf(fminf(px ? x1 : x0, py ? y1 : y0), fminf(pz ? z1 : z0, tmax));
+    return a <= b;
+}
+
 // What the opacity coin of a ray needs from the lane that owns it.
 struct CoinState {
     uint32_t k0, k1, p0, p1, event;
@@ -691,6 +720,11 @@ struct CoinState {
 // to the lower facet id, so it does not depend on the order or the lanes
 // the tests run on.
 //
+// With at most 8 tasks on the stack (a wave with few rays: a run's tail, or
+// a small run) a node step gives each of them 8 lanes, one for each child:
+// the serial chain of 8 box tests and the loops that push the children
+// shrink to one test and one store a lane.
+//
 // Bounds. A node step commits the tasks of its first lanes only, as many as
 // leave the stack below its capacity less a reserve and the list within
 // its capacity; the other tasks stay where they are. Lane 0 (the topmost
@@ -711,7 +745,41 @@ __device__ void walk(const TraceParams& P, WaveLds& W, PassLds* pass, const uint
     }
     wave_sync();
     while (top + waiting != 0) {
-        if (waiting < 64u && top != 0) {
+        if (top != 0 && top <= 8u && waiting < 64u && P.child_lanes) {
+            const uint32_t c = lane & 7u, below = (1u << c) - 1u;
+            const bool on = (lane >> 3) < top;
+            uint32_t tag = 0, kid = 0, cnt = 0;
+            bool inner = false, leaf = false;
+            if (on) {
+                const uint32_t w = W.nodes[top - 1u - (lane >> 3)], ray = w >> bits, node = w & low;
+                tag = w & ~low;
+                ChildRegs nd;
+                if (node < P.lds_nodes) nd = load_child(lnodes + (size_t)node * 8, c);
+                else nd = load_child(P.nodes + node, c);
+                const float4 a = W.ra[ray], b = W.rb[ray];
+                const uint32_t im = nd.c1.w & 0xffu, lm = nd.c0.w >> 24;
+                if (child_hit(nd, Ray32{a.x, a.y, a.z, b.x, b.y, b.z}, a.w)) {
+                    inner = ((im >> c) & 1u) != 0;
+                    leaf = ((lm >> c) & 1u) != 0;
+                }
+                if (inner) kid = nd.c1.x + (uint32_t)__popc(im & below);
+                if (leaf) {
+                    kid = nd.c1.y + (uint32_t)__popc(lm & below) + nibble_sum(nd.c1.z & ((1u << (4u * c)) - 1u));
+                    cnt = ((nd.c1.z >> (4u * c)) & 15u) + 1u;
+                }
+            }
+            const uint64_t m = __ballot(inner);
+            wave_sync();
+            if (inner) W.nodes[mbcnt(m)] = tag | kid;
+            top = (uint32_t)__popcll(m);
+            for (uint32_t k = 0;; ++k) {
+                const uint64_t ml = __ballot(cnt > k);
+                if (ml == 0) break;
+                if (cnt > k) W.leaves[waiting + mbcnt(ml)] = tag | (kid + k);
+                waiting += (uint32_t)__popcll(ml);
+            }
+            wave_sync();
+        } else if (waiting < 64u && top != 0) {
             const bool on = lane < top;
             uint32_t tag = 0, inner = 0, im = 0, lm = 0, cw = 0, own = 0;
             int32_t node_base = 0;
@@ -887,7 +955,7 @@ struct Tracer {
     // the two path sums are one
     uint32_t acc_hits, acc_des, acc_absorbed;
     double acc_hit_equiv, acc_abs_equiv, acc_dist_total, acc_dist_full;
-    uint32_t acc_leak, acc_decay;
+    uint32_t acc_decay;
     uint32_t tr_n;
     uint32_t* adj_cnt;
     uint32_t seg_n;                   // adjoint: target scores since the last survived sticky collision
@@ -905,13 +973,13 @@ struct Tracer {
     MFG_IN Tracer(const TraceParams& p, WaveLds& w, PassLds* pl, int32_t* sp) : P(p), W(w), pass(pl), spill(sp) {
         acc_hits = acc_des = acc_absorbed = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
-        acc_leak = acc_decay = 0;
+        acc_decay = 0;
         tr_n = 0;
         adj_cnt = nullptr;
         seg_n = 0;
         seg_t = nullptr;
         seg_x = nullptr;
-        var = nullptr;
+        var = ONE ? p.variants : nullptr;
         hot = profs = nullptr;
         lnodes = nullptr;
         maxwell = nullptr;
@@ -1733,11 +1801,10 @@ struct Tracer {
         if (acc_des) atomic_addu(&gl->nb_desorbed, acc_des);
         if (hit_equiv() != 0.0) atomic_addd(&gl->nb_hit_equiv, hit_equiv());
         if (abs_equiv() != 0.0) atomic_addd(&gl->nb_abs_equiv, abs_equiv());
-        if (acc_leak) atomic_addu(&gl->nb_leak, acc_leak);
         if (acc_dist_total != 0.0) atomic_addd(&gl->dist_total, acc_dist_total);
         if (dist_full() != 0.0) atomic_addd(&gl->dist_full, dist_full());
         if (acc_decay) atomic_addu(&gl->nb_decayed, acc_decay);
-        acc_hits = acc_des = acc_absorbed = acc_leak = acc_decay = 0;
+        acc_hits = acc_des = acc_absorbed = acc_decay = 0;
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
     }
 
@@ -1768,7 +1835,7 @@ struct Tracer {
         constexpr bool TR = (FEAT & FEAT_TRANSPARENT) != 0;
         HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
         if (h.facet < 0) {  // leak
-            ++acc_leak;
+            atomic_addu(&P.glob[vc().glob_index].nb_leak, 1ull);   // rare: no register kept for it
             unsigned long long at = atomicAdd(P.leak_count, 1ull);
             if (at < P.leak_cap) {
                 double* L = P.leaks + at * 6;
@@ -2017,8 +2084,8 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                     if constexpr (!ONE) {
                         vi = r.variant;
                         if (T.var != P.variants + vi) T.flush_lane();
+                        T.var = P.variants + vi;
                     }
-                    T.var = P.variants + vi;
                     events_left = T.restore(r);
                     alive = true;
                 } else if (g < limit) {
@@ -2026,8 +2093,8 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                     if constexpr (!ONE) {
                         vi = find_variant(P.var_prefix, P.n_variants, d);
                         if (T.var != P.variants + vi) T.flush_lane();
+                        T.var = P.variants + vi;
                     }
-                    T.var = P.variants + vi;
                     ++T.acc_des;
                     uint64_t lp = (ONE ? d : d - P.var_prefix[vi]) + T.var->pid_base;
                     src = T.start(lp);
@@ -2132,14 +2199,13 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
         double he = wave_sum(T.hit_equiv()), ae = wave_sum(T.abs_equiv());
         double d1 = wave_sum(T.acc_dist_total), d2 = wave_sum(T.dist_full());
         unsigned long long hits = wave_sum_u(T.acc_hits), des = wave_sum_u(T.acc_des);
-        unsigned long long lk = wave_sum_u(T.acc_leak), dc = wave_sum_u(T.acc_decay);
+        unsigned long long dc = wave_sum_u(T.acc_decay);
         if (lane == 0) {
             DGlobal* gl = P.glob + P.one.glob_index;
             if (hits) atomic_addu(&gl->nb_mc_hit, hits);
             if (des) atomic_addu(&gl->nb_desorbed, des);
             if (he != 0.0) atomic_addd(&gl->nb_hit_equiv, he);
             if (ae != 0.0) atomic_addd(&gl->nb_abs_equiv, ae);
-            if (lk) atomic_addu(&gl->nb_leak, lk);
             if (d1 != 0.0) atomic_addd(&gl->dist_total, d1);
             if (d2 != 0.0) atomic_addd(&gl->dist_full, d2);
             if (dc) atomic_addu(&gl->nb_decayed, dc);
@@ -2233,6 +2299,7 @@ __global__ void __launch_bounds__(256) k_intersect(IsectParams p) {
     WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     TraceParams tp{};
     tp.poly = p.poly; tp.nodes = p.nodes; tp.leaves = p.leaves; tp.leaf_uv = p.leaf_uv; tp.task_bits = p.task_bits;
+    tp.child_lanes = p.child_lanes;
     const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint64_t i = wave * p.rays_per_wave + lane;
     const bool live = lane < p.rays_per_wave && i < p.n;
