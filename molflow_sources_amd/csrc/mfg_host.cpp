@@ -1628,6 +1628,8 @@ void add_tallies(mfg_context* c, uint32_t vi, const mfg_tally_view* o) {
         // to this read: every hit weighs 1
         if (!c->dvars[vi].low_flux)
             for (uint64_t i = 0; i < h.size(); ++i) h[i].nb_hit_equiv = (double)h[i].nb_mc_hit;
+        else   // part of them is summed in the records' spare word, beside the other sums
+            for (uint64_t i = 0; i < h.size(); ++i) h[i].nb_hit_equiv += h[i].reserved;
         for (size_t i = 0; i < h.size(); ++i) {
             auto& a = o->facets[i]; const auto& b = h[i];
             a.nb_mc_hit += b.nb_mc_hit; a.nb_hit_equiv += b.nb_hit_equiv; a.nb_desorbed += b.nb_desorbed;

@@ -187,9 +187,23 @@ static_assert(sizeof(LeafUV) == 64, "LeafUV layout");
 // LDS of one wave's walk: slot r holds ray r (the ray of lane r). The FP32
 // copy serves the box tests, the FP64 one the facet tests.
 struct alignas(16) WaveLds {
-    float4 ra[64];                     // origin, nearest t so far (widened)
-    float4 rb[64];                     // 1 / direction, facet to skip (bits)
-    double2 p01[64], p2d0[64], d12[64];   // position x y | z, direction x | y z
+    // (after the walk the same memory holds the event's tally updates)
+    union {
+        struct {
+            float4 ra[64];             // origin, nearest t so far (widened)
+            float4 rb[64];             // 1 / direction, facet to skip (bits)
+        };
+        double cell[3 * 64];           // texture cell updates, t names the cells
+    };
+    union {
+        struct {
+            double2 p01[64], p2d0[64], d12[64];   // position x y | z, direction x | y z
+        };
+        struct {
+            double sums[5 * 64];       // facet counter updates (words 3.. of a record)
+            unsigned long long record[64];
+        };
+    };
     unsigned long long t[64];          // nearest t so far (bits of a positive double)
     int32_t facet[64];                 // its facet, -1 none
     uint32_t nodes[MFG_WALK_NODES];    // ray << task_bits | node

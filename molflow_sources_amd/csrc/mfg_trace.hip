@@ -643,6 +643,14 @@ struct LaneStack {
     }
 };
 
+// The same value, unknown to the optimiser: what is computed from it belongs
+// to this place of the loop instead of being kept in registers all through
+// it (LDS addresses of a lane's slots cost an instruction or two).
+__device__ __forceinline__ uint32_t here(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Orders this wave's LDS accesses before and after it (the hardware runs
 // them in order; this keeps the compiler from moving them or from splitting
 // the control flow around it).
@@ -1220,20 +1228,37 @@ struct Tracer {
     }
     MFG_IN double ort(const HitRegs& H) const { return fabs(dot(dir, H.N)); }
     // RecordHitOnTexture (Particle.cpp:977-1004)
-    MFG_IN void texture(const HitRegs& H, int32_t f, int m, bool count, double vf, double of) {
+    // The steady-state cell of an event's records is added to in this lane's
+    // slot of W (staged: W.t names the cell, ~0 none yet) and goes to memory
+    // with the wave's others after the event.
+    MFG_IN void texture(const HitRegs& H, int32_t f, int m, bool count, double vf, double of, bool staged = true) {
         const DPhys& ph = P.phys[f];
         uint32_t add;
         if (!cell(ph, add)) return;
         double ov = vc().c_factor * vel * ort(H);
-        double inc = P.tex_inc[vc().tex_base + (size_t)ph.tex_off + add];
+        const uint64_t at = vc().tex_base + (uint64_t)ph.tex_off + add;
+        const double n = count ? w() : 0.0, sv = w() * of * ov * P.tex_inc[at], s1 = w() * vf / ov;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             int slot = k == 0 ? 0 : m;
             if (k == 1 && m <= 0) break;
-            mfg_texture_cell* c = P.tex + vc().tex_base + (size_t)slot * vc().n_tex + (size_t)ph.tex_off + add;
-            if (count) atomic_addd(&c->count_equiv, ori);
-            atomic_addd(&c->sum_1_per_ort_velocity, ori * vf / ov);
-            atomic_addd(&c->sum_v_ort_per_area, ori * of * ov * inc);
+            if (k == 0 && staged) {
+                const uint32_t lane = here(__lane_id());
+                double* S = W.cell + 3u * lane;
+                if (W.t[lane] == ~0ull) {
+                    W.t[lane] = at;
+                    S[0] = n; S[1] = sv; S[2] = s1;
+                    continue;
+                }
+                if (W.t[lane] == at) {
+                    S[0] += n; S[1] += sv; S[2] += s1;
+                    continue;
+                }
+            }
+            mfg_texture_cell* c = P.tex + at + (size_t)slot * vc().n_tex;
+            if (count) atomic_addd(&c->count_equiv, n);
+            atomic_addd(&c->sum_1_per_ort_velocity, s1);
+            atomic_addd(&c->sum_v_ort_per_area, sv);
         }
     }
     // RecordDirectionVector (Particle.cpp:1006-1023)
@@ -1570,7 +1595,7 @@ struct Tracer {
         }
         profile(H, src, m, false, 2.0, 1.0);
         log_hit(H, src);
-        if ((H.flags & FF_COUNT_DES) && (H.flags & FF_TEXTURE)) texture(H, src, m, true, 2.0, 1.0);
+        if ((H.flags & FF_COUNT_DES) && (H.flags & FF_TEXTURE)) texture(H, src, m, true, 2.0, 1.0, false);
         trace(src, 0);
     }
 
@@ -1815,7 +1840,7 @@ struct Tracer {
     // One event of an alive particle (one SimulationMCStep iteration): its
     // ray goes into the wave's walk, which all lanes run together (also
     // those without a particle), then finish() treats what it met.
-    MFG_IN void trace_ray(uint32_t lane, bool alive) {
+    MFG_IN HitRec trace_ray(uint32_t lane, bool alive) {
         int32_t root = -1;
         if (alive) {
             if constexpr (CLOCKED) ++nb_events;
@@ -1824,16 +1849,19 @@ struct Tracer {
             if constexpr ((FEAT & FEAT_TRANSPARENT) != 0) pass->n[lane] = 0;
         }
         const CoinState cs{rng.k0, rng.k1, rng.p0, rng.p1, nb_events, time, var};
-        walk<(FEAT & FEAT_TRANSPARENT) != 0>(P, W, pass, lnodes, lane, alive, root, cs);
+        walk<(FEAT & FEAT_TRANSPARENT) != 0>(P, W, pass, lnodes, here(lane), alive, root, cs);
+        lane = here(lane);
         // the ray is read back from its slot: not held in registers meanwhile
         const double2 a = W.p01[lane], b = W.p2d0[lane], c = W.d12[lane];
         pos = mk(a.x, a.y, b.x);
         dir = mk(b.y, c.x, c.y);
+        const HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
+        W.t[lane] = ~0ull;   // now the texture cell of the event
+        return h;
     }
     // Returns false when the particle ends.
-    MFG_IN bool finish(uint32_t lane) {
+    MFG_IN bool finish(uint32_t lane, HitRec h) {
         constexpr bool TR = (FEAT & FEAT_TRANSPARENT) != 0;
-        HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
         if (h.facet < 0) {  // leak
             atomic_addu(&P.glob[vc().glob_index].nb_leak, 1ull);   // rare: no register kept for it
             unsigned long long at = atomicAdd(P.leak_count, 1ull);
@@ -1982,6 +2010,8 @@ __device__ __forceinline__ uint32_t find_variant(const uint64_t* prefix, uint32_
     while (hi - lo > 1) { uint32_t mid = (lo + hi) / 2; if (prefix[mid] <= g) lo = mid; else hi = mid; }
     return lo;
 }
+
+constexpr int kFewRecords = 8;   // fewer records than this go out lane by lane (nothing to merge, one LDS round trip less)
 
 template <uint32_t FEAT, bool ONE>
 __device__ __forceinline__ void trace_body(const TraceParams& P) {
@@ -2163,9 +2193,9 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
             break;
         }
         if (!__ballot(!done)) break;
-        T.trace_ray(lane, alive);
+        const HitRec met = T.trace_ray(here(lane), alive);
         if (alive) {
-            alive = T.finish(lane);
+            alive = T.finish(here(lane), met);
             if (alive && --events_left == 0) alive = false;
         }
         // slot-0 facet counters of this iteration: lanes that updated the
@@ -2190,7 +2220,51 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
                     T.clear_pending();
                 }
             }
-            if (T.pend_f >= 0) T.flush_pending_direct();
+            // the records of the other facets: adjacent lanes add adjacent words
+            // (3.. of a record), which leave the CU as one request. Device-
+            // scope atomics are served at 2.35e10 requests a second however
+            // many words one holds (1e5 records: 7.8e9 records a second with
+            // a request for each of 3 words, 2.3e10 with 3 or 4 words in one).
+            const bool cold = T.pend_f >= 0 && T.pend_hot < 0;
+            const uint64_t cm = __ballot(cold);
+            if (T.pend_f >= 0 && (!cold || __popcll(cm) < kFewRecords)) T.flush_pending_direct();
+            if (__popcll(cm) >= kFewRecords) {
+                constexpr uint32_t NW = decltype(T)::WEIGHTED ? 5 : 4;
+                const uint32_t ln = here(lane);
+                unsigned long long at = ~0ull;
+                if (cold) {
+                    at = T.vc().fc_base + (uint32_t)T.local(T.pend_f);
+                    double* a = W.sums + NW * ln;
+                    a[0] = T.pend_abs; a[1] = T.pend_s1v; a[2] = T.pend_svo; a[3] = T.pend_s1pv;
+                    if constexpr (NW == 5) a[4] = T.weighted() ? T.pend_he : 0.0;   // in `reserved`: the read adds it
+                    if (T.pend_hits) atomic_addu(&P.fc[at].nb_mc_hit, T.pend_hits);
+                    T.clear_pending();
+                }
+                W.record[ln] = at;
+                wave_sync();
+#pragma unroll
+                for (uint32_t q = 0; q < NW; ++q) {
+                    const uint32_t j = q * 64u + ln, r = j / NW;
+                    const unsigned long long rec = W.record[r];
+                    const double v = W.sums[j];
+                    if (rec != ~0ull && v != 0.0) atomic_addd(reinterpret_cast<double*>(P.fc + rec) + 3u + j % NW, v);
+                }
+                wave_sync();
+            }
+        }
+        // the texture cells of this iteration, three words each, likewise
+        const uint32_t ln = here(lane);
+        if (__ballot(W.t[ln] != ~0ull)) {
+            wave_sync();
+#pragma unroll
+            for (uint32_t q = 0; q < 3; ++q) {
+                const uint32_t j = q * 64u + ln, r = j / 3u;
+                const unsigned long long at = W.t[r];
+                if (at == ~0ull) continue;
+                const double v = W.cell[j];
+                if (v != 0.0) atomic_addd(reinterpret_cast<double*>(P.tex + at) + j % 3u, v);
+            }
+            wave_sync();
         }
     }
     // flush lane accumulators: one set of atomics per wave for a single
