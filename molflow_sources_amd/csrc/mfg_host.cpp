@@ -883,9 +883,6 @@ struct mfg_context {
     DevBuf<int32_t> stack_spill;         // per-lane entries beyond the LDS part (transparent models)
     uint32_t task_bits = 26;             // bits of a node or leaf record index in a walk task
     int bvh_width = MFG_BVH_WIDTH, leaf_size = 2;   // children per BVH node, facets per leaf
-    // BVH nodes a block of up to 256 lanes keeps in LDS at most (top of the
-    // breadth-first array)
-    uint32_t node_cache = 128;
     size_t lds_per_block = 65536;        // the device's LDS limit for one block
     // device data
     DevBuf<DFacet> facets;
@@ -1385,8 +1382,7 @@ uint32_t lds_node_count(const mfg_context* c, uint32_t feats, int block, int wav
     size_t share = block > 256 ? c->lds_per_block : c->lds_per_block * (size_t)block / 256 / (size_t)std::max(1, waves);
     share = share / kLdsGrain * kLdsGrain;
     const size_t used = (size_t)(block / 64) * mfg_wave_lds(feats) + c->hot_bytes();
-    size_t n = share > used ? (share - used) / sizeof(BvhNode) : 0;
-    if (block <= 256) n = std::min<size_t>(n, c->node_cache);
+    const size_t n = share > used ? (share - used) / sizeof(BvhNode) : 0;
     return (uint32_t)std::min<size_t>(n, c->nodes.n);
 }
 
