@@ -1529,6 +1529,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     const uint64_t n_waves = (uint64_t)grid * (uint64_t)(block / 64);
     const uint64_t cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
     p.lane_quota = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cap, (total + c->in_flight + n_waves - 1) / n_waves));
+    p.dealt = n_waves * p.lane_quota;
     std::vector<uint64_t> key(n_des, n_des + nv);
     key.push_back(max_events); key.push_back(feats); key.push_back((uint64_t)grid); key.push_back(block);
     key.push_back((uint64_t)waves);
@@ -1546,7 +1547,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
             throw Err(MFG_ERR_DEVICE, "zero kernel launch failed");
         if (events) HIPCHK(hipEventRecord(c->ev0, s));
         if (mfg_launch_trace(p, feats, nv == 1, waves, grid, block, s)) throw Err(MFG_ERR_DEVICE, std::string("trace launch failed: ") + hipGetErrorString(hipGetLastError()));
-        if (p.carry && mfg_launch_carry_flip(p.carry_ctl, p.next_particle, p.carry, p.carry_cap, c->counters.p + 7, s))
+        if (p.carry && mfg_launch_carry_flip(p.carry_ctl, p.next_particle, p.dealt, p.carry, p.carry_cap, c->counters.p + 7, s))
             throw Err(MFG_ERR_DEVICE, "carry flip launch failed");
     };
     if (c->graph_on) {

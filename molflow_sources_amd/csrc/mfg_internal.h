@@ -308,6 +308,7 @@ struct TraceParams {
     uint32_t task_bits;               // bits of a walk task's node or record index (the rest: its ray)
     uint32_t child_lanes;             // 1: leaves so small (at most 3 facets) that 8 nodes' facets fit the list
     uint32_t lane_quota;              // lanes of a wave that take particles
+    uint64_t dealt;                   // items dealt out by wave index (waves * lane_quota) before the queue's
     uint32_t stack_total;             // entries a lane's own walk may need; the ones past MFG_LANE_STACK
     int32_t* stack_spill;             // live in this per-lane global area (lane-major)
     const double* src_cum;            // cumulative source weights
@@ -430,7 +431,7 @@ int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int w
 int mfg_launch_intersect(const IsectParams& p, void* stream);
 // after a carry launch: append the parked particles the launch did not
 // claim (time limit) to the output half, then swap the halves
-int mfg_launch_carry_flip(unsigned long long* carry_ctl, const unsigned long long* claimed, CarryRec* carry,
+int mfg_launch_carry_flip(unsigned long long* carry_ctl, const unsigned long long* claimed, uint64_t dealt, CarryRec* carry,
                           uint64_t cap, unsigned long long* overflow, void* stream);
 int mfg_launch_zero(void* ptr, uint64_t bytes, void* stream);
 int mfg_launch_backward(const double* jac, const double* up, double* grad, uint32_t n_targets, uint32_t n_groups,

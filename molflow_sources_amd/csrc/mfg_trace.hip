@@ -2100,8 +2100,15 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
             uint32_t cnt = (uint32_t)__popcll(mask);
             uint32_t leader = (uint32_t)__ffsll((unsigned long long)mask) - 1;
             unsigned long long base = 0;
-            if (lane == leader) base = atomicAdd(P.next_particle, (unsigned long long)cnt);
-            base = __shfl(base, leader, 64);
+            if (iter == 1) {
+                // the first items are dealt out by wave index: thousands of
+                // waves taking them from the queue's one word would wait for
+                // each other
+                base = (unsigned long long)(gl >> 6) * P.lane_quota;
+            } else {
+                if (lane == leader) base = P.dealt + atomicAdd(P.next_particle, (unsigned long long)cnt);
+                base = __shfl(base, leader, 64);
+            }
             // after a stop request no new particle starts; resumed ones still
             // run (to the end, or back into the carry buffer)
             const uint64_t limit = stop ? n_in : items;
@@ -2327,24 +2334,24 @@ __global__ void __launch_bounds__(256 * WAVES, WAVES) k_trace_cu(TraceParams P) 
     trace_body<FEAT, true>(P);
 }
 
-// Parked particles that a launch did not claim: the queue hands out items
-// [0, claimed) and the first n_in of them are the resumed particles, so
-// [min(claimed, n_in), n_in) were never taken. That happens only when the
+// Parked particles that a launch did not claim: the launch deals out items
+// [0, dealt), its queue hands out the `claimed` next ones, and the first n_in of them are the resumed particles, so
+// [min(dealt + claimed, n_in), n_in) were never taken. That happens only when the
 // launch time limit stops the claims (a dry queue means every item was
 // claimed). These records are appended to the output half after the ones
 // the waves parked themselves.
-__device__ __forceinline__ void carry_counts(const unsigned long long* ctl, const unsigned long long* claimed,
+__device__ __forceinline__ void carry_counts(const unsigned long long* ctl, const unsigned long long* claimed, uint64_t dealt,
                                              uint64_t& half, uint64_t& first, uint64_t& n, uint64_t& n_out) {
     half = ctl[2] & 1ull;
     const uint64_t n_in = ctl[half];
-    first = *claimed < n_in ? *claimed : n_in;
+    first = dealt + *claimed < n_in ? dealt + *claimed : n_in;
     n = n_in - first;
     n_out = ctl[half ^ 1ull];
 }
-__global__ void k_carry_rescue(const unsigned long long* ctl, const unsigned long long* claimed, CarryRec* carry,
-                               uint64_t cap) {
+__global__ void k_carry_rescue(const unsigned long long* ctl, const unsigned long long* claimed, uint64_t dealt,
+                               CarryRec* carry, uint64_t cap) {
     uint64_t half, first, n, n_out;
-    carry_counts(ctl, claimed, half, first, n, n_out);
+    carry_counts(ctl, claimed, dealt, half, first, n, n_out);
     const CarryRec* in = carry + half * cap;
     CarryRec* out = carry + (half ^ 1ull) * cap;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -2353,11 +2360,11 @@ __global__ void k_carry_rescue(const unsigned long long* ctl, const unsigned lon
 // After a launch (and the rescue): the half it resumed from is consumed,
 // and the half that received its leftovers becomes the next launch's
 // input. overflow is set if the rescued records did not fit.
-__global__ void k_carry_flip(unsigned long long* ctl, const unsigned long long* claimed, uint64_t cap,
+__global__ void k_carry_flip(unsigned long long* ctl, const unsigned long long* claimed, uint64_t dealt, uint64_t cap,
                              unsigned long long* overflow) {
     if (threadIdx.x == 0) {
         uint64_t half, first, n, n_out;
-        carry_counts(ctl, claimed, half, first, n, n_out);
+        carry_counts(ctl, claimed, dealt, half, first, n, n_out);
         uint64_t total = n_out + n;
         if (total > cap) { *overflow = 1ull; total = cap; }
         ctl[half ^ 1ull] = total;
@@ -2509,15 +2516,15 @@ int mfg_launch_trace(const TraceParams& p, uint32_t features, bool single, int w
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int mfg_launch_carry_flip(unsigned long long* ctl, const unsigned long long* claimed, CarryRec* carry, uint64_t cap,
+int mfg_launch_carry_flip(unsigned long long* ctl, const unsigned long long* claimed, uint64_t dealt, CarryRec* carry, uint64_t cap,
                           unsigned long long* overflow, void* stream) {
     uint64_t blocks = (cap + 255) / 256;
     if (blocks > 1024) blocks = 1024;
     if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(k_carry_rescue, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, ctl, claimed, carry,
-                       cap);
+    hipLaunchKernelGGL(k_carry_rescue, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, ctl, claimed, dealt,
+                       carry, cap);
     if (hipGetLastError() != hipSuccess) return -1;
-    hipLaunchKernelGGL(k_carry_flip, dim3(1), dim3(64), 0, (hipStream_t)stream, ctl, claimed, cap, overflow);
+    hipLaunchKernelGGL(k_carry_flip, dim3(1), dim3(64), 0, (hipStream_t)stream, ctl, claimed, dealt, cap, overflow);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
