@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -851,6 +852,11 @@ struct DevBuf {
     size_t bytes() const { return n * sizeof(T); }
 };
 
+// Tally reads go through pinned memory in pieces of at most kStagePiece bytes,
+// kStagePieces of them on their way at once.
+constexpr size_t kStagePiece = (size_t)1 << 20;
+constexpr int kStagePieces = 8;
+
 struct VariantLayout {
     uint32_t n_facets, n_slots, n_struct;
     uint64_t fc, force, tex, n_tex, dir, n_dir, prof, n_prof, am, n_am, gh, n_gh, fh, n_fh;
@@ -935,6 +941,13 @@ struct mfg_context {
     DevBuf<mfg_profile_slice> prof;
     DevBuf<unsigned long long> am, counters;   // counters: next_particle, log_count, leak_count, time-limit flag, carry control[3]
     DevBuf<DGlobal> glob;
+    std::vector<DGlobal> glob_seen;      // what glob held after the last run (zeros after a clear)
+    DGlobal* pin_glob = nullptr;         // pinned: glob and `counters` as a run left them
+    unsigned long long* pin_counters = nullptr;
+    // pinned staging of tally reads: grown to what they need, 8 MB at most
+    unsigned char* stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t stage_ev[kStagePieces] = {};
     DevBuf<mfg_log_entry> log;
     DevBuf<double> leaks;
     uint32_t log_cap = 0;
@@ -1205,11 +1218,15 @@ void upload_models(mfg_context* c) {
     if (c->pin_cap < c->dvars.size() + 1) {
         if (c->pin_vars) (void)hipHostFree(c->pin_vars);
         if (c->pin_prefix) (void)hipHostFree(c->pin_prefix);
-        c->pin_vars = nullptr; c->pin_prefix = nullptr;
+        if (c->pin_glob) (void)hipHostFree(c->pin_glob);
+        c->pin_vars = nullptr; c->pin_prefix = nullptr; c->pin_glob = nullptr;
         HIPCHK(hipHostMalloc((void**)&c->pin_vars, (c->dvars.size() + 1) * sizeof(DVariant), hipHostMallocDefault));
         HIPCHK(hipHostMalloc((void**)&c->pin_prefix, (c->dvars.size() + 1) * sizeof(uint64_t), hipHostMallocDefault));
+        HIPCHK(hipHostMalloc((void**)&c->pin_glob, (c->dvars.size() + 1) * sizeof(DGlobal) + 16 * sizeof(unsigned long long),
+                             hipHostMallocDefault));
         c->pin_cap = c->dvars.size() + 1;
     }
+    c->pin_counters = reinterpret_cast<unsigned long long*>(c->pin_glob + c->pin_cap);
     c->features = feat;
     c->pid_base.assign(c->models.size(), 0);
     c->loaded = true;
@@ -1223,19 +1240,21 @@ void upload_models(mfg_context* c) {
 // (ResetSimulation) the parked particles are dropped too.
 void zero_tallies(mfg_context* c, bool keep_particles = false) {
     hipStream_t s = c->stream;
-    auto z = [&](void* p, size_t b) { if (mfg_launch_zero(p, b, s)) throw Err(MFG_ERR_DEVICE, "zero kernel launch failed"); };
-    z(c->fc.p, c->fc.bytes()); z(c->force.p, c->force.bytes()); z(c->tex.p, c->tex.bytes());
-    z(c->dir.p, c->dir.bytes()); z(c->prof.p, c->prof.bytes()); z(c->am.p, c->am.bytes());
-    z(c->gh.p, c->gh.bytes()); z(c->fh.p, c->fh.bytes()); z(c->glob.p, c->glob.bytes());
+    ZeroList z;
+    z.add(c->fc.p, c->fc.bytes()); z.add(c->force.p, c->force.bytes()); z.add(c->tex.p, c->tex.bytes());
+    z.add(c->dir.p, c->dir.bytes()); z.add(c->prof.p, c->prof.bytes()); z.add(c->am.p, c->am.bytes());
+    z.add(c->gh.p, c->gh.bytes()); z.add(c->fh.p, c->fh.bytes()); z.add(c->glob.p, c->glob.bytes());
     if (keep_particles) {
         // log and leak counts, time-limit flag; not the carry words (4..6)
-        z(c->counters.p + 1, 3 * sizeof(unsigned long long));
-        z(c->counters.p + 7, sizeof(unsigned long long));
+        z.add(c->counters.p + 1, 3 * sizeof(unsigned long long));
+        z.add(c->counters.p + 7, sizeof(unsigned long long));
     } else {
-        z(c->counters.p, c->counters.bytes());
+        z.add(c->counters.p, c->counters.bytes());
     }
-    if (c->adj_j0.p) { z(c->adj_j0.p, c->adj_j0.bytes()); z(c->adj_jac.p, c->adj_jac.bytes()); }
+    if (c->adj_j0.p) { z.add(c->adj_j0.p, c->adj_j0.bytes()); z.add(c->adj_jac.p, c->adj_jac.bytes()); }
+    if (mfg_launch_zero(z, s)) throw Err(MFG_ERR_DEVICE, "zero kernel launch failed");
     HIPCHK(hipStreamSynchronize(s));
+    c->glob_seen.assign(c->dvars.size(), DGlobal{});
     c->adj_des = 0;
     if (!keep_particles) c->in_flight = 0;   // the counters above include the carry control words
 }
@@ -1514,10 +1533,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
         size_t need = (size_t)grid * block * (c->stack_size - MFG_LANE_STACK);
         if (c->stack_spill.n < need) { c->stack_spill.alloc(need); reset_graph(c); }
     }
-    // read the global counters before the run to report this run's hits
-    std::vector<DGlobal> before(nv);
     hipStream_t s = c->stream;
-    HIPCHK(hipMemcpyAsync(before.data(), c->glob.p, nv * sizeof(DGlobal), hipMemcpyDeviceToHost, s));
     *c->stop_host = 0;
     TraceParams p = make_params(c, total, max_events);
     p.lds_nodes = lds_node_count(c, feats, block, waves);
@@ -1541,9 +1557,11 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     auto enqueue = [&](bool events) {
         HIPCHK(hipMemcpyAsync(c->variants.p, c->pin_vars, nv * sizeof(DVariant), hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(c->prefix.p, c->pin_prefix, (nv + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, s));
-        if (mfg_launch_zero(c->counters.p, sizeof(unsigned long long), s) ||
-            mfg_launch_zero(c->counters.p + 3, sizeof(unsigned long long), s) ||
-            (c->adj_groups && mfg_launch_zero(c->counters.p + 8, sizeof(unsigned long long), s)))
+        ZeroList z;
+        z.add(c->counters.p, sizeof(unsigned long long));
+        z.add(c->counters.p + 3, sizeof(unsigned long long));
+        if (c->adj_groups) z.add(c->counters.p + 8, sizeof(unsigned long long));
+        if (mfg_launch_zero(z, s))
             throw Err(MFG_ERR_DEVICE, "zero kernel launch failed");
         if (events) HIPCHK(hipEventRecord(c->ev0, s));
         if (mfg_launch_trace(p, feats, nv == 1, waves, grid, block, s)) throw Err(MFG_ERR_DEVICE, std::string("trace launch failed: ") + hipGetErrorString(hipGetLastError()));
@@ -1565,29 +1583,28 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
         enqueue(true);
     }
     HIPCHK(hipEventRecord(c->ev1, s));
+    HIPCHK(hipMemcpyAsync(c->pin_glob, c->glob.p, nv * sizeof(DGlobal), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(c->pin_counters, c->counters.p, c->counters.bytes(), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    std::vector<DGlobal> after(nv);
-    HIPCHK(hipMemcpy(after.data(), c->glob.p, nv * sizeof(DGlobal), hipMemcpyDeviceToHost));
-    unsigned long long expired = 0;
-    HIPCHK(hipMemcpy(&expired, c->counters.p + 3, sizeof(expired), hipMemcpyDeviceToHost));
+    // this run's hits: against what the counters held before it
+    uint64_t hits = 0, des = 0;
+    c->glob_seen.resize(nv);
+    for (size_t v = 0; v < nv; ++v) {
+        hits += c->pin_glob[v].nb_mc_hit - c->glob_seen[v].nb_mc_hit;
+        des += c->pin_glob[v].nb_desorbed - c->glob_seen[v].nb_desorbed;
+        c->glob_seen[v] = c->pin_glob[v];
+    }
+    const unsigned long long expired = c->pin_counters[3];
     if (p.carry) {
-        unsigned long long ctl[4];   // carry control words and the overflow flag
-        HIPCHK(hipMemcpy(ctl, c->counters.p + 4, sizeof(ctl), hipMemcpyDeviceToHost));
+        const unsigned long long* ctl = c->pin_counters + 4;   // carry control words and the overflow flag
         c->in_flight = ctl[ctl[2] & 1ull];
         if (ctl[3]) throw Err(MFG_ERR_STATE, "carry buffer overflow: parked particles were lost");
     }
-    uint64_t hits = 0, des = 0;
-    for (size_t v = 0; v < nv; ++v) {
-        hits += after[v].nb_mc_hit - before[v].nb_mc_hit;
-        des += after[v].nb_desorbed - before[v].nb_desorbed;
-        c->pid_base[v] += n_des[v];
-    }
+    for (size_t v = 0; v < nv; ++v) c->pid_base[v] += n_des[v];
     if (c->adj_groups) {
-        unsigned long long ov = 0;
-        HIPCHK(hipMemcpy(&ov, c->counters.p + 8, sizeof(ov), hipMemcpyDeviceToHost));
-        if (ov) throw Err(MFG_ERR_LIMIT, "adjoint: a particle scored on targets more than " + std::to_string(MFG_ADJ_SEG) +
+        if (c->pin_counters[8]) throw Err(MFG_ERR_LIMIT, "adjoint: a particle scored on targets more than " + std::to_string(MFG_ADJ_SEG) +
                                              " times between two sticky collisions (cutoff term incomplete)");
         c->adj_des += des;
     }
@@ -1601,92 +1618,176 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     }
 }
 
+// One device array of a tally read: `n` units of `unit` bytes, handed to
+// add(host copy, first unit, units) piece by piece, from several threads.
+struct StageJob {
+    const void* dev;
+    size_t unit, n;
+    std::function<void(const void*, size_t, size_t)> add;
+};
+
+// Copies the jobs' arrays to the host through the pinned staging memory and
+// adds them. A read into the caller's fresh buffers is bound by the first
+// touch of their pages, so larger ones are added by several threads, each
+// piece as soon as its copy has landed. Through pageable vectors (allocated,
+// zeroed, filled by the runtime's own staging, then added by one thread) the
+// 32 MB of a beam pipe took 8.5 ms, this way 2.6.
+void run_stage(mfg_context* c, const std::vector<StageJob>& jobs) {
+    struct Piece { const StageJob* job; size_t first, n; };
+    std::vector<Piece> pieces;
+    size_t bytes = 0;
+    for (const StageJob& j : jobs) {
+        const size_t per = std::max<size_t>(1, kStagePiece / j.unit);
+        for (size_t i = 0; i < j.n; i += per) pieces.push_back({&j, i, std::min(per, j.n - i)});
+        bytes += j.n * j.unit;
+    }
+    hipStream_t s = c->stream;
+    const size_t want = bytes <= kStagePiece ? (bytes + 64 * pieces.size() + 65535) / 65536 * 65536 : kStagePiece * kStagePieces;
+    if (c->stage_bytes < want) {
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
+        HIPCHK(hipHostMalloc((void**)&c->stage, want, hipHostMallocDefault));
+        c->stage_bytes = want;
+    }
+    if (bytes <= kStagePiece) {
+        // small: all copies, one wait
+        size_t at = 0;
+        for (const Piece& p : pieces) {
+            HIPCHK(hipMemcpyAsync(c->stage + at, p.job->dev, p.n * p.job->unit, hipMemcpyDeviceToHost, s));
+            at += (p.n * p.job->unit + 63) / 64 * 64;
+        }
+        HIPCHK(hipStreamSynchronize(s));
+        at = 0;
+        for (const Piece& p : pieces) {
+            p.job->add(c->stage + at, p.first, p.n);
+            at += (p.n * p.job->unit + 63) / 64 * 64;
+        }
+        return;
+    }
+    for (hipEvent_t& e : c->stage_ev)
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // piece k uses slot k mod kStagePieces; thread t adds the pieces of the
+    // slots t, t + T, ... and sends for the slot's next piece when it is free
+    const int T = (int)std::min<size_t>(std::min<unsigned>(std::max(1u, std::thread::hardware_concurrency()), 4), pieces.size());
+    auto send = [&](size_t k) -> hipError_t {
+        const Piece& p = pieces[k];
+        const size_t slot = k % kStagePieces;
+        hipError_t e = hipMemcpyAsync(c->stage + slot * kStagePiece, (const char*)p.job->dev + p.first * p.job->unit,
+                                      p.n * p.job->unit, hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipEventRecord(c->stage_ev[slot], s);
+    };
+    for (size_t k = 0; k < std::min<size_t>(pieces.size(), kStagePieces); ++k) HIPCHK(send(k));
+    std::vector<hipError_t> errs((size_t)T, hipSuccess);
+    auto work = [&](int t) {
+        hipError_t& e = errs[(size_t)t];
+        e = hipSetDevice(c->device);
+        for (size_t k = 0; k < pieces.size() && e == hipSuccess; ++k) {
+            const size_t slot = k % kStagePieces;
+            if ((int)(slot % (size_t)T) != t) continue;
+            e = hipEventSynchronize(c->stage_ev[slot]);
+            if (e != hipSuccess) break;
+            pieces[k].job->add(c->stage + slot * kStagePiece, pieces[k].first, pieces[k].n);
+            if (k + kStagePieces < pieces.size()) e = send(k + kStagePieces);
+        }
+    };
+    std::vector<std::thread> th;
+    try {
+        for (int t = 1; t < T; ++t) th.emplace_back(work, t);
+    } catch (...) {
+        // a thread could not be started: its slots are done here below
+    }
+    work(0);
+    const int started = (int)th.size();
+    for (auto& x : th) x.join();
+    for (int t = started + 1; t < T; ++t) work(t);
+    HIPCHK(hipStreamSynchronize(s));
+    for (hipError_t e : errs) HIPCHK(e);
+}
+
 void add_tallies(mfg_context* c, uint32_t vi, const mfg_tally_view* o) {
     if (!o || o->struct_size != sizeof(mfg_tally_view)) throw Err(MFG_ERR_INVALID, "mfg_tally_view size mismatch");
     if (vi >= c->layouts.size()) throw Err(MFG_ERR_INVALID, "variant index out of range");
     const VariantLayout& L = c->layouts[vi];
-    auto fetch = [&](auto* dev, uint64_t off, uint64_t n) {
+    std::vector<StageJob> jobs;
+    auto job = [&](auto* dev, uint64_t off, uint64_t n, auto add) {
         using T = std::remove_pointer_t<decltype(dev)>;
-        std::vector<T> h(n);
-        if (n) HIPCHK(hipMemcpy(h.data(), dev + off, n * sizeof(T), hipMemcpyDeviceToHost));
-        return h;
+        if (n) jobs.push_back({dev + off, sizeof(T), (size_t)n, [add](const void* h, size_t first, size_t cnt) { add((const T*)h, first, cnt); }});
     };
+    auto plain = [&](auto* dev, uint64_t off, uint64_t n, auto* out) {
+        job(dev, off, n, [out](const auto* h, size_t first, size_t cnt) { for (size_t i = 0; i < cnt; ++i) out[first + i] += h[i]; });
+    };
+    const uint64_t S = L.n_slots;
+    uint64_t log_n = 0, leak_n = 0;
+    job(c->counters.p, 1, 2, [&](const unsigned long long* h, size_t, size_t) { log_n = h[0]; leak_n = h[1]; });
     if (o->global) {
-        auto g = fetch(c->glob.p, vi, 1);
-        mfg_global_counters& a = *o->global;
-        a.nb_mc_hit += g[0].nb_mc_hit; a.nb_hit_equiv += g[0].nb_hit_equiv; a.nb_desorbed += g[0].nb_desorbed;
-        a.nb_abs_equiv += g[0].nb_abs_equiv; a.nb_leak_total += g[0].nb_leak; a.dist_traveled_total += g[0].dist_total;
-        a.dist_traveled_full_hits_only += g[0].dist_full; a.nb_decayed += g[0].nb_decayed;
+        job(c->glob.p, vi, 1, [o](const DGlobal* g, size_t, size_t) {
+            mfg_global_counters& a = *o->global;
+            a.nb_mc_hit += g[0].nb_mc_hit; a.nb_hit_equiv += g[0].nb_hit_equiv; a.nb_desorbed += g[0].nb_desorbed;
+            a.nb_abs_equiv += g[0].nb_abs_equiv; a.nb_leak_total += g[0].nb_leak; a.dist_traveled_total += g[0].dist_total;
+            a.dist_traveled_full_hits_only += g[0].dist_full; a.nb_decayed += g[0].nb_decayed;
+        });
     }
-    uint64_t S = L.n_slots;
     if (o->facets) {
-        auto h = fetch(c->fc.p, L.fc, S * L.n_facets);
-        // without low-flux weighting the kernel leaves the hit equivalents
-        // to this read: every hit weighs 1
-        if (!c->dvars[vi].low_flux)
-            for (uint64_t i = 0; i < h.size(); ++i) h[i].nb_hit_equiv = (double)h[i].nb_mc_hit;
-        else   // part of them is summed in the records' spare word, beside the other sums
-            for (uint64_t i = 0; i < h.size(); ++i) h[i].nb_hit_equiv += h[i].reserved;
-        for (size_t i = 0; i < h.size(); ++i) {
-            auto& a = o->facets[i]; const auto& b = h[i];
-            a.nb_mc_hit += b.nb_mc_hit; a.nb_hit_equiv += b.nb_hit_equiv; a.nb_desorbed += b.nb_desorbed;
-            a.nb_abs_equiv += b.nb_abs_equiv; a.sum_1_per_ort_velocity += b.sum_1_per_ort_velocity;
-            a.sum_v_ort += b.sum_v_ort; a.sum_1_per_velocity += b.sum_1_per_velocity;
-        }
+        const bool weighted = c->dvars[vi].low_flux != 0;
+        job(c->fc.p, L.fc, S * L.n_facets, [o, weighted](const mfg_facet_counters* h, size_t first, size_t cnt) {
+            for (size_t i = 0; i < cnt; ++i) {
+                auto& a = o->facets[first + i]; const auto& b = h[i];
+                // without low-flux weighting the kernel leaves the hit
+                // equivalents to this read (every hit weighs 1); with it part
+                // of them is summed in the records' spare word, beside the
+                // other sums
+                a.nb_mc_hit += b.nb_mc_hit; a.nb_hit_equiv += weighted ? b.nb_hit_equiv + b.reserved : (double)b.nb_mc_hit;
+                a.nb_desorbed += b.nb_desorbed;
+                a.nb_abs_equiv += b.nb_abs_equiv; a.sum_1_per_ort_velocity += b.sum_1_per_ort_velocity;
+                a.sum_v_ort += b.sum_v_ort; a.sum_1_per_velocity += b.sum_1_per_velocity;
+            }
+        });
     }
-    if (o->forces && L.enable_force) {
-        auto h = fetch(c->force.p, L.force, S * L.n_facets * 9);
-        for (size_t i = 0; i < h.size(); ++i) o->forces[i] += h[i];
-    }
-    if (o->textures && L.n_tex) {
-        auto h = fetch(c->tex.p, L.tex, S * L.n_tex);
-        for (size_t i = 0; i < h.size(); ++i) {
-            o->textures[i].count_equiv += h[i].count_equiv;
-            o->textures[i].sum_v_ort_per_area += h[i].sum_v_ort_per_area;
-            o->textures[i].sum_1_per_ort_velocity += h[i].sum_1_per_ort_velocity;
-        }
-    }
-    if (o->directions && L.n_dir) {
-        auto h = fetch(c->dir.p, L.dir, S * L.n_dir);
-        for (size_t i = 0; i < h.size(); ++i) {
-            for (int k = 0; k < 3; ++k) o->directions[i].dir[k] += h[i].dir[k];
-            o->directions[i].count += h[i].count;
-        }
-    }
-    if (o->profiles && L.n_prof) {
-        auto h = fetch(c->prof.p, L.prof, S * L.n_prof);
-        for (size_t i = 0; i < h.size(); ++i) {
-            o->profiles[i].count_equiv += h[i].count_equiv;
-            o->profiles[i].sum_v_ort += h[i].sum_v_ort;
-            o->profiles[i].sum_1_per_ort_velocity += h[i].sum_1_per_ort_velocity;
-        }
-    }
-    if (o->angle_maps && L.n_am) {
-        auto h = fetch(c->am.p, L.am, L.n_am);
-        for (size_t i = 0; i < h.size(); ++i) o->angle_maps[i] += h[i];
-    }
-    if (o->global_hist && L.n_gh) {
-        auto h = fetch(c->gh.p, L.gh, S * L.n_gh);
-        for (size_t i = 0; i < h.size(); ++i) o->global_hist[i] += h[i];
-    }
-    if (o->facet_hist && L.n_fh) {
-        auto h = fetch(c->fh.p, L.fh, S * L.n_fh);
-        for (size_t i = 0; i < h.size(); ++i) o->facet_hist[i] += h[i];
-    }
+    if (o->forces && L.enable_force) plain(c->force.p, L.force, S * L.n_facets * 9, o->forces);
+    if (o->textures && L.n_tex)
+        job(c->tex.p, L.tex, S * L.n_tex, [o](const mfg_texture_cell* h, size_t first, size_t cnt) {
+            for (size_t i = 0; i < cnt; ++i) {
+                mfg_texture_cell& a = o->textures[first + i];
+                a.count_equiv += h[i].count_equiv;
+                a.sum_v_ort_per_area += h[i].sum_v_ort_per_area;
+                a.sum_1_per_ort_velocity += h[i].sum_1_per_ort_velocity;
+            }
+        });
+    if (o->directions && L.n_dir)
+        job(c->dir.p, L.dir, S * L.n_dir, [o](const mfg_direction_cell* h, size_t first, size_t cnt) {
+            for (size_t i = 0; i < cnt; ++i) {
+                mfg_direction_cell& a = o->directions[first + i];
+                for (int k = 0; k < 3; ++k) a.dir[k] += h[i].dir[k];
+                a.count += h[i].count;
+            }
+        });
+    if (o->profiles && L.n_prof)
+        job(c->prof.p, L.prof, S * L.n_prof, [o](const mfg_profile_slice* h, size_t first, size_t cnt) {
+            for (size_t i = 0; i < cnt; ++i) {
+                mfg_profile_slice& a = o->profiles[first + i];
+                a.count_equiv += h[i].count_equiv;
+                a.sum_v_ort += h[i].sum_v_ort;
+                a.sum_1_per_ort_velocity += h[i].sum_1_per_ort_velocity;
+            }
+        });
+    if (o->angle_maps && L.n_am) plain(c->am.p, L.am, L.n_am, o->angle_maps);
+    if (o->global_hist && L.n_gh) plain(c->gh.p, L.gh, S * L.n_gh, o->global_hist);
+    if (o->facet_hist && L.n_fh) plain(c->fh.p, L.fh, S * L.n_fh, o->facet_hist);
+    run_stage(c, jobs);
+    // log and leak entries: as many as there are
+    jobs.clear();
     if (o->log && o->log_count && c->log_cap) {
-        auto n = fetch(c->counters.p, 1, 1);
-        uint64_t cnt = std::min<uint64_t>(n[0], L.log_limit);
-        auto h = fetch(c->log.p, 0, cnt);
-        for (uint64_t i = 0; i < cnt; ++i) o->log[i] = h[i];
+        const uint64_t cnt = std::min<uint64_t>(log_n, L.log_limit);
+        job(c->log.p, 0, cnt, [o](const mfg_log_entry* h, size_t first, size_t n) { std::copy(h, h + n, o->log + first); });
         *o->log_count = cnt;
     }
     if (o->leak_pos_dir && o->leak_count) {
-        auto n = fetch(c->counters.p, 2, 1);
-        uint64_t cnt = std::min<uint64_t>(n[0], kLeakCap);
-        auto h = fetch(c->leaks.p, 0, cnt * 6);
-        if (!h.empty()) std::memcpy(o->leak_pos_dir, h.data(), h.size() * sizeof(double));
-        *o->leak_count = n[0];
+        job(c->leaks.p, 0, std::min<uint64_t>(leak_n, kLeakCap) * 6,
+            [o](const double* h, size_t first, size_t n) { std::copy(h, h + n, o->leak_pos_dir + first); });
+        *o->leak_count = leak_n;
     }
+    if (!jobs.empty()) run_stage(c, jobs);
 }
 
 void fill_layout(mfg_context* c, uint32_t vi, mfg_tally_layout* L) {
@@ -1801,6 +1902,9 @@ void mfg_destroy(mfg_context* c) {
     if (c->stop_host) (void)hipHostFree(c->stop_host);
     if (c->pin_vars) (void)hipHostFree(c->pin_vars);
     if (c->pin_prefix) (void)hipHostFree(c->pin_prefix);
+    if (c->pin_glob) (void)hipHostFree(c->pin_glob);
+    if (c->stage) (void)hipHostFree(c->stage);
+    for (hipEvent_t e : c->stage_ev) if (e) (void)hipEventDestroy(e);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     hipStream_t s = c->stream;
@@ -1908,7 +2012,9 @@ int mfg_take_tallies(mfg_context* c, const mfg_tally_view* o) {
 int mfg_reinit_particle_log(mfg_context* c) {
     return guarded(c, [&] {
         if (!c->loaded) throw Err(MFG_ERR_STATE, "no model loaded");
-        if (mfg_launch_zero(c->counters.p + 1, sizeof(unsigned long long), c->stream))
+        ZeroList z;
+        z.add(c->counters.p + 1, sizeof(unsigned long long));
+        if (mfg_launch_zero(z, c->stream))
             throw Err(MFG_ERR_DEVICE, "zero kernel launch failed");
         HIPCHK(hipStreamSynchronize(c->stream));
     });

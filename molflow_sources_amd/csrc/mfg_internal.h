@@ -433,7 +433,18 @@ int mfg_launch_intersect(const IsectParams& p, void* stream);
 // claim (time limit) to the output half, then swap the halves
 int mfg_launch_carry_flip(unsigned long long* carry_ctl, const unsigned long long* claimed, uint64_t dealt, CarryRec* carry,
                           uint64_t cap, unsigned long long* overflow, void* stream);
-int mfg_launch_zero(void* ptr, uint64_t bytes, void* stream);
+// arrays of 8-byte words to clear in one launch
+struct ZeroList {
+    uint64_t* p[16];
+    uint64_t words[16];
+    uint32_t n = 0;
+    void add(void* ptr, uint64_t bytes) {
+        if (bytes < 8) return;
+        p[n] = (uint64_t*)ptr;
+        words[n++] = bytes / 8;
+    }
+};
+int mfg_launch_zero(const ZeroList& z, void* stream);
 int mfg_launch_backward(const double* jac, const double* up, double* grad, uint32_t n_targets, uint32_t n_groups,
                         double scale, void* stream);
 uint32_t mfg_trace_kernel_features(uint32_t model_features);

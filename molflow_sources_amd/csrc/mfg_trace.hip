@@ -2404,10 +2404,11 @@ __global__ void __launch_bounds__(256) k_intersect(IsectParams p) {
     p.out_v[i] = v;
 }
 
-__global__ void k_zero(uint64_t* p, uint64_t n) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = 0;
+// Clears several arrays of 8-byte words in one launch.
+__global__ void __launch_bounds__(256) k_zero(ZeroList z) {
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint32_t k = 0; k < z.n; ++k)
+        for (uint64_t i = first; i < z.words[k]; i += stride) z.p[k][i] = 0;
 }
 
 __global__ void k_backward(const double* jac, const double* up, double* grad, uint32_t nt, uint32_t ng, double scale) {
@@ -2537,12 +2538,13 @@ int mfg_launch_intersect(const IsectParams& p, void* stream) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int mfg_launch_zero(void* ptr, uint64_t bytes, void* stream) {
-    uint64_t n = bytes / 8;
-    if (n == 0) return 0;
-    uint64_t grid = (n + 255) / 256;
+int mfg_launch_zero(const ZeroList& z, void* stream) {
+    uint64_t most = 0;
+    for (uint32_t k = 0; k < z.n; ++k) most = most > z.words[k] ? most : z.words[k];
+    if (most == 0) return 0;
+    uint64_t grid = (most + 255) / 256;
     if (grid > 4096) grid = 4096;
-    hipLaunchKernelGGL(k_zero, dim3((uint32_t)grid), dim3(256), 0, (hipStream_t)stream, (uint64_t*)ptr, n);
+    hipLaunchKernelGGL(k_zero, dim3((uint32_t)grid), dim3(256), 0, (hipStream_t)stream, z);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
