@@ -1413,7 +1413,7 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     p.facets = c->facets.p; p.phys = c->phys.p; p.poly = c->poly.p; p.nodes = c->nodes.p;
     p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p; p.roots = c->roots.p; p.variants = c->variants.p;
     p.var_prefix = c->prefix.p; p.n_variants = (uint32_t)c->dvars.size();
-    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3;
+    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3 ? (uint32_t)c->leaf_size : 0u;
     p.stack_total = c->stack_size;
     p.stack_spill = p.stack_total > MFG_LANE_STACK ? c->stack_spill.p : nullptr;
     p.src_cum = c->src_cum.p; p.src_facet = c->src_facet.p; p.og_cdf = c->og_cdf.p; p.am_src = c->am_src.p;
@@ -1857,7 +1857,7 @@ void launch_batch(mfg_context* c, uint64_t n, const double* dO, const double* dD
     // share their walks)
     const uint64_t spread = n / ((uint64_t)c->n_cu * 8), cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
     p.rays_per_wave = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(8, spread));
-    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
+    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3 ? (uint32_t)c->leaf_size : 0u; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
     p.out_facet = dF; p.out_t = dT; p.out_u = dU; p.out_v = dV; p.facet_base = c->dvars[0].facet_base;
     if (mfg_launch_intersect(p, c->stream)) throw Err(MFG_ERR_DEVICE, "intersect launch failed");
 }

@@ -306,7 +306,7 @@ struct TraceParams {
     const uint64_t* var_prefix;       // n_variants+1 prefix of this run's desorptions
     uint32_t n_variants;
     uint32_t task_bits;               // bits of a walk task's node or record index (the rest: its ray)
-    uint32_t child_lanes;             // 1: leaves so small (at most 3 facets) that 8 nodes' facets fit the list
+    uint32_t child_lanes;             // facets a leaf may hold if so few (at most 3) that 8 nodes' facets fit the list, else 0
     uint32_t lane_quota;              // lanes of a wave that take particles
     uint64_t dealt;                   // items dealt out by wave index (waves * lane_quota) before the queue's
     uint32_t stack_total;             // entries a lane's own walk may need; the ones past MFG_LANE_STACK

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "mfg_internal.h"
 
@@ -671,33 +672,101 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
     return v;
 }
 
-// One child of a node against a ray: the test of node_hits for slot c alone,
-// from the node's header and that slot's six plane steps.
+// CH children of a node against a ray (the test of node_hits for the slots
+// from c on), from the node's header and those slots' plane steps.
+template <int CH>
 struct ChildRegs {
+    typedef typename std::conditional<CH == 1, uint16_t, uint32_t>::type Steps;   // CH FP16 steps
     uint4 c0, c1;
-    uint16_t lx, ly, lz, hx, hy, hz;
+    Steps lx, ly, lz, hx, hy, hz;
 };
-template <typename Q>
-__device__ __forceinline__ ChildRegs load_child(const Q* nd, uint32_t c) {
+template <int CH, typename Q>
+__device__ __forceinline__ ChildRegs<CH> load_child(const Q* nd, uint32_t part) {
     const uint4* q = reinterpret_cast<const uint4*>(nd);
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(nd) + 16 + c;
-    return {q[0], q[1], h[0], h[8], h[16], h[24], h[32], h[40]};
+    const auto* h = reinterpret_cast<const typename ChildRegs<CH>::Steps*>(nd) + 16 / CH + part;
+    constexpr int A = 8 / CH;   // one axis
+    return {q[0], q[1], h[0], h[A], h[2 * A], h[3 * A], h[4 * A], h[5 * A]};
 }
-__device__ __forceinline__ float half_bits(uint16_t v) { return (float)__builtin_bit_cast(_Float16, v); }
-__device__ __forceinline__ bool child_hit(const ChildRegs& n, const Ray32& r, float tmax) {
+__device__ __forceinline__ float half_bits(uint32_t v) { return (float)__builtin_bit_cast(_Float16, (unsigned short)v); }
+// bit k: child k of the CH is entered before tmax (a slot without a child is
+// masked by the caller)
+template <int CH>
+__device__ __forceinline__ uint32_t child_hits(const ChildRegs<CH>& n, const Ray32& r, float tmax) {
     const uint32_t ew = n.c0.w;
     const float ax = exp2i((int)(int8_t)(ew & 0xffu)) * r.ix, ay = exp2i((int)(int8_t)((ew >> 8) & 0xffu)) * r.iy;
     const float az = exp2i((int)(int8_t)((ew >> 16) & 0xffu)) * r.iz;
     const float bx = (__uint_as_float(n.c0.x) - r.ox) * r.ix, by = (__uint_as_float(n.c0.y) - r.oy) * r.iy;
     const float bz = (__uint_as_float(n.c0.z) - r.oz) * r.iz;
-    const float x0 = fmaf(half_bits(n.lx), ax, bx), x1 = fmaf(half_bits(n.hx), ax, bx);
-    const float y0 = fmaf(half_bits(n.ly), ay, by), y1 = fmaf(half_bits(n.hy), ay, by);
-    const float z0 = fmaf(half_bits(n.lz), az, bz), z1 = fmaf(half_bits(n.hz), az, bz);
-    // low planes first along +axis rays; a slot without a child is masked by the caller
     const bool px = r.ix >= 0.0f, py = r.iy >= 0.0f, pz = r.iz >= 0.0f;
-    const float a = fmaxf(fmaxf(px ? x0 : x1, py ? y0 : y1), fmaxf(pz ? z0 : z1, 0.0f));
-    const float b = fminf(fminf(px ? x1 : x0, py ? y1 : y0), fminf(pz ? z1 : z0, tmax));
-    return a <= b;
+    const uint32_t nx = px ? n.lx : n.hx, fx = px ? n.hx : n.lx, ny = py ? n.ly : n.hy, fy = py ? n.hy : n.ly;
+    const uint32_t nz = pz ? n.lz : n.hz, fz = pz ? n.hz : n.lz;
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        const int sh = 16 * k;
+        const float a = fmaxf(fmaxf(fmaf(half_bits(nx >> sh), ax, bx), fmaf(half_bits(ny >> sh), ay, by)),
+                              fmaxf(fmaf(half_bits(nz >> sh), az, bz), 0.0f));
+        const float b = fminf(fminf(fmaf(half_bits(fx >> sh), ax, bx), fmaf(half_bits(fy >> sh), ay, by)),
+                              fminf(fmaf(half_bits(fz >> sh), az, bz), tmax));
+        if (a <= b) m |= 1u << k;
+    }
+    return m;
+}
+
+// A node step of a wave with at most 8 CH tasks on its stack: 8 / CH lanes a
+// node, CH children a lane. False, with nothing done, if the facets of the
+// leaves met might not fit the list.
+template <int CH>
+__device__ __forceinline__ bool few_nodes(const TraceParams& P, WaveLds& W, const uint4* lnodes, uint32_t lane,
+                                          uint32_t& top, uint32_t& waiting) {
+    constexpr uint32_t G = 8u / CH;
+    const uint32_t bits = P.task_bits, low = (1u << bits) - 1u;
+    const uint32_t part = lane % G, group = lane / G;
+    const bool on = group < top;
+    uint32_t tag = 0, hit = 0, im = 0, lm = 0;
+    uint4 hd{};
+    if (on) {
+        const uint32_t w = W.nodes[top - 1u - group], ray = w >> bits, node = w & low;
+        tag = w & ~low;
+        ChildRegs<CH> nd;
+        if (node < P.lds_nodes) nd = load_child<CH>(lnodes + (size_t)node * 8, part);
+        else nd = load_child<CH>(P.nodes + node, part);
+        const float4 a = W.ra[ray], b = W.rb[ray];
+        im = nd.c1.w & 0xffu;
+        lm = nd.c0.w >> 24;
+        hit = child_hits<CH>(nd, Ray32{a.x, a.y, a.z, b.x, b.y, b.z}, a.w) << (CH * part);
+        hd = nd.c1;
+    }
+    uint64_t leaves[CH];
+    uint32_t n_leaves = 0;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        leaves[k] = __ballot((hit & lm) >> (CH * part + k) & 1u);
+        n_leaves += (uint32_t)__popcll(leaves[k]);
+    }
+    if (CH > 1 && waiting + n_leaves * P.child_lanes > MFG_WALK_LEAVES) return false;
+    wave_sync();
+    top = 0;
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        const uint32_t c = CH * part + k, below = (1u << c) - 1u;
+        const bool inner = ((hit & im) >> c) & 1u;
+        const uint64_t m = __ballot(inner);
+        if (inner) W.nodes[top + mbcnt(m)] = tag | (hd.x + (uint32_t)__popc(im & below));
+        top += (uint32_t)__popcll(m);
+        if (leaves[k]) {
+            const bool leaf = ((hit & lm) >> c) & 1u;
+            const uint32_t first = hd.y + (uint32_t)__popc(lm & below) + nibble_sum(hd.z & ((1u << (4u * c)) - 1u));
+            const uint32_t cnt = leaf ? ((hd.z >> (4u * c)) & 15u) + 1u : 0u;
+            uint64_t ml = leaves[k];
+            for (uint32_t i = 0; ml; ml = __ballot(cnt > ++i)) {
+                if (cnt > i) W.leaves[waiting + mbcnt(ml)] = tag | (first + i);
+                waiting += (uint32_t)__popcll(ml);
+            }
+        }
+    }
+    wave_sync();
+    return true;
 }
 
 // What the opacity coin of a ray needs from the lane that owns it.
@@ -728,10 +797,10 @@ struct CoinState {
 // to the lower facet id, so it does not depend on the order or the lanes
 // the tests run on.
 //
-// With at most 8 tasks on the stack (a wave with few rays: a run's tail, or
-// a small run) a node step gives each of them 8 lanes, one for each child:
-// the serial chain of 8 box tests and the loops that push the children
-// shrink to one test and one store a lane.
+// With at most 8 (16) tasks on the stack (a wave with few rays: a run's
+// tail, or a small run) a node step gives each of them 8 (4) lanes, one for
+// each child (two): the serial chain of 8 box tests and the loops that push
+// the children shrink to one or two tests and stores a lane.
 //
 // Bounds. A node step commits the tasks of its first lanes only, as many as
 // leave the stack below its capacity less a reserve and the list within
@@ -753,41 +822,10 @@ __device__ void walk(const TraceParams& P, WaveLds& W, PassLds* pass, const uint
     }
     wave_sync();
     while (top + waiting != 0) {
-        if (top != 0 && top <= 8u && waiting < 64u && P.child_lanes) {
-            const uint32_t c = lane & 7u, below = (1u << c) - 1u;
-            const bool on = (lane >> 3) < top;
-            uint32_t tag = 0, kid = 0, cnt = 0;
-            bool inner = false, leaf = false;
-            if (on) {
-                const uint32_t w = W.nodes[top - 1u - (lane >> 3)], ray = w >> bits, node = w & low;
-                tag = w & ~low;
-                ChildRegs nd;
-                if (node < P.lds_nodes) nd = load_child(lnodes + (size_t)node * 8, c);
-                else nd = load_child(P.nodes + node, c);
-                const float4 a = W.ra[ray], b = W.rb[ray];
-                const uint32_t im = nd.c1.w & 0xffu, lm = nd.c0.w >> 24;
-                if (child_hit(nd, Ray32{a.x, a.y, a.z, b.x, b.y, b.z}, a.w)) {
-                    inner = ((im >> c) & 1u) != 0;
-                    leaf = ((lm >> c) & 1u) != 0;
-                }
-                if (inner) kid = nd.c1.x + (uint32_t)__popc(im & below);
-                if (leaf) {
-                    kid = nd.c1.y + (uint32_t)__popc(lm & below) + nibble_sum(nd.c1.z & ((1u << (4u * c)) - 1u));
-                    cnt = ((nd.c1.z >> (4u * c)) & 15u) + 1u;
-                }
-            }
-            const uint64_t m = __ballot(inner);
-            wave_sync();
-            if (inner) W.nodes[mbcnt(m)] = tag | kid;
-            top = (uint32_t)__popcll(m);
-            for (uint32_t k = 0;; ++k) {
-                const uint64_t ml = __ballot(cnt > k);
-                if (ml == 0) break;
-                if (cnt > k) W.leaves[waiting + mbcnt(ml)] = tag | (kid + k);
-                waiting += (uint32_t)__popcll(ml);
-            }
-            wave_sync();
-        } else if (waiting < 64u && top != 0) {
+        if (top != 0 && top <= 16u && waiting < 64u && P.child_lanes) {
+            if (top <= 8u ? few_nodes<1>(P, W, lnodes, lane, top, waiting) : few_nodes<2>(P, W, lnodes, lane, top, waiting)) continue;
+        }
+        if (waiting < 64u && top != 0) {
             const bool on = lane < top;
             uint32_t tag = 0, inner = 0, im = 0, lm = 0, cw = 0, own = 0;
             int32_t node_base = 0;

@@ -32,7 +32,7 @@ def triangle_soup(n, seed=3):
     return Model(V, np.arange(3 * n).reshape(n, 3).tolist(), F, name="soup")
 
 
-@pytest.mark.parametrize("width,leaf", [(8, 1), (8, 2), (8, 16), (4, 2)])
+@pytest.mark.parametrize("width,leaf", [(8, 1), (8, 2), (8, 3), (8, 16), (4, 2)])
 @pytest.mark.parametrize("n_rays", [1, 63, 65, 140_000])
 def test_overlapping_boxes_first_hits(sim, width, leaf, n_rays):
     m = triangle_soup(1500)
