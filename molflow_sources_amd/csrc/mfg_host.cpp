@@ -1288,6 +1288,27 @@ void breadth_first(std::vector<WideNode>& nodes, std::vector<int32_t>& roots) {
         if (r >= 0) r = idx[(size_t)r];
 }
 
+// Corner code of a triangle's leaf record (mfg_internal.h), or 0 where the
+// record would not give back its corners and 1/|V|^2 bit for bit (it does for
+// every finite triangle: the frame is the corners' bounding rectangle).
+uint32_t corner_code(const double* uv, const DFacet& F) {
+    static_assert(FF_OGMAP < (1u << 24), "the code shares a word with the facet flags");
+    uint32_t code = 0;
+    for (int axis = 0; axis < 2; ++axis) {
+        int zero = -1, one = -1;
+        for (int k = 0; k < 3; ++k) {
+            const double x = uv[2 * k + axis];
+            if (zero < 0 && x == 0.0 && !std::signbit(x)) zero = k;
+            else if (one < 0 && x == 1.0) one = k;
+        }
+        if (zero < 0 || one < 0) return 0;
+        code |= ((uint32_t)zero | ((uint32_t)one << 2)) << (4 * axis);
+    }
+    const double vv = F.V[0] * F.V[0] + F.V[1] * F.V[1] + F.V[2] * F.V[2];
+    const double iv = 1.0 / vv;
+    return std::memcmp(&iv, &F.invV2, sizeof(iv)) == 0 ? code : 0u;
+}
+
 void build_accel(mfg_context* c, int width, int leaf) {
     if (!c->loaded) throw Err(MFG_ERR_STATE, "no model loaded");
     if (width == 0) width = MFG_BVH_WIDTH;
@@ -1366,17 +1387,29 @@ void build_accel(mfg_context* c, int width, int leaf) {
     c->nodes.upload(nodes, s);
     // leaf-ordered copies of the test data (each facet sits in one leaf)
     std::vector<LeafFacet> lf(leafs.size());
-    std::vector<LeafUV> luv(leafs.size());
+    std::vector<LeafUV> luv;   // empty without quadrilaterals
     for (size_t i = 0; i < leafs.size(); ++i) {
         const DFacet& F = c->h_facets.at((size_t)leafs[i]);
         LeafFacet& L = lf[i];
         std::memset(&L, 0, sizeof(L));
-        std::memset(&luv[i], 0, sizeof(LeafUV));
         for (int k = 0; k < 3; ++k) { L.O[k] = F.O[k]; L.N[k] = F.N[k]; L.U[k] = F.U[k]; L.V[k] = F.V[k]; }
-        L.invU2 = F.invU2; L.invV2 = F.invV2;
-        L.id = leafs[i]; L.flags = F.flags; L.poly_off = F.poly_off; L.poly_n = F.poly_n;
-        if (F.poly_n == 3 || F.poly_n == 4)
-            for (uint32_t k = 0; k < 2 * F.poly_n; ++k) luv[i].uv[k] = c->h_poly[2 * (size_t)F.poly_off + k];
+        L.invU2 = F.invU2;
+        L.id = leafs[i]; L.flags = F.flags;
+        const double* uv = &c->h_poly[2 * (size_t)F.poly_off];
+        const uint32_t code = F.poly_n == 3 ? corner_code(uv, F) : 0u;
+        if (code) {
+            L.flags |= code << 24;
+            L.a = uv[2 * (3 - (code & 3u) - ((code >> 2) & 3u))];
+            L.b = uv[2 * (3 - ((code >> 4) & 3u) - (code >> 6)) + 1];
+        } else {
+            const uint64_t at = (uint64_t)F.poly_off | ((uint64_t)F.poly_n << 32);
+            std::memcpy(&L.a, &at, sizeof(at));
+            L.b = F.invV2;
+        }
+        if (F.poly_n == 4) {
+            if (luv.empty()) luv.resize(leafs.size());
+            std::memcpy(luv[i].uv, uv, sizeof(luv[i].uv));
+        }
     }
     c->leaves.upload(lf, s);
     c->leaf_uv.upload(luv, s);

@@ -6,9 +6,9 @@
 //   DPhys[nF_total]       physics and recording parameters, read on a hit
 //   double2 poly[]        normalised (u,v) polygon vertices
 //   BvhNode[]             up to 8-wide nodes, 128 B each, 8-bit quantised boxes
-//   LeafFacet[]           the ray/facet test data in leaf order (128 B) and
-//   LeafUV[]              triangle/quad (u,v) polygons (64 B): a leaf is a
-//                         contiguous run, no index indirection
+//   LeafFacet[]           the ray/facet test data in leaf order (128 B): a
+//                         leaf is a contiguous run, no index indirection
+//   LeafUV[]              quadrilateral (u,v) corners (64 B), leaf order
 //   DVariant[nV]          per-variant bases and settings
 //   tallies               [variant][slot][facet] 64 B counters, textures,
 //                         profiles, ... (layout of include/molflow_gpu.h)
@@ -166,18 +166,29 @@ static_assert(sizeof(BvhNode) == 128, "BvhNode must be 128 bytes");
 // Exact (FP64) ray/facet test data of one leaf entry, stored in leaf order
 // so that a leaf's facets are contiguous (no index indirection). One record
 // is one 128 B line, loaded as eight 16 B loads issued together.
+//
+// A triangle's record is complete: of the three u values of its corners one
+// is 0, one is 1 (the facet's frame is their bounding rectangle) and the same
+// holds for v, so two numbers and which corner has which give all six, in
+// the place of 1/|V|^2 (recomputed, one division) and of the polygon. That
+// spares a second line a test, read after the first.
 struct alignas(128) LeafFacet {
     int32_t id;            // global facet index
-    uint32_t flags;        // FF_* of the facet
-    uint32_t poly_off;     // first (u,v) pair in poly (polygons of > 3 vertices)
-    uint32_t poly_n;
+    uint32_t flags;        // FF_* of the facet (low 24 bits), corner code << 24
     double O[3], N[3], U[3], V[3];
-    double invU2, invV2;
+    double invU2;
+    // triangle (corner code not 0): the u and the v that are not 0 or 1.
+    // Others: first (u,v) pair in poly | vertices << 32 (bits), and 1/|V|^2
+    double a, b;
 };
 static_assert(sizeof(LeafFacet) == 128, "LeafFacet must be one 128 B line");
-// (u,v) of the vertices of a triangle or quadrilateral, parallel to
-// LeafFacet (read only when the ray meets the facet's (u,v) rectangle);
-// larger polygons are read from poly
+// Corner code of a triangle: bits 0-1 the corner with u = 0, 2-3 with u = 1,
+// 4-5 with v = 0, 6-7 with v = 1 (never 0, the two of an axis differ)
+#define MFG_LEAF_FLAGS 0xffffffu
+
+// (u,v) of the corners of a quadrilateral, parallel to LeafFacet in models
+// that have one (read when the ray meets the facet's (u,v) rectangle); larger
+// polygons are read from poly
 struct alignas(64) LeafUV {
     double uv[8];
 };

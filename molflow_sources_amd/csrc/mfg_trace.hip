@@ -276,24 +276,22 @@ __device__ __forceinline__ bool crossing(double ui, double vi, double uj, double
     }
     return false;
 }
+__device__ __forceinline__ bool in_tri(double2 p0, double2 p1, double2 p2, double u, double v) {
+    bool inside = false;
+    if (crossing(p0.x, p0.y, p2.x, p2.y, u, v)) inside = !inside;
+    if (crossing(p1.x, p1.y, p0.x, p0.y, u, v)) inside = !inside;
+    if (crossing(p2.x, p2.y, p1.x, p1.y, u, v)) inside = !inside;
+    return inside;
+}
 // in_poly for a quadrilateral held in registers (n = 4, same order)
-__device__ __forceinline__ bool in_quad(const LeafUV* __restrict__ LU, double u, double v) {
-    const double2* q = reinterpret_cast<const double2*>(LU->uv);
+__device__ __forceinline__ bool in_quad(const double* __restrict__ uv, double u, double v) {
+    const double2* q = reinterpret_cast<const double2*>(uv);
     const double2 p0 = q[0], p1 = q[1], p2 = q[2], p3 = q[3];
     bool inside = false;
     if (crossing(p0.x, p0.y, p3.x, p3.y, u, v)) inside = !inside;
     if (crossing(p1.x, p1.y, p0.x, p0.y, u, v)) inside = !inside;
     if (crossing(p2.x, p2.y, p1.x, p1.y, u, v)) inside = !inside;
     if (crossing(p3.x, p3.y, p2.x, p2.y, u, v)) inside = !inside;
-    return inside;
-}
-__device__ __forceinline__ bool in_tri(const LeafUV* __restrict__ LU, double u, double v) {
-    const double2* q = reinterpret_cast<const double2*>(LU->uv);
-    const double2 p0 = q[0], p1 = q[1], p2 = q[2];
-    bool inside = false;
-    if (crossing(p0.x, p0.y, p2.x, p2.y, u, v)) inside = !inside;
-    if (crossing(p1.x, p1.y, p0.x, p0.y, u, v)) inside = !inside;
-    if (crossing(p2.x, p2.y, p1.x, p1.y, u, v)) inside = !inside;
     return inside;
 }
 
@@ -318,21 +316,27 @@ __device__ __forceinline__ bool facet_test(const DFacet* __restrict__ F, const d
     return in_polygon(poly + 2 * (size_t)F->poly_off, F->poly_n, u, v);
 }
 
+// A triangle's corner k on one axis: 0, 1 or the third value (code: which
+// corner has 0, which has 1).
+__device__ __forceinline__ double corner(uint32_t code, uint32_t k, double other) {
+    return (code & 3u) == k ? 0.0 : ((code >> 2) & 3u) == k ? 1.0 : other;
+}
+
 // facet_test on a leaf record: the same operations in the same order. The
 // record's 128 B are loaded together before the first decision (one round
-// trip); the (u,v) polygon of a triangle or quadrilateral is fetched only
-// when the ray meets the facet's rectangle.
+// trip); polygons of 4 and more corners are read only when the ray meets the
+// facet's rectangle.
 __device__ __forceinline__ bool leaf_test(const LeafFacet* __restrict__ L, const LeafUV* __restrict__ LU,
-                                          const double* __restrict__ poly, d3 P, d3 D, int32_t skip, double& t,
-                                          double& u, double& v, int32_t& id, uint32_t& flags) {
+                                          const double* __restrict__ poly, d3 P, d3 D, int32_t skip, double& t, double& u, double& v, int32_t& id, uint32_t& flags) {
     const uint4 hd = reinterpret_cast<const uint4*>(L)[0];
     const double2* q = reinterpret_cast<const double2*>(L);
     const double2 q1 = q[1], q2 = q[2], q3 = q[3], q4 = q[4], q5 = q[5], q6 = q[6], q7 = q[7];
     id = (int32_t)hd.x;
-    flags = hd.y;
-    const d3 O = mk(q1.x, q1.y, q2.x), N = mk(q2.y, q3.x, q3.y);
-    const d3 U = mk(q4.x, q4.y, q5.x), V = mk(q5.y, q6.x, q6.y);
-    const double iu = q7.x, iv = q7.y;
+    flags = hd.y & MFG_LEAF_FLAGS;
+    const uint32_t code = hd.y >> 24;
+    const d3 O = mk(__longlong_as_double((long long)(((unsigned long long)hd.w << 32) | hd.z)), q1.x, q1.y);
+    const d3 N = mk(q2.x, q2.y, q3.x), U = mk(q3.y, q4.x, q4.y), V = mk(q5.x, q5.y, q6.x);
+    const double iu = q6.y, iv = code ? 1.0 / dot(V, V) : q7.y;
     double denom = fdot(N, D);
     d3 w = sub(O, P);
     t = fdot(N, w) / denom;
@@ -340,14 +344,20 @@ __device__ __forceinline__ bool leaf_test(const LeafFacet* __restrict__ L, const
     d3 r = sub(X, O);
     u = fdot(r, U) * iu;
     v = fdot(r, V) * iv;
-    const uint32_t n = hd.w;
     // non-short-circuit: every operand (the whole record) is needed here
     bool ok = (denom != 0.0) & (((flags & FF_2SIDED) != 0u) | !(denom > 0.0)) & (t > 0.0) &
-              !((u < 0.0) | (u > 1.0) | (v < 0.0) | (v > 1.0)) & (id != skip) & (n >= 3u) & (hd.z != ~0u);
+              !((u < 0.0) | (u > 1.0) | (v < 0.0) | (v > 1.0)) & (id != skip);
     if (!ok) return false;
-    if (n == 3) return in_tri(LU, u, v);
-    if (n == 4) return in_quad(LU, u, v);
-    return in_poly_slabs(poly + 2 * (size_t)hd.z, n, u, v);
+    if (code) {
+        const uint32_t cv = code >> 4;
+        return in_tri(make_double2(corner(code, 0, q7.x), corner(cv, 0, q7.y)),
+                      make_double2(corner(code, 1, q7.x), corner(cv, 1, q7.y)),
+                      make_double2(corner(code, 2, q7.x), corner(cv, 2, q7.y)), u, v);
+    }
+    const unsigned long long at = (unsigned long long)__double_as_longlong(q7.x);
+    const double* p = poly + 2 * (size_t)(uint32_t)at;
+    const uint32_t n = (uint32_t)(at >> 32);
+    return n == 4u ? in_quad(LU->uv, u, v) : in_polygon(p, n, u, v);
 }
 
 struct Ray32 { float ox, oy, oz, ix, iy, iz; };
