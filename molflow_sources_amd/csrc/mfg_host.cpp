@@ -1484,7 +1484,9 @@ int default_waves(uint32_t feats) {
     return (k & FEAT_ADJOINT) ? 1 : 2;
 }
 
-void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& waves) {
+// items: particles the launch will trace. share: blocks of 256 lanes among
+// which a CU's LDS is split.
+void launch_shape(mfg_context* c, uint32_t feats, uint64_t items, int& grid, int& block, int& waves, int& share) {
     block = (int)c->block;
     waves = c->waves ? c->waves : default_waves(feats);
     if (block > 256) {
@@ -1494,16 +1496,25 @@ void launch_shape(mfg_context* c, uint32_t feats, int& grid, int& block, int& wa
         if (mfg_trace_has_cu_block(feats, c->dvars.size() == 1, block)) waves = block / 256;
         else block = 256;
     }
+    share = waves;
+    // up to 8 particles for each wave of a single block per CU (as many rays
+    // as a node step can give 8 lanes each): more waves would not shorten the
+    // longest of them, and one block a CU gets the whole LDS for the top of
+    // the tree. 1000 tube particles 1.00 -> 0.79 ms, 8000 0.99 -> 0.82, 3000
+    // low-flux ones 49.8 -> 46.2; from 12 a wave on low flux is slower (62 ->
+    // 66 ms at 1.2e4)
+    const bool thin = items <= (uint64_t)c->n_cu * 32 && block == 256 && c->waves == 0 && c->blocks_per_cu == 0;
+    if (thin) share = 1;
     auto lds_bytes = [&](int b) {
         return (size_t)(b / 64) * mfg_wave_lds(feats) + c->hot_bytes() +
-               (size_t)lds_node_count(c, feats, b, waves) * sizeof(BvhNode);
+               (size_t)lds_node_count(c, feats, b, share) * sizeof(BvhNode);
     };
     if (block > 256 && mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block)) < 1) {
         block = 256;   // the block's LDS does not fit
-        waves = c->waves ? c->waves : default_waves(feats);
+        share = waves = c->waves ? c->waves : default_waves(feats);
     }
     uint32_t per_cu = c->blocks_per_cu;
-    if (block > 256) per_cu = 1;
+    if (block > 256 || thin) per_cu = 1;
     if (per_cu == 0) {
         // fill every CU to its occupancy limit (persistent launch)
         int occ = mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block));
@@ -1550,8 +1561,8 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     uint32_t feats = c->features;
     if (c->trace_n) feats |= FEAT_TRACE;
     if (c->adj_groups) feats |= FEAT_ADJOINT;
-    int grid, block, waves;
-    launch_shape(c, feats, grid, block, waves);
+    int grid, block, waves, share;
+    launch_shape(c, feats, total + c->in_flight, grid, block, waves, share);
     if (c->adj_groups) {
         if (c->carry_on || c->in_flight) throw Err(MFG_ERR_STATE, "the adjoint traces every particle to its end: disable carry and drain first");
         if (!c->adj_s_ok)
@@ -1569,7 +1580,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     hipStream_t s = c->stream;
     *c->stop_host = 0;
     TraceParams p = make_params(c, total, max_events);
-    p.lds_nodes = lds_node_count(c, feats, block, waves);
+    p.lds_nodes = lds_node_count(c, feats, block, share);
     // lanes of a wave that take particles: all once there is one for every
     // lane, else the items are spread over all waves, whose other lanes then
     // help with the walks (a wave's step gets shorter the fewer rays it has:
@@ -2295,8 +2306,8 @@ int mfg_autotune(mfg_context* c, uint64_t n_probe, mfg_tune_result* out) {
                     double hs = sr.kernel_ms > 0 ? (double)sr.hits / (sr.kernel_ms * 1e-3) : 0.0;
                     if (hs > best) {
                         best = hs;
-                        int grid, block, waves;
-                        launch_shape(c, feats, grid, block, waves);
+                        int grid, block, waves, share;
+                        launch_shape(c, feats, n_probe, grid, block, waves, share);
                         r.waves = (uint32_t)waves; r.block = (uint32_t)block; r.blocks_per_cu = (uint32_t)(grid / c->n_cu);
                         r.hits_per_s = hs; r.bvh_width = (uint32_t)width; r.leaf_size = (uint32_t)leaf;
                     }

@@ -48,10 +48,11 @@ def test_overlapping_boxes_first_hits(sim, width, leaf, n_rays):
         assert np.allclose(a[hit], b[hit], rtol=1e-12, atol=1e-12)
 
 
-@pytest.mark.parametrize("n_des", [1, 64, 3071, 3073, 200_001])
+@pytest.mark.parametrize("n_des", [1, 64, 1025, 8192, 8193, 200_001])
 def test_lane_quota_same_seed_tallies(sim, n_des):
-    """Runs of fewer particles than waves, of about one per wave and of more
-    than lanes (lane quota 1, 1, 2, 64) count what the oracle counts."""
+    """Runs of fewer particles than waves, of a few per wave of one block per
+    CU, just beyond that, and of more than lanes (lane quota 1, 1, 2, 8, 3,
+    64) count what the oracle counts."""
     m = geometry.tube_model(1.0, 3.0, 16, 6)
     sim.load(m)
     sim.rebuild_accel()
