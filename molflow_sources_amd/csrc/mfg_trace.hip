@@ -295,37 +295,17 @@ __device__ __forceinline__ bool in_quad(const double* __restrict__ uv, double u,
     return inside;
 }
 
-// Ray/facet test; the same arithmetic, operation for operation, as the CPU
-// restatement (explicit fma dot products, contraction off elsewhere).
-__device__ __forceinline__ bool facet_test(const DFacet* __restrict__ F, const double* __restrict__ poly, d3 P, d3 D,
-                                           double& t, double& u, double& v) {
-    d3 N = ld3(F->N);
-    double denom = fdot(N, D);
-    uint32_t flags = F->flags;
-    if (denom == 0.0) return false;
-    if (!(flags & FF_2SIDED) && denom > 0.0) return false;
-    d3 O = ld3(F->O);
-    d3 w = sub(O, P);
-    t = fdot(N, w) / denom;
-    if (!(t > 0.0)) return false;
-    d3 X = mk(fma(t, D.x, P.x), fma(t, D.y, P.y), fma(t, D.z, P.z));
-    d3 r = sub(X, O);
-    u = fdot(r, ld3(F->U)) * F->invU2;
-    v = fdot(r, ld3(F->V)) * F->invV2;
-    if (u < 0.0 || u > 1.0 || v < 0.0 || v > 1.0) return false;
-    return in_polygon(poly + 2 * (size_t)F->poly_off, F->poly_n, u, v);
-}
-
 // A triangle's corner k on one axis: 0, 1 or the third value (code: which
 // corner has 0, which has 1).
 __device__ __forceinline__ double corner(uint32_t code, uint32_t k, double other) {
     return (code & 3u) == k ? 0.0 : ((code >> 2) & 3u) == k ? 1.0 : other;
 }
 
-// facet_test on a leaf record: the same operations in the same order. The
-// record's 128 B are loaded together before the first decision (one round
-// trip); polygons of 4 and more corners are read only when the ray meets the
-// facet's rectangle.
+// Ray/facet test on a leaf record; the same arithmetic, operation for
+// operation, as the CPU restatement (explicit fma dot products, contraction
+// off elsewhere). The record's 128 B are loaded together before the first
+// decision (one round trip); polygons of 4 and more corners are read only
+// when the ray meets the facet's rectangle.
 __device__ __forceinline__ bool leaf_test(const LeafFacet* __restrict__ L, const LeafUV* __restrict__ LU,
                                           const double* __restrict__ poly, d3 P, d3 D, int32_t skip, double& t, double& u, double& v, int32_t& id, uint32_t& flags) {
     const uint4 hd = reinterpret_cast<const uint4*>(L)[0];
@@ -475,7 +455,7 @@ __device__ __forceinline__ float widen(double t) {
     return (float)t * 1.000004f + 1e-30f;
 }
 
-struct HitRec { int32_t facet; double t, u, v; };
+struct HitRec { int32_t facet; double t; };
 
 // ---------------------------------------------------------------- DES_ANGLEMAP
 // Sampling of a recorded incident-angle map (AnglemapGeneration.cpp:15-410),
@@ -955,7 +935,7 @@ __device__ __forceinline__ void walk_load(WaveLds& W, uint32_t lane, d3 p, d3 d,
     W.facet[lane] = -1;
 }
 
-// (u,v) of a hit at distance t on a facet: the operations of facet_test.
+// (u,v) of a hit at distance t on a facet: the operations of leaf_test.
 __device__ __forceinline__ void hit_uv(const DFacet* __restrict__ F, d3 P, d3 D, double t, double& u, double& v) {
     d3 X = mk(fma(t, D.x, P.x), fma(t, D.y, P.y), fma(t, D.z, P.z));
     d3 r = sub(X, ld3(F->O));
@@ -1903,7 +1883,7 @@ struct Tracer {
         const double2 a = W.p01[lane], b = W.p2d0[lane], c = W.d12[lane];
         pos = mk(a.x, a.y, b.x);
         dir = mk(b.y, c.x, c.y);
-        const HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane]), 0.0, 0.0};
+        const HitRec h{W.facet[lane], __longlong_as_double((long long)W.t[lane])};
         W.t[lane] = ~0ull;   // now the texture cell of the event
         return h;
     }
