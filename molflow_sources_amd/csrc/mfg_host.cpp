@@ -895,7 +895,8 @@ struct mfg_context {
     DevBuf<DPhys> phys;
     DevBuf<DHit> hits;                   // derived from facets and phys (upload_phys)
     DevBuf<double> poly, src_cum, og_cdf, tab_x, tab_y, mom_start, mom_end, tex_inc, am_src;
-    DevBuf<int32_t> src_facet, roots;
+    DevBuf<int32_t> src_facet;
+    DevBuf<Root> roots;
     DevBuf<LeafFacet> leaves;
     DevBuf<LeafUV> leaf_uv;
     std::vector<DPhys> h_phys;           // host copy of the uploaded physics records
@@ -981,7 +982,7 @@ struct mfg_context {
     // staging array of mfg_intersect_batch_static: the device address of
     // the library's static `scratch` array on this context's device
     StaticRays* scratch = nullptr;
-    std::vector<int32_t> h_roots;        // host copy of the BVH roots
+    std::vector<Root> h_roots;           // host copy of the BVH roots
 };
 
 namespace {
@@ -1315,8 +1316,7 @@ void build_accel(mfg_context* c, int width, int leaf) {
     if (width != 4 && width != 8) throw Err(MFG_ERR_INVALID, "BVH width must be 4 or 8 (0 = 8)");
     c->bvh_width = width;
     if (leaf <= 0) leaf = 2;
-    // a traversal stack entry holds a leaf as 27 bits of first record and
-    // 4 bits of facet count
+    // a node holds a leaf's facet count in 4 bits
     if (leaf > 16) throw Err(MFG_ERR_INVALID, "leaf size above 16");
     c->leaf_size = leaf;
     size_t nv = c->models.size();
@@ -1359,7 +1359,8 @@ void build_accel(mfg_context* c, int width, int leaf) {
     for (auto& e : errors) if (!e.empty()) throw Err(MFG_ERR_INVALID, e);
     // concatenate with global node / leaf offsets
     std::vector<BvhNode> nodes;
-    std::vector<int32_t> leafs, roots;
+    std::vector<int32_t> leafs;
+    std::vector<Root> roots;
     int depth = 0;
     for (size_t vi = 0; vi < nv; ++vi) {
         int32_t nb = (int32_t)nodes.size(), lb = (int32_t)leafs.size();
@@ -1372,7 +1373,13 @@ void build_accel(mfg_context* c, int width, int leaf) {
         }
         leafs.insert(leafs.end(), vleaf[vi].begin(), vleaf[vi].end());
         c->dvars[vi].root_base = (uint32_t)roots.size();
-        for (int32_t r : vroots[vi]) roots.push_back(r < 0 ? -1 : r + nb);
+        for (int32_t r : vroots[vi]) {
+            if (r < 0) { roots.push_back({-1, 0u}); continue; }
+            const uint32_t node = (uint32_t)(r + nb);
+            const BvhNode& n = nodes[node];
+            const uint32_t kids = (uint32_t)__builtin_popcount(n.inner_mask);
+            roots.push_back({(int32_t)node, n.leaf_mask || !kids ? (node << 4) | 1u : ((uint32_t)n.node_base << 4) | kids});
+        }
         depth = std::max(depth, vdepth[vi]);
     }
     // stack entries: a walk pushes at most width-1 per level
@@ -1441,7 +1448,7 @@ uint32_t lds_node_count(const mfg_context* c, uint32_t feats, int block, int wav
 TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     TraceParams p{};
     p.one = c->dvars[0];
-    p.one_root = c->dvars.size() == 1 && c->dvars[0].n_struct == 1 ? c->h_roots.at(c->dvars[0].root_base) : -2;
+    p.one_root = c->dvars.size() == 1 && c->dvars[0].n_struct == 1 ? c->h_roots.at(c->dvars[0].root_base) : Root{-2, 0u};
     p.hits = c->hits.p;
     p.facets = c->facets.p; p.phys = c->phys.p; p.poly = c->poly.p; p.nodes = c->nodes.p;
     p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p; p.roots = c->roots.p; p.variants = c->variants.p;

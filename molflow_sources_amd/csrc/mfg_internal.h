@@ -229,6 +229,14 @@ struct alignas(16) PassLds {
     uint32_t rec[64][MFG_PASSES];      // facet records
 };
 
+// Where the rays of a structure start: its root node (-1: no facets), and
+// the nodes a wave with few rays starts from, first << 4 | how many: the
+// root's children if none of them is a leaf, else the root.
+struct Root {
+    int32_t node;
+    uint32_t first;
+};
+
 // global counters of one variant (mfg_global_counters)
 struct DGlobal {
     unsigned long long nb_mc_hit;
@@ -304,7 +312,7 @@ struct TraceParams {
     // read as scalars; seed and pid_base change between replays of a captured
     // launch and are read from `variants`
     DVariant one;
-    int32_t one_root;                 // root of its only structure, or -2: look it up
+    Root one_root;                    // root of its only structure; node -2: look it up
     const DHit* hits;
     const DFacet* facets;
     const DPhys* phys;
@@ -312,7 +320,7 @@ struct TraceParams {
     const BvhNode* nodes;
     const LeafFacet* leaves;
     const LeafUV* leaf_uv;
-    const int32_t* roots;             // per (variant, structure): root node or -1
+    const Root* roots;                // per (variant, structure)
     const DVariant* variants;
     const uint64_t* var_prefix;       // n_variants+1 prefix of this run's desorptions
     uint32_t n_variants;
@@ -408,7 +416,7 @@ struct IsectParams {
     const BvhNode* nodes;
     const LeafFacet* leaves;
     const LeafUV* leaf_uv;
-    int32_t root;
+    Root root;
     uint32_t task_bits, child_lanes;
     uint32_t rays_per_wave;
     uint64_t n;

@@ -792,6 +792,14 @@ struct CoinState {
 // each child (two): the serial chain of 8 box tests and the loops that push
 // the children shrink to one or two tests and stores a lane.
 //
+// A wave with at most kSeedRays rays starts them at the children of their
+// roots (Root::first): the step that tests a root's 8 boxes for one ray has 8
+// of 64 lanes at work, and the next one has lanes for all 8 children anyway.
+// 16 variants 137.9 -> 131.2 ms, 5k-facet pipe 25.6 -> 25.0, 1000 tube
+// particles 0.80 -> 0.77 ms; with up
+// to 8 rays (a full node step) 134.6 and 0.79, with 16 138 and low flux 73.8
+// -> 81.4.
+//
 // Bounds. A node step commits the tasks of its first lanes only, as many as
 // leave the stack below its capacity less a reserve and the list within
 // its capacity; the other tasks stay where they are. Lane 0 (the topmost
@@ -799,16 +807,26 @@ struct CoinState {
 // first, which adds at most width - 1 entries a level: the reserve holds
 // that for the deepest tree the host accepts. The list has room for lane
 // 0's facets (8 leaves of 16) whenever a node step runs (below 64 waiting).
+constexpr uint32_t kSeedRays = 2;
 template <bool TRANSP>
-__device__ void walk(const TraceParams& P, WaveLds& W, PassLds* pass, const uint4* lnodes, uint32_t lane, bool live, int32_t root,
+__device__ void walk(const TraceParams& P, WaveLds& W, PassLds* pass, const uint4* lnodes, uint32_t lane, bool live, Root root,
                      const CoinState& cs) {
     const uint32_t bits = P.task_bits, low = (1u << bits) - 1u;
     uint32_t top, waiting = 0;   // wave-uniform
     {
-        const bool on = live && root >= 0;
-        const uint64_t m = __ballot(on);
+        const bool on = live && root.node >= 0;
+        uint64_t m = __ballot(on);
         top = (uint32_t)__popcll(m);
-        if (on) W.nodes[mbcnt(m)] = (lane << bits) | (uint32_t)root;
+        if (top <= kSeedRays) {
+            for (top = 0; m; m &= m - 1ull) {
+                const uint32_t ray = (uint32_t)__builtin_ctzll(m);
+                const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)root.first, (int)ray);
+                if (lane < (s & 15u)) W.nodes[top + lane] = (ray << bits) | ((s >> 4) + lane);
+                top += s & 15u;
+            }
+        } else if (on) {
+            W.nodes[mbcnt(m)] = (lane << bits) | (uint32_t)root.node;
+        }
     }
     wave_sync();
     while (top + waiting != 0) {
@@ -1861,15 +1879,15 @@ struct Tracer {
         acc_hit_equiv = acc_abs_equiv = acc_dist_total = acc_dist_full = 0.0;
     }
 
-    MFG_IN int32_t find_root() const {
-        if constexpr (ONE) { if (P.one_root != -2) return P.one_root; }
+    MFG_IN Root find_root() const {
+        if constexpr (ONE) { if (P.one_root.node != -2) return P.one_root; }
         return P.roots[vc().root_base + (uint32_t)structure];
     }
     // One event of an alive particle (one SimulationMCStep iteration): its
     // ray goes into the wave's walk, which all lanes run together (also
     // those without a particle), then finish() treats what it met.
     MFG_IN HitRec trace_ray(uint32_t lane, bool alive) {
-        int32_t root = -1;
+        Root root{-1, 0u};
         if (alive) {
             if constexpr (CLOCKED) ++nb_events;
             root = find_root();
@@ -1935,7 +1953,7 @@ struct Tracer {
                         transparent_pass(f, t);
                     }
                 } else if (n_pass != 0) {
-                    const int32_t root = find_root();
+                    const int32_t root = find_root().node;
                     const LaneStack S{W.nodes + lane, MFG_LANE_STACK, P.stack_total, spill};
                     Ray32 r = make_ray32(pos, dir);
                     float tbf = widen(travel);
@@ -2369,9 +2387,10 @@ __global__ void __launch_bounds__(256 * WAVES, WAVES) k_trace_cu(TraceParams P) 
 }
 
 // Parked particles that a launch did not claim: the launch deals out items
-// [0, dealt), its queue hands out the `claimed` next ones, and the first n_in of them are the resumed particles, so
-// [min(dealt + claimed, n_in), n_in) were never taken. That happens only when the
-// launch time limit stops the claims (a dry queue means every item was
+// [0, dealt), its queue hands out the `claimed` next ones, and the first
+// n_in of all items are the resumed particles, so
+// [min(dealt + claimed, n_in), n_in) were never taken. That happens only
+// when the launch time limit stops the claims (a dry queue means every item was
 // claimed). These records are appended to the output half after the ones
 // the waves parked themselves.
 __device__ __forceinline__ void carry_counts(const unsigned long long* ctl, const unsigned long long* claimed, uint64_t dealt,

@@ -48,6 +48,26 @@ def test_overlapping_boxes_first_hits(sim, width, leaf, n_rays):
         assert np.allclose(a[hit], b[hit], rtol=1e-12, atol=1e-12)
 
 
+@pytest.mark.parametrize("n_facets", [1, 2, 8, 9, 12, 64, 1500])
+@pytest.mark.parametrize("n_rays", [1, 2, 3])
+def test_few_rays_first_hits(sim, n_facets, n_rays):
+    """Waves of one and two rays, which start at the children of the root,
+    and of three, on trees whose root is a leaf's parent only, has leaves
+    beside inner children, and has inner children only."""
+    m = triangle_soup(n_facets)
+    cpu = CpuModel(m)
+    sim.load(m)
+    o, d = random_rays(40 * n_rays, [-1] * 3, [11] * 3, seed=7)
+    last = np.random.default_rng(8).integers(-1, m.n_facets, len(o)).astype(np.int32)
+    ref = cpu.intersect(o, d, last, brute=True)
+    for width, leaf in ((8, 1), (4, 2)):
+        sim.rebuild_accel(width, leaf)
+        for i in range(0, len(o), n_rays):
+            got = sim.intersect(o[i:i + n_rays], d[i:i + n_rays], last[i:i + n_rays])
+            assert np.array_equal(got[0], ref[0][i:i + n_rays]), f"rays from {i}"
+            assert np.allclose(got[1], np.where(got[0] >= 0, ref[1][i:i + n_rays], got[1]), rtol=1e-12, atol=1e-12)
+
+
 @pytest.mark.parametrize("n_des", [1, 64, 1025, 8192, 8193, 200_001])
 def test_lane_quota_same_seed_tallies(sim, n_des):
     """Runs of fewer particles than waves, of a few per wave of one block per
