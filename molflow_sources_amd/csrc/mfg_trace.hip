@@ -796,9 +796,8 @@ struct CoinState {
 // roots (Root::first): the step that tests a root's 8 boxes for one ray has 8
 // of 64 lanes at work, and the next one has lanes for all 8 children anyway.
 // 16 variants 137.9 -> 131.2 ms, 5k-facet pipe 25.6 -> 25.0, 1000 tube
-// particles 0.80 -> 0.77 ms; with up
-// to 8 rays (a full node step) 134.6 and 0.79, with 16 138 and low flux 73.8
-// -> 81.4.
+// particles 0.80 -> 0.77; with up to 8 rays (a full node step) 134.6, 25.7
+// and 0.79, with 16 138 and low flux 73.8 -> 81.4.
 //
 // Bounds. A node step commits the tasks of its first lanes only, as many as
 // leave the stack below its capacity less a reserve and the list within
