@@ -888,7 +888,8 @@ struct mfg_context {
     uint32_t stack_size = 0;             // traversal stack entries a walk may need
     DevBuf<int32_t> stack_spill;         // per-lane entries beyond the LDS part (transparent models)
     uint32_t task_bits = 26;             // bits of a node or leaf record index in a walk task
-    int bvh_width = MFG_BVH_WIDTH, leaf_size = 2;   // children per BVH node, facets per leaf
+    int bvh_width = MFG_BVH_WIDTH, leaf_size = 2;   // children per BVH node, facets per leaf asked for
+    uint32_t leaf_most = 0;              // facets of the largest leaf on the device
     size_t lds_per_block = 65536;        // the device's LDS limit for one block
     // device data
     DevBuf<DFacet> facets;
@@ -1310,15 +1311,17 @@ uint32_t corner_code(const double* uv, const DFacet& F) {
     return std::memcmp(&iv, &F.invV2, sizeof(iv)) == 0 ? code : 0u;
 }
 
+// Builds the tree and puts it on the device. Nothing of the context changes
+// before the new tree has passed every check, so after a refusal (too deep,
+// a limit) the previous tree stays in use with its own parameters; from the
+// first upload on there is no tree until the last one is done.
 void build_accel(mfg_context* c, int width, int leaf) {
     if (!c->loaded) throw Err(MFG_ERR_STATE, "no model loaded");
     if (width == 0) width = MFG_BVH_WIDTH;
     if (width != 4 && width != 8) throw Err(MFG_ERR_INVALID, "BVH width must be 4 or 8 (0 = 8)");
-    c->bvh_width = width;
     if (leaf <= 0) leaf = 2;
     // a node holds a leaf's facet count in 4 bits
     if (leaf > 16) throw Err(MFG_ERR_INVALID, "leaf size above 16");
-    c->leaf_size = leaf;
     size_t nv = c->models.size();
     std::vector<std::vector<WideNode>> vnodes(nv);
     std::vector<std::vector<int32_t>> vleaf(nv), vroots(nv);
@@ -1361,6 +1364,8 @@ void build_accel(mfg_context* c, int width, int leaf) {
     std::vector<BvhNode> nodes;
     std::vector<int32_t> leafs;
     std::vector<Root> roots;
+    std::vector<uint32_t> root_base(nv);
+    uint32_t leaf_most = 0;
     int depth = 0;
     for (size_t vi = 0; vi < nv; ++vi) {
         int32_t nb = (int32_t)nodes.size(), lb = (int32_t)leafs.size();
@@ -1368,11 +1373,12 @@ void build_accel(mfg_context* c, int width, int leaf) {
             for (int k = 0; k < 8; ++k) {
                 if (!(nd.valid & (1u << k))) continue;
                 nd.child[k] += (nd.leaf_mask & (1u << k)) ? lb : nb;
+                if (nd.leaf_mask & (1u << k)) leaf_most = std::max<uint32_t>(leaf_most, nd.count[k]);
             }
             nodes.push_back(pack_node(nd));
         }
         leafs.insert(leafs.end(), vleaf[vi].begin(), vleaf[vi].end());
-        c->dvars[vi].root_base = (uint32_t)roots.size();
+        root_base[vi] = (uint32_t)roots.size();
         for (int32_t r : vroots[vi]) {
             if (r < 0) { roots.push_back({-1, 0u}); continue; }
             const uint32_t node = (uint32_t)(r + nb);
@@ -1382,16 +1388,13 @@ void build_accel(mfg_context* c, int width, int leaf) {
         }
         depth = std::max(depth, vdepth[vi]);
     }
-    // stack entries: a walk pushes at most width-1 per level
+    // (ray, node) tasks: a depth-first walk adds at most width-1 per level
     uint32_t need = (uint32_t)((width - 1) * depth + width);
-    if (need > MFG_MAX_STACK) throw Err(MFG_ERR_LIMIT, "BVH too deep for the LDS traversal stack (depth " + std::to_string(depth) + ")");
-    c->stack_size = need;
+    if (need > MFG_MAX_STACK) throw Err(MFG_ERR_LIMIT, "BVH too deep for the walk's task stack (depth " + std::to_string(depth) + ")");
     // a walk task packs its ray above the index of its node or record
-    c->task_bits = 26;
-    while (c->task_bits < 31 && std::max(nodes.size(), leafs.size()) > ((size_t)1 << c->task_bits)) ++c->task_bits;
+    uint32_t task_bits = 26;
+    while (task_bits < 31 && std::max(nodes.size(), leafs.size()) > ((size_t)1 << task_bits)) ++task_bits;
     if (leafs.size() >= ((size_t)1 << 27)) throw Err(MFG_ERR_LIMIT, "more than 2^27 BVH leaf records");
-    hipStream_t s = c->stream;
-    c->nodes.upload(nodes, s);
     // leaf-ordered copies of the test data (each facet sits in one leaf)
     std::vector<LeafFacet> lf(leafs.size());
     std::vector<LeafUV> luv;   // empty without quadrilaterals
@@ -1418,13 +1421,22 @@ void build_accel(mfg_context* c, int width, int leaf) {
             std::memcpy(luv[i].uv, uv, sizeof(luv[i].uv));
         }
     }
+    hipStream_t s = c->stream;
+    c->accel = false;
+    reset_graph(c);
+    c->nodes.upload(nodes, s);
     c->leaves.upload(lf, s);
     c->leaf_uv.upload(luv, s);
     c->roots.upload(roots, s);
-    c->h_roots = roots;
     HIPCHK(hipStreamSynchronize(s));
+    c->h_roots = std::move(roots);
+    for (size_t vi = 0; vi < nv; ++vi) c->dvars[vi].root_base = root_base[vi];
+    c->bvh_width = width;
+    c->leaf_size = leaf;
+    c->leaf_most = leaf_most;
+    c->stack_size = need;
+    c->task_bits = task_bits;
     c->accel = true;
-    reset_graph(c);
 }
 
 // LDS is allocated in units of 1280 B on gfx950; the occupancy query does
@@ -1453,7 +1465,7 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
     p.facets = c->facets.p; p.phys = c->phys.p; p.poly = c->poly.p; p.nodes = c->nodes.p;
     p.leaves = c->leaves.p; p.leaf_uv = c->leaf_uv.p; p.roots = c->roots.p; p.variants = c->variants.p;
     p.var_prefix = c->prefix.p; p.n_variants = (uint32_t)c->dvars.size();
-    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3 ? (uint32_t)c->leaf_size : 0u;
+    p.task_bits = c->task_bits; p.child_lanes = c->leaf_most <= 3 ? c->leaf_most : 0u;
     p.stack_total = c->stack_size;
     p.stack_spill = p.stack_total > MFG_LANE_STACK ? c->stack_spill.p : nullptr;
     p.src_cum = c->src_cum.p; p.src_facet = c->src_facet.p; p.og_cdf = c->og_cdf.p; p.am_src = c->am_src.p;
@@ -1908,7 +1920,7 @@ void launch_batch(mfg_context* c, uint64_t n, const double* dO, const double* dD
     // share their walks)
     const uint64_t spread = n / ((uint64_t)c->n_cu * 8), cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
     p.rays_per_wave = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(8, spread));
-    p.task_bits = c->task_bits; p.child_lanes = c->leaf_size <= 3 ? (uint32_t)c->leaf_size : 0u; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
+    p.task_bits = c->task_bits; p.child_lanes = c->leaf_most <= 3 ? c->leaf_most : 0u; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
     p.out_facet = dF; p.out_t = dT; p.out_u = dU; p.out_v = dV; p.facet_base = c->dvars[0].facet_base;
     if (mfg_launch_intersect(p, c->stream)) throw Err(MFG_ERR_DEVICE, "intersect launch failed");
 }
