@@ -345,7 +345,10 @@ struct Ray32 { float ox, oy, oz, ix, iy, iz; };
 __device__ __forceinline__ float safe_inv(double d) {
     float f = (float)d;
     if (fabsf(f) < 1e-30f) f = (f < 0.0f) ? -1e-30f : 1e-30f;
-    return __builtin_amdgcn_rcpf(f);   // within 1 ulp, as the boxes' padding allows
+    // correctly rounded: of 6 million rays from 500 to 900 model extents away
+    // 105 lost their first hit with v_rcp_f32 (1 ulp) and not with this
+    // division, 69 the other way round
+    return 1.0f / f;
 }
 
 __device__ __forceinline__ Ray32 make_ray32(d3 P, d3 D) {
@@ -419,7 +422,10 @@ __device__ __forceinline__ uint32_t word_of(const uint4& v, uint32_t i) {
 // the unpadded box spends at least 1e-5 extent / |d| of its parameter
 // inside the padded one (within [0, tmax] as well, since tmax is at or
 // beyond that hit), against FP32 errors near 1e-7 extent / |d|, so no
-// tolerance is added to a <= b.
+// tolerance is added to a <= b. The errors grow with the distance R of the
+// ray's origin, to about 3e-7 R / |d| (five roundings), so this holds up to
+// R of some 30 extents; farther out a hit near a box's edge can be lost (1 of
+// 200,000 at 320 extents).
 __device__ __forceinline__ uint32_t node_hits(const NodeRegs& n, const Ray32& r, float tmax) {
     const float ox = __uint_as_float(n.c0.x), oy = __uint_as_float(n.c0.y), oz = __uint_as_float(n.c0.z);
     const uint32_t ew = n.c0.w;
