@@ -1608,6 +1608,17 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     const uint64_t n_waves = (uint64_t)grid * (uint64_t)(block / 64);
     const uint64_t cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
     p.lane_quota = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cap, (total + c->in_flight + n_waves - 1) / n_waves));
+    p.refill_at = std::min<uint32_t>(p.lane_quota, MFG_REFILL);
+    if (c->carry_on) {
+        // A run that parks what is left ends when every wave has found the
+        // queue empty, which a wave looks up when lanes of it are free. With
+        // the particles spread, a wave's few would all have to end first:
+        // the waves are filled, and the first free lane looks where nothing
+        // is left to take after the first deal, or where fewer particles are
+        // new than lanes would end in waiting for several.
+        p.lane_quota = (uint32_t)cap;
+        p.refill_at = total < MFG_REFILL * n_waves || total + c->in_flight <= n_waves * cap ? 1u : MFG_REFILL;
+    }
     p.dealt = n_waves * p.lane_quota;
     std::vector<uint64_t> key(n_des, n_des + nv);
     key.push_back(max_events); key.push_back(feats); key.push_back((uint64_t)grid); key.push_back(block);
@@ -1615,6 +1626,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     key.push_back((uint64_t)(uintptr_t)p.carry); key.push_back(p.carry_keep);
     key.push_back((uint64_t)(uintptr_t)p.hot_fc); key.push_back(p.n_hot); key.push_back(p.time_limit);
     key.push_back(p.lds_nodes); key.push_back(p.lane_quota);
+    key.push_back(p.refill_at);
     // the events bracket the trace kernel alone (eager path) or the whole
     // graph (replay path)
     auto enqueue = [&](bool events) {

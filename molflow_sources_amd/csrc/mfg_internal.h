@@ -25,6 +25,8 @@
 #define MFG_WALK_LEAVES 256      // (ray, facet record) tasks waiting: below 64 plus one node's 8 leaves of 16
 static_assert(MFG_WALK_LEAVES >= 63 + 64 * 3, "a step of 8 nodes with leaves of 3 facets fits the list");
 #define MFG_LANE_STACK ((MFG_WALK_NODES + MFG_WALK_LEAVES) / 64)   // entries of a lane's own stack in the same LDS
+#define MFG_REFILL 6             // TraceParams::refill_at of a long queue (1e6-particle tube 4.0 -> 3.5 ms; 12 and
+                                 // more leave a steady beam-pipe launch slower)
 #define MFG_MAX_GROUPS 64
 #define MFG_MAXWELL_POINTS 100
 #define MFG_MAXWELL_GUIDE 128
@@ -327,6 +329,7 @@ struct TraceParams {
     uint32_t task_bits;               // bits of a walk task's node or record index (the rest: its ray)
     uint32_t child_lanes;             // facets a leaf may hold if so few (at most 3) that 8 nodes' facets fit the list, else 0
     uint32_t lane_quota;              // lanes of a wave that take particles
+    uint32_t refill_at;               // lanes without a particle that make a wave refill them
     uint64_t dealt;                   // items dealt out by wave index (waves * lane_quota) before the queue's
     uint32_t stack_total;             // entries a lane's own walk may need; the ones past MFG_LANE_STACK
     int32_t* stack_spill;             // live in this per-lane global area (lane-major)

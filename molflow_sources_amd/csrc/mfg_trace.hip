@@ -2062,8 +2062,6 @@ __device__ __forceinline__ uint32_t find_variant(const uint64_t* prefix, uint32_
     return lo;
 }
 
-constexpr uint32_t kRefill = 6;   // lanes without a particle that make a wave refill them (1e6-particle tube
-                                  // 4.0 -> 3.5 ms; 12 and more leave a steady beam-pipe launch slower)
 constexpr int kFewRecords = 8;   // fewer records than this go out lane by lane (nothing to merge, one LDS round trip less)
 
 template <uint32_t FEAT, bool ONE>
@@ -2133,7 +2131,6 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     }
     const uint64_t items = n_in + P.total;
     const uint64_t t_start = wall_clock64();
-    const uint32_t refill_at = P.lane_quota < kRefill ? P.lane_quota : kRefill;
     uint32_t iter = 0;   // the loop is wave-uniform, and so is this count
     // the stop flag lives in host memory: a read crosses the bus, so it is
     // polled every 64 iterations, not at every refill
@@ -2151,7 +2148,7 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
         uint64_t mask = expired ? 0ull : __ballot(need);
         // a refill costs the wave about the same for one lane as for many,
         // and a lane without a ray is no loss to the walk: wait for several
-        if ((uint32_t)__popcll(mask) < refill_at && __ballot(alive)) mask = 0ull;
+        if ((uint32_t)__popcll(mask) < P.refill_at && __ballot(alive)) mask = 0ull;
         bool dry = false;   // some lane of this wave found the queue exhausted
         if (mask) {
             uint32_t cnt = (uint32_t)__popcll(mask);
