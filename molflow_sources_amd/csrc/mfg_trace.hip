@@ -2131,6 +2131,9 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     }
     const uint64_t items = n_in + P.total;
     const uint64_t t_start = wall_clock64();
+    // kept in a register: read from the arguments at every event it cost a
+    // lone particle 2 % (5k-facet pipe 27.5 ms, 27.0 so)
+    const uint32_t refill_at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(P.lane_quota < P.refill_at ? P.lane_quota : P.refill_at));
     uint32_t iter = 0;   // the loop is wave-uniform, and so is this count
     // the stop flag lives in host memory: a read crosses the bus, so it is
     // polled every 64 iterations, not at every refill
@@ -2148,7 +2151,7 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
         uint64_t mask = expired ? 0ull : __ballot(need);
         // a refill costs the wave about the same for one lane as for many,
         // and a lane without a ray is no loss to the walk: wait for several
-        if ((uint32_t)__popcll(mask) < P.refill_at && __ballot(alive)) mask = 0ull;
+        if ((uint32_t)__popcll(mask) < refill_at && __ballot(alive)) mask = 0ull;
         bool dry = false;   // some lane of this wave found the queue exhausted
         if (mask) {
             uint32_t cnt = (uint32_t)__popcll(mask);
