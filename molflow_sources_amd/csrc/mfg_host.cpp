@@ -1503,11 +1503,23 @@ int default_waves(uint32_t feats) {
     return (k & FEAT_ADJOINT) ? 1 : 2;
 }
 
+// Waves per SIMD of the kernel that a choice of `waves` runs: the kernels are
+// built for a range of them, and the CU's LDS is split among as many blocks as
+// that kernel has. (A choice of 1 on the lean set, which starts at 2, would
+// else give one block all of it and leave half the waves out; 5 would leave
+// no LDS for the tree.)
+int built_waves(uint32_t feats, int waves) {
+    int wl[8];
+    const int n = mfg_trace_variants(feats, wl, 8);
+    return std::max(wl[0], std::min(waves, wl[n - 1]));
+}
+
 // items: particles the launch will trace. share: blocks of 256 lanes among
 // which a CU's LDS is split.
 void launch_shape(mfg_context* c, uint32_t feats, uint64_t items, int& grid, int& block, int& waves, int& share) {
     block = (int)c->block;
-    waves = c->waves ? c->waves : default_waves(feats);
+    const int waves_256 = built_waves(feats, c->waves ? c->waves : default_waves(feats));
+    waves = waves_256;
     if (block > 256) {
         // the one-block-per-CU kernels exist for the lean and low-flux
         // feature sets (768 lanes: 3 waves per SIMD, 1024: 4); other runs
@@ -1530,7 +1542,7 @@ void launch_shape(mfg_context* c, uint32_t feats, uint64_t items, int& grid, int
     };
     if (block > 256 && mfg_trace_occupancy(feats, c->dvars.size() == 1, waves, block, lds_bytes(block)) < 1) {
         block = 256;   // the block's LDS does not fit
-        share = waves = c->waves ? c->waves : default_waves(feats);
+        share = waves = waves_256;
     }
     uint32_t per_cu = c->blocks_per_cu;
     if (block > 256 || thin) per_cu = 1;
