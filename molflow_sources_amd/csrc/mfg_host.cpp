@@ -1532,9 +1532,12 @@ void launch_shape(mfg_context* c, uint32_t feats, uint64_t items, int& grid, int
     // as a node step can give 8 lanes each): more waves would not shorten the
     // longest of them, and one block a CU gets the whole LDS for the top of
     // the tree. 1000 tube particles 1.00 -> 0.79 ms, 8000 0.99 -> 0.82, 3000
-    // low-flux ones 49.8 -> 46.2; from 12 a wave on low flux is slower (62 ->
-    // 66 ms at 1.2e4)
-    const bool thin = items <= (uint64_t)c->n_cu * 32 && block == 256 && c->waves == 0 && c->blocks_per_cu == 0;
+    // low-flux ones 49.8 -> 46.2, 3000 in teleporting tubes 1.36 -> 1.30; from
+    // 12 a wave on low flux is slower (62 -> 66 ms at 1.2e4). Several variants
+    // keep no tree in LDS and gain nothing: 8000 particles on 16 variants 77
+    // ms, 82 with this rule (1500: 46 and 49, 400: 49 and 46)
+    const bool thin = c->dvars.size() == 1 && items <= (uint64_t)c->n_cu * 32 && block == 256 && c->waves == 0 &&
+                      c->blocks_per_cu == 0;
     if (thin) share = 1;
     auto lds_bytes = [&](int b) {
         return (size_t)(b / 64) * mfg_wave_lds(feats) + c->hot_bytes() +
