@@ -1621,7 +1621,7 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
     // 1000 tube particles 3.1 -> 1.6 ms, 2e4 adjoint ones 394 -> 114 ms with
     // the shared walk, one wave in ten having had all of the latter before)
     const uint64_t n_waves = (uint64_t)grid * (uint64_t)(block / 64);
-    const uint64_t cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
+    const uint64_t cap = mfg_task_rays(c->task_bits);
     p.lane_quota = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cap, (total + c->in_flight + n_waves - 1) / n_waves));
     p.refill_at = std::min<uint32_t>(p.lane_quota, MFG_REFILL);
     if (c->carry_on) {
@@ -1945,7 +1945,7 @@ void launch_batch(mfg_context* c, uint64_t n, const double* dO, const double* dD
     p.root = c->h_roots.at(c->dvars[0].root_base + (uint32_t)structure);
     // few rays are spread over the CUs, 8 a wave at least (the wave's lanes
     // share their walks)
-    const uint64_t spread = n / ((uint64_t)c->n_cu * 8), cap = std::min<uint64_t>(64, 1ull << (32 - c->task_bits));
+    const uint64_t spread = n / ((uint64_t)c->n_cu * 8), cap = mfg_task_rays(c->task_bits);
     p.rays_per_wave = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(8, spread));
     p.task_bits = c->task_bits; p.child_lanes = c->leaf_most <= 3 ? c->leaf_most : 0u; p.n = n; p.origins = dO; p.dirs = dD; p.last_hit = dL;
     p.out_facet = dF; p.out_t = dT; p.out_u = dU; p.out_v = dV; p.facet_base = c->dvars[0].facet_base;

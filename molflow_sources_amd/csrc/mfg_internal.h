@@ -19,11 +19,22 @@
 
 #define MFG_ADJ_SEG 32            // target scores kept per lane for the adjoint's cutoff term
 #define MFG_BVH_WIDTH 8          // children per node (a 4-wide build uses 4 of the 8 slots)
-#define MFG_MAX_STACK 64
+#define MFG_MAX_STACK 64         // (width - 1) * depth + width of the deepest tree the host accepts
 #define MFG_WALK_NODES 512       // (ray, node) tasks of one wave's walk
 #define MFG_WALK_RESERVE 72      // of these for the depth-first tail: width - 1 entries a level, + width
 #define MFG_WALK_LEAVES 256      // (ray, facet record) tasks waiting: below 64 plus one node's 8 leaves of 16
 static_assert(MFG_WALK_LEAVES >= 63 + 64 * 3, "a step of 8 nodes with leaves of 3 facets fits the list");
+static_assert(MFG_WALK_LEAVES >= 63 + 8 * 16, "a node's 8 leaves of 16 facets fit the list whenever a node step runs");
+static_assert(MFG_WALK_RESERVE >= MFG_MAX_STACK, "the reserve holds a depth-first walk of the deepest tree");
+static_assert(MFG_WALK_NODES - MFG_WALK_RESERVE >= 64 && MFG_WALK_NODES >= 16 * 8,
+              "64 roots, or the children of 16 nodes, fit below the reserve");
+// Rays of a wave whose walk tasks give `bits` bits to the index of a node or
+// record (26 up to 2^26 of them, else as many as they need).
+constexpr uint32_t mfg_task_rays(uint32_t bits) { return bits <= 26u ? 64u : 1u << (32u - bits); }
+constexpr bool mfg_task_fits(uint32_t bits) {
+    return mfg_task_rays(bits) <= 64u && ((uint64_t)(mfg_task_rays(bits) - 1u) << bits | ((1ull << bits) - 1ull)) <= 0xffffffffull;
+}
+static_assert(mfg_task_fits(26) && mfg_task_fits(27) && mfg_task_fits(28), "ray and index fit a task's word");
 #define MFG_LANE_STACK ((MFG_WALK_NODES + MFG_WALK_LEAVES) / 64)   // entries of a lane's own stack in the same LDS
 #define MFG_REFILL 6             // TraceParams::refill_at of a long queue (1e6-particle tube 4.0 -> 3.5 ms; 12 and
                                  // more leave a steady beam-pipe launch slower)
@@ -233,7 +244,8 @@ struct alignas(16) PassLds {
 
 // Where the rays of a structure start: its root node (-1: no facets), and
 // the nodes a wave with few rays starts from, first << 4 | how many: the
-// root's children if none of them is a leaf, else the root.
+// root's children if none of them is a leaf, else the root (a model has fewer
+// than 2^27 leaf records, and no more nodes than those).
 struct Root {
     int32_t node;
     uint32_t first;
