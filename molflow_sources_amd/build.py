@@ -20,7 +20,7 @@ SOURCES = ["mfg_trace.hip", "mfg_host.cpp"]
 # whole event, and hoisting the FP64 constants of sincos, pow, acos and log
 # out of it kept some 80 VGPRs live across the walk, which then spilled (336 B
 # of scratch a lane at 3 waves per SIMD, 0 without; the full kernel at 2
-# waves: 628 B and 44 B).
+# waves: 628 B, now 16 B).
 SOURCE_FLAGS = {"mfg_trace.hip": ["-mllvm", "-disable-machine-licm"]}
 
 

@@ -1493,7 +1493,7 @@ TraceParams make_params(mfg_context* c, uint64_t total, uint64_t max_events) {
 }
 
 // Waves per SIMD without a choice by the caller or the autotuner. The lean
-// kernel runs 3 without scratch. The weighted ones spill at 3 (100 B a lane),
+// kernel runs 3 without scratch. The weighted ones spill at 3 (84 B a lane),
 // and their runs are mostly long thin tails: 2 waves took 2e4 low-flux
 // particles from 97 to 78 ms and the adjoint from 80 to 65. The full kernel
 // fits 2; with the adjoint it takes 1.

@@ -2,12 +2,16 @@
 // host runtime (mfg_host.cpp) and the HIP kernels (mfg_trace.hip).
 //
 // HBM layout (all variants concatenated; a plain model is one variant):
-//   DFacet[nF_total]      128 B, one cache line per ray/facet test
-//   DPhys[nF_total]       physics and recording parameters, read on a hit
-//   double2 poly[]        normalised (u,v) polygon vertices
-//   BvhNode[]             up to 8-wide nodes, 128 B each, 8-bit quantised boxes
 //   LeafFacet[]           the ray/facet test data in leaf order (128 B): a
 //                         leaf is a contiguous run, no index indirection
+//   BvhNode[]             up to 8-wide nodes, 128 B each, 8-bit quantised boxes
+//   DHit[nF_total]        128 B, what a wall event always needs of its facet
+//   DFacet[nF_total]      frame and polygon: sources, teleport destinations and
+//                         the (u,v) of hits that are recorded by place
+//   DPhys[nF_total]       physics and recording parameters beyond DHit, read
+//                         for what the facet's flags name
+//   Root[]                where the rays of each (variant, structure) start
+//   double2 poly[]        normalised (u,v) polygon vertices
 //   LeafUV[]              quadrilateral (u,v) corners (64 B), leaf order
 //   DVariant[nV]          per-variant bases and settings
 //   tallies               [variant][slot][facet] 64 B counters, textures,

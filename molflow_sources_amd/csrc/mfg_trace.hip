@@ -1020,11 +1020,12 @@ struct Tracer {
     uint32_t seg_n;                   // adjoint: target scores since the last survived sticky collision
     int32_t* seg_t;
     double* seg_x;
-    double* hot;                      // LDS table of the hot facets' slot-0 counters (8 words each)
+    double* hot;                      // LDS counters of the hot facets' first P.hot_slots slots (8 words each)
     double* profs;                    // LDS slices of the profiles kept there
     const uint4* lnodes;              // LDS copy of the first P.lds_nodes BVH nodes
     const MaxwellLds* maxwell;        // LDS copy of the Maxwell CDF (P.maxwell_scale > 0)
-    // pending slot-0 facet counter update of this lane
+    // pending slot-0 facet counter update of this lane (the event's other
+    // slots are added at once)
     int32_t pend_f, pend_hot;
     uint32_t pend_hits;
     double pend_he, pend_abs, pend_s1v, pend_svo, pend_s1pv;
@@ -2071,8 +2072,13 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     WaveLds& W = reinterpret_cast<WaveLds*>(lds_base)[threadIdx.x >> 6];
     const size_t gl = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     int32_t* spill = P.stack_spill ? P.stack_spill + gl * (P.stack_total - MFG_LANE_STACK) : nullptr;
-    // after the waves' walk areas: their pass areas (transparent models),
-    // then the hot-facet counters
+    // after the waves' walk areas: their pass areas (transparent models), the
+    // hot-facet counters, the profile slices, the Maxwell table, and the copy
+    // of the top of the tree (128 B a node), whose 16 B loads set the
+    // alignment that every part keeps
+    static_assert(sizeof(WaveLds) % 16 == 0 && sizeof(PassLds) % 16 == 0 && sizeof(MaxwellLds) % 16 == 0 &&
+                  3 * MFG_PROFILE_SIZE * sizeof(double) % 16 == 0 && sizeof(mfg_facet_counters) % 16 == 0,
+                  "parts of a block's LDS are multiples of 16 B");
     unsigned char* lds_next = lds_base + (blockDim.x >> 6) * sizeof(WaveLds);
     PassLds* pass = nullptr;
     if constexpr ((FEAT & FEAT_TRANSPARENT) != 0) {
@@ -2083,8 +2089,6 @@ __device__ __forceinline__ void trace_body(const TraceParams& P) {
     double* hot = reinterpret_cast<double*>(lds_next);
     const uint32_t hot_words = 8u * P.n_hot * P.hot_slots;
     for (uint32_t i = threadIdx.x; i < hot_words; i += blockDim.x) hot[i] = 0.0;
-    // then the block's copy of the top of the tree (128 B per node; the
-    // offsets above are multiples of 64 B)
     double* profs = hot + hot_words;
     const uint32_t prof_words = 3u * MFG_PROFILE_SIZE * P.n_prof_hot * P.prof_slots;
     for (uint32_t i = threadIdx.x; i < prof_words; i += blockDim.x) profs[i] = 0.0;
