@@ -434,6 +434,9 @@ def plain_leg(args, tube):
         out["roofline"]["traffic_GBps"] = rate
         out["roofline"]["random_line_read_GBps"] = g
         out["roofline"]["traffic_frac_of_random_line_rate"] = rate / g["64MiB_GBps"]
+    if not tube:
+        out["roofline"]["note"] = ("achieved counts the bytes of the reference's binary tree, of which the kernel reads a "
+                                   "part: frac can exceed 1; traffic, issue and atomics are what the kernel itself does")
     if tube:
         # 3,202 facets: nodes, leaf records, facet data and tallies (about
         # 2 MB) stay in each XCD's 4 MB L2, so the HBM fraction is nominal
