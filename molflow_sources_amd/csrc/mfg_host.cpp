@@ -1630,7 +1630,11 @@ void run_variants(mfg_context* c, const uint64_t* n_des, const uint64_t* seeds, 
         // the particles spread, a wave's few would all have to end first:
         // the waves are filled, and the first free lane looks where nothing
         // is left to take after the first deal, or where fewer particles are
-        // new than lanes would end in waiting for several.
+        // new than lanes would end in waiting for several. Spread and filled,
+        // steady time of a run: 5k-facet pipe, 100 particles 11.2 and 0.85
+        // ms, 10,000 22.4 and 2.3; tube of 10,000 1.11 and 0.47; 64 variants
+        // of 100 48.5 and 3.3. From 6 a wave on both wait for several lanes
+        // (5k-facet pipe, 100,000: 11.7 and 11.8).
         p.lane_quota = (uint32_t)cap;
         p.refill_at = total < MFG_REFILL * n_waves || total + c->in_flight <= n_waves * cap ? 1u : MFG_REFILL;
     }
